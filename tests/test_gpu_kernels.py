@@ -364,6 +364,39 @@ def test_query_rows_outside_the_layer_are_skipped(ucm, dev, repre_dtype):
                 assert np.all(got[l][seg] == -5.0), (l, r)
 
 
+@pytest.mark.parametrize("repre_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tile", [16, 64])
+def test_fused_selection_of_whole_split_and_unfollowed_requests(ucm, dev, repre_dtype, tile):
+    """The one-launch call selects from LDS when a workgroup holds the whole request, from memory otherwise; a request
+    whose query row is out of range keeps the scores it had and is selected from them, as the two calls do."""
+    from ucm_amd import ops
+
+    hkv, g, d, n_tok = 8, 4, 128, 6
+    lens = np.array([1, 15, 16, 17, 63, 64, 65, 130, 16, 70], np.int32)
+    q_rows = np.array([0, 1, 2, 3, 4, 5, 0, 1, n_tok, -1], np.int32)        # the last two are not followed
+    off = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    topk = np.array([1, 6, 5, 7, 19, 64, 20, 9, 5, 8], np.int32)
+    rows, mx = int(lens.sum()), int(lens.max())
+    q = torch.from_numpy(synth.normal_bf16_as_f32(71, (2, n_tok, hkv * g, d))).to(dev).to(torch.bfloat16)
+    repre = torch.from_numpy(synth.normal_f32(72, (2, rows, hkv * d))).to(dev).to(repre_dtype)
+    old = torch.from_numpy(synth.normal_f32(73, (2, rows))).to(dev)
+    args = (i32(off, dev), i32(lens, dev))
+    out = []
+    for fused in (False, True):
+        scores, idx = old.clone(), torch.full((2, len(lens), mx), -1, dtype=torch.int32, device=dev)
+        cnt, tickets = torch.full((2, len(lens)), -1, dtype=torch.int32, device=dev), torch.zeros((2, len(lens)), dtype=torch.int32, device=dev)
+        if fused:
+            ops.score_select(q, repre, *args, i32(topk, dev), mx, hkv, scores, idx, cnt, tickets, q_rows=i32(q_rows, dev), tile_blocks=tile)
+            assert not tickets.any()
+        else:
+            ops.score_blocks(q, repre, *args, mx, hkv, scores, q_rows=i32(q_rows, dev), tile_blocks=tile)
+            ops.topk_windows(scores, *args, i32(topk, dev), mx, idx, cnt)
+        out.append((scores, idx, cnt))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    assert torch.equal(out[1][0][:, off[8]:], old[:, off[8]:])
+
+
 def test_many_requests_dense_tile_lookup(ucm, dev):
     """More requests than one wavefront scans at once (the tile -> request lookup runs in trips of 64),
     with empty requests in between, and the grid sized from the host-known total."""

@@ -15,6 +15,11 @@
 // cross threads are quad_perm DPP moves, and the last fold is in-register.
 // The request's group-mean query is staged once per workgroup in LDS and then
 // kept in registers (a thread's head never changes because kv_heads divides 16).
+//
+// The table is read in whole 128-byte lines with the non-temporal hint: a read-only loop over 1 GiB reaches 7.0 TB/s with
+// the hint and 6.2 TB/s without it.  80 layers x 8 requests x 6399 blocks (bf16 table, 1.06 GB, with the selection): 177 us
+// = 6.0 TB/s, and 161 us = 6.6 TB/s for the scores alone; 192-208 us with plain loads of 32 bytes per vector and
+// instruction (which the hint makes worse: a line then does not stay in the L1 for the other pieces).
 #include <algorithm>
 #include <cfloat>
 
@@ -26,10 +31,12 @@
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+using ucm::u32x4;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxRow = 16 * 128;  // kv_heads * head_dim: what the staged query row may hold
+constexpr int kMaxTile = 2048;     // blocks of a workgroup: 128 KiB of the narrowest rows (32 bf16)
 
 template <int kCtrl>
 __device__ __forceinline__ float quad_perm(float x)
@@ -88,32 +95,78 @@ __device__ __forceinline__ f32x4 group_mean4_any(const QT* src, int head_stride,
     return acc * inv;
 }
 
-// Plain loads on purpose: one instruction touches only 64 bytes (32 for the bf16
-// table) of each 128-byte line and the next steps touch the rest, so the line
-// has to stay in the vector L1 between them.  Nontemporal loads do not keep it
-// there and every step then fetches the line from L2 again (bf16 table: 88 us
-// instead of 47 us at 16 requests x 32 layers).
-template <int kSteps>
-__device__ __forceinline__ void load_pass(f32x4 (&kv)[kSteps], const float* p)
+// The 128-byte lines of a vector are loaded whole: an instruction reads `kGroup` steps of 16 dims of a vector with
+// neighbouring lanes, and what the lanes then hold of each other's vectors is exchanged in registers.  (A lane that loads
+// its own vector's pieces step by step has every instruction touch a piece of each of the wave's vectors, and
+// the L1 looks up one line per lane pair instead of one per eight lanes.)  swap_halves / swap_rows exchange bit 5 / bit 4
+// of the lane number with the bit that tells the two registers apart.
+__device__ __forceinline__ void swap_halves(unsigned& a, unsigned& b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void swap_rows(unsigned& a, unsigned& b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// One pass of a wave: kSteps 16-byte loads per lane over 64/kLanes vectors, kLanes adjacent lanes per vector and step.
+// Register g*kGroup + n of lane L receives step g*kGroup + (L's top bits) of vector n*(vectors/kGroup) + (L / kLanes);
+// own_vectors then leaves step i of vector L/kLanes in register i.  A block past `last` is read as block `last`.
+template <int kSteps, int kGroup, int kLanes, typename T>
+__device__ __forceinline__ void load_vectors(u32x4 (&kv)[kSteps], const T* __restrict__ rbase, int base, int last, int vecs, int lane)
+{
+    constexpr int kPer = 64 / kLanes / kGroup;           // vectors per load instruction
+    constexpr int kElems = 16 / kLanes;                  // elements of a 16-byte piece
+    const int step = lane / (64 / kGroup), mine = (lane / kLanes) & (kPer - 1);
+    const int lg = __builtin_ctz(vecs);                  // vecs is a power of two (host checked)
+#pragma unroll
+    for (int n = 0; n < kGroup; ++n) {
+        const int v = n * kPer + mine;
+        const int vec = (min(base + (v >> lg), last) << lg) + (v & (vecs - 1));
+        const T* p = rbase + static_cast<size_t>(static_cast<unsigned>(vec)) * (kSteps * 16) + step * 16 + (lane & (kLanes - 1)) * kElems;
+#pragma unroll
+        for (int g = 0; g < kSteps / kGroup; ++g) { kv[g * kGroup + n] = ucm::gload16_nt(p + g * kGroup * 16); }
+    }
+}
+
+template <int kGroup>
+__device__ __forceinline__ void own_vectors(u32x4* kv)
 {
 #pragma unroll
-    for (int i = 0; i < kSteps; ++i) {
-        kv[i] = *reinterpret_cast<const f32x4*>(p + 16 * i);
+    for (int w = 0; w < 4; ++w) {
+        unsigned r[kGroup];
+#pragma unroll
+        for (int n = 0; n < kGroup; ++n) { r[n] = kv[n][w]; }
+        if constexpr (kGroup == 4) {
+            swap_halves(r[0], r[2]);
+            swap_halves(r[1], r[3]);
+            swap_rows(r[0], r[1]);
+            swap_rows(r[2], r[3]);
+        } else {
+            swap_halves(r[0], r[1]);
+        }
+#pragma unroll
+        for (int n = 0; n < kGroup; ++n) { kv[n][w] = r[n]; }
     }
 }
 
 // One (block, head) dot product in the reference's order; all four threads of
 // the quad return the same value.
 template <int kSteps>
-__device__ __forceinline__ float quad_dot(const f32x4 (&qr)[kSteps], const f32x4 (&kv)[kSteps])
+__device__ __forceinline__ float quad_dot(const f32x4 (&qr)[kSteps], u32x4 (&kv)[kSteps])
 {
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
-        a0 = __builtin_fmaf(qr[i].x, kv[i].x, a0);
-        a1 = __builtin_fmaf(qr[i].y, kv[i].y, a1);
-        a2 = __builtin_fmaf(qr[i].z, kv[i].z, a2);
-        a3 = __builtin_fmaf(qr[i].w, kv[i].w, a3);
+        if (i % 2 == 0) { own_vectors<2>(&kv[i]); }
+        a0 = __builtin_fmaf(qr[i].x, __uint_as_float(kv[i].x), a0);
+        a1 = __builtin_fmaf(qr[i].y, __uint_as_float(kv[i].y), a1);
+        a2 = __builtin_fmaf(qr[i].z, __uint_as_float(kv[i].z), a2);
+        a3 = __builtin_fmaf(qr[i].w, __uint_as_float(kv[i].w), a3);
     }
     // lanes j and j+8 live two threads apart, j and j+4 one thread apart
     a0 = quad_perm<kQuadXor2>(a0) + a0; a1 = quad_perm<kQuadXor2>(a1) + a1;
@@ -121,6 +174,18 @@ __device__ __forceinline__ float quad_dot(const f32x4 (&qr)[kSteps], const f32x4
     a0 = quad_perm<kQuadXor1>(a0) + a0; a1 = quad_perm<kQuadXor1>(a1) + a1;
     a2 = quad_perm<kQuadXor1>(a2) + a2; a3 = quad_perm<kQuadXor1>(a3) + a3;
     return (a0 + a2) + (a1 + a3);
+}
+
+// Inclusive sum over the wave's lanes: within rows of sixteen, then from row to row.
+__device__ __forceinline__ int inclusive_scan(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+    return x;
 }
 
 // Finds the request that owns dense tile index `w` (tiles of all requests laid
@@ -133,10 +198,11 @@ __device__ __forceinline__ int clamped_len(int n, int max_seg_len) { return min(
 
 // The owner's other descriptors come back with it: every lane fetches its request's first row and query row together
 // with its length, so the workgroup waits for memory once here, not once for the lengths and again for what they lead to.
+// (topk_len is null unless the selection is fused in.)
 __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ seg_len, const int32_t* __restrict__ seg_off,
-                                          const int32_t* __restrict__ q_rows, int n_req, int tile_blocks, int max_seg_len,
-                                          int min_tiles, int w, int lane, int& r_out, int& tile_out, int& len_out,
-                                          int& off_out, int& q_row_out)
+                                          const int32_t* __restrict__ q_rows, const int32_t* __restrict__ topk_len, int n_req,
+                                          int tile_blocks, int max_seg_len, int min_tiles, int w, int lane, int& r_out,
+                                          int& tile_out, int& len_out, int& off_out, int& q_row_out, int& topk_out)
 {
     int base = 0;
     for (int c = 0; c < n_req; c += 64) {
@@ -145,24 +211,21 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ seg_len, c
         const int len = live ? clamped_len(seg_len[r], max_seg_len) : 0;
         const int off = live ? seg_off[r] : 0;
         const int qr = live && q_rows ? q_rows[r] : r;
+        const int top = live && topk_len ? topk_len[r] : 0;
         const int t = live ? max((len + tile_blocks - 1) / tile_blocks, min_tiles) : 0;
-        int incl = t;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int up = __shfl_up(incl, d, 64);
-            if (lane >= d) { incl += up; }
-        }
+        const int incl = inclusive_scan(t);
         const unsigned long long owner = __ballot(w < base + incl);
         if (owner) {
             const int src = __builtin_ctzll(owner);
             r_out = c + src;
-            tile_out = w - (base + __shfl(incl - t, src, 64));
+            tile_out = w - (base + __builtin_amdgcn_readlane(incl - t, src));
             len_out = __builtin_amdgcn_readlane(len, src);       // (scalar results: what follows stays uniform)
             off_out = __builtin_amdgcn_readlane(off, src);
             q_row_out = __builtin_amdgcn_readlane(qr, src);
+            topk_out = __builtin_amdgcn_readlane(top, src);
             return true;
         }
-        base += __shfl(incl, 63, 64);
+        base += __builtin_amdgcn_readlane(incl, 63);
     }
     return false;
 }
@@ -191,17 +254,17 @@ struct ScoreArgs {
 
 // What a workgroup works on: request, tile, and whether the request's descriptors may be followed.
 struct TileInfo {
-    int r, tile, n;
+    int r, tile, n, topk;
     int64_t seg0, q_row;
     bool ok;
 };
 
 template <int kD>
-__device__ __forceinline__ bool locate(const ScoreArgs& a, int lane, TileInfo& t)
+__device__ __forceinline__ bool locate(const ScoreArgs& a, const int32_t* topk_len, int lane, TileInfo& t)
 {
     int len = 0, off = 0, q_row = 0;
-    if (!find_tile(a.seg_len, a.seg_off, a.q_rows, a.n_req, a.tile_blocks, a.max_seg_len, a.tickets ? 1 : 0, blockIdx.y, lane,
-                   t.r, t.tile, len, off, q_row)) {
+    if (!find_tile(a.seg_len, a.seg_off, a.q_rows, topk_len, a.n_req, a.tile_blocks, a.max_seg_len, a.tickets ? 1 : 0, blockIdx.y, lane,
+                   t.r, t.tile, len, off, q_row, t.topk)) {
         return false;
     }
     t.n = len;
@@ -243,41 +306,56 @@ __device__ __forceinline__ float head_sum(float dot, int first, int step, int kv
     return s;
 }
 
-// A score on its way out.  With the selection fused in, another workgroup of this launch reads it: the store then
-// goes through to memory at device scope (no cache of another part of the chip keeps it back), and the reader
-// uses device-scope loads.
-__device__ __forceinline__ void store_score(float* p, float v, bool through)
+// The request's selection with the smallest tier of key registers that holds it (the host allows at most 1024 blocks here).
+__device__ __forceinline__ void select_tier(const ucm::SelectArgs& sel, const TileInfo& t, int l, int lane, const float* lds)
 {
-    if (through) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    else { *p = v; }
+    if (t.n <= 64) { ucm::select_wave<1, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
+    else if (t.n <= 128) { ucm::select_wave<2, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
+    else if (t.n <= 256) { ucm::select_wave<4, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
+    else if (t.n <= 512) { ucm::select_wave<8, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
+    else { ucm::select_wave<16, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
 }
 
-// The fused kernel's tail.  Every workgroup of a request takes a ticket once its scores have reached memory; the
-// one that draws the last ticket resets the counter and its first wave runs the request's selection
-// (TopkBlockSelector::TopKImpl, select_topk_block.cpp:20-51) on the scores all of them wrote.  Ordering: a wave's
-// score stores are device-scope write-through stores, complete when the wave's memory counter reaches zero (the
-// workgroup-scope fence below waits for that); the barrier then orders all waves' stores before thread 0's ticket;
-// the last workgroup reads the scores with device-scope loads after it has seen every other ticket.  (A
-// device-scope release/acquire pair would also do, but it writes the whole L2 back per wave: 7x the kernel's time.)
-__device__ __forceinline__ void select_if_last(const ScoreArgs& a, const ucm::SelectArgs& sel, const TileInfo& t, int l)
+// A tile's scores on their way out: collected in LDS and written as whole lines when the tile is done.  (One store per
+// pass puts 16 bytes at a time on the memory bus between the reads, and with the selection fused in every one of them goes
+// all the way to memory: 80 layers x 8 requests x 6399 blocks took 192 us that way.)
+//
+// With the selection fused in, another workgroup of this launch reads the scores.  One wave then stores them at device scope
+// (write-through: no cache of another part of the chip keeps them back), waits until they have reached memory and takes
+// the request's ticket; the others are done before that.  The workgroup that draws the last ticket resets the counter and
+// its wave runs the request's selection (TopkBlockSelector::TopKImpl, select_topk_block.cpp:20-51) on the scores all of
+// them wrote, which it reads with device-scope loads after it has seen every other ticket.  (A device-scope
+// release/acquire pair would also do, but it writes the whole L2 back per wave: 7x the kernel's time.)
+__device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::SelectArgs& sel, const TileInfo& t, int l, int tile0,
+                                            int n_tile, const float* tile_scores)
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    float* sout = a.scores + static_cast<int64_t>(l) * a.scores_layer_stride + t.seg0 + tile0;
+    if (!a.tickets) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < n_tile; i += kThreads) { sout[i] = tile_scores[i]; }
+        return;
+    }
     __syncthreads();
     if (threadIdx.x >= 64) { return; }                           // the other waves are done: their registers are free again
     const int lane = threadIdx.x;
+    const int tiles = max((t.n + a.tile_blocks - 1) / a.tile_blocks, 1);
+    if (tiles == 1 && t.ok) {                                    // all of the request's scores are here: nobody to wait for
+        for (int i = lane; i < n_tile; i += 64) { sout[i] = tile_scores[i]; }
+        select_tier(sel, t, l, lane, tile_scores);
+        return;
+    }
+    for (int i = lane; i < n_tile; i += 64) {
+        __hip_atomic_store(sout + i, tile_scores[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");       // (the stores are complete when the wave's memory counter is zero)
+    __builtin_amdgcn_s_waitcnt(0);
     int drawn = 0;
     int32_t* ticket = a.tickets + static_cast<int64_t>(l) * sel.cnt_layer_stride + t.r;
     if (lane == 0) { drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
     drawn = __builtin_amdgcn_readfirstlane(drawn);
-    const int tiles = max((t.n + a.tile_blocks - 1) / a.tile_blocks, 1);
     if (drawn != tiles - 1) { return; }
     if (lane == 0) { __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    // the smallest tier of key registers that holds the request (the host allows at most 1024 blocks here)
-    if (t.n <= 64) { ucm::select_wave<1, false, true>(sel, t.r, l, lane); }
-    else if (t.n <= 128) { ucm::select_wave<2, false, true>(sel, t.r, l, lane); }
-    else if (t.n <= 256) { ucm::select_wave<4, false, true>(sel, t.r, l, lane); }
-    else if (t.n <= 512) { ucm::select_wave<8, false, true>(sel, t.r, l, lane); }
-    else { ucm::select_wave<16, false, true>(sel, t.r, l, lane); }
+    select_tier(sel, t, l, lane, nullptr);
 }
 
 // grid: x = layer, y = dense tile index over all requests (workgroups past the
@@ -293,12 +371,12 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
 {
     constexpr int kSteps = kD / 16;
     __shared__ __attribute__((aligned(16))) float qbar[kMaxRow];
+    __shared__ float tile_scores[kMaxTile];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l = blockIdx.x;
-    const bool fused = a.tickets != nullptr;
     TileInfo t;
-    if (!locate<kD>(a, lane, t)) { return; }
+    if (!locate<kD>(a, sel.topk_len, lane, t)) { return; }
     const int tile0 = t.tile * a.tile_blocks;
     const int tile_end = min(tile0 + a.tile_blocks, t.n);
     if (t.ok && tile0 < tile_end) {                                  // (uniform over the workgroup)
@@ -313,15 +391,15 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
         const int h = vb / a.num_repre;         // its kv head
         const int stride = kWaves * blocks_per_pass;
 
-        const float* rbase = static_cast<const float*>(a.repre) + static_cast<int64_t>(l) * a.repre_layer_stride +
-                             t.seg0 * row + vb * kD + 4 * m;
-        float* sout = a.scores + static_cast<int64_t>(l) * a.scores_layer_stride + t.seg0;
+        const float* rbase = static_cast<const float*>(a.repre) + static_cast<int64_t>(l) * a.repre_layer_stride + t.seg0 * row;
 
         // the first pass's representatives are requested before the query is
         // touched, so the two latencies overlap
         int b0 = tile0 + wave * blocks_per_pass;
-        f32x4 kv_a[kSteps], kv_b[kSteps];
-        if (b0 < tile_end) { load_pass<kSteps>(kv_a, rbase + static_cast<int64_t>(min(b0 + bl, tile_end - 1)) * row); }
+        u32x4 kv_a[kSteps], kv_b[kSteps];
+        auto load_pass = [&](u32x4 (&kv)[kSteps], int base) { load_vectors<kSteps, 2, 4>(kv, rbase, base, tile_end - 1, vecs, lane); };
+        load_pass(kv_a, b0);
+        asm volatile("" ::: "memory");
 
         stage_query<kD, QT>(a, l, t.q_row, qbar);
         __syncthreads();
@@ -333,24 +411,26 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
         }
 
         // two passes per trip: the loads of the next pass are in flight while this one is reduced
-        auto finish = [&](const f32x4 (&kv)[kSteps], int base) {
+        auto finish = [&](u32x4 (&kv)[kSteps], int base) {
             const float dot = quad_dot<kSteps>(qr, kv);
             const float s = head_sum(dot, bl * vecs * 4, 4, a.kv_heads, a.num_repre);
-            const int b = base + bl;
-            if (b < tile_end && vb == 0 && m == 0) { store_score(sout + b, s * a.scale, fused); }   // (a scale of 1 changes no bit)
+            // the lanes of a block all hold its score; a scale of 1 changes no bit
+            tile_scores[min(base + bl, tile_end - 1) - tile0] = s * a.scale;
         };
         while (b0 < tile_end) {
             const int b1 = b0 + stride;
-            if (b1 < tile_end) { load_pass<kSteps>(kv_b, rbase + static_cast<int64_t>(min(b1 + bl, tile_end - 1)) * row); }
+            load_pass(kv_b, b1);
+            asm volatile("" ::: "memory");
             finish(kv_a, b0);
             if (b1 >= tile_end) { break; }
             const int b2 = b1 + stride;
-            if (b2 < tile_end) { load_pass<kSteps>(kv_a, rbase + static_cast<int64_t>(min(b2 + bl, tile_end - 1)) * row); }
+            load_pass(kv_a, b2);
+            asm volatile("" ::: "memory");
             finish(kv_b, b1);
             b0 = b2;
         }
     }
-    if (fused) { select_if_last(a, sel, t, l); }
+    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores);
 }
 
 // ---- bf16 representative table ------------------------------------------------
@@ -361,32 +441,35 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
 // bf16 (16 bytes) per 16-dim step, a wave covers 32 vectors = 8 KiB per pass;
 // the j/j+8 fold crosses the pair (one DPP), the j/j+4 and final folds are
 // in-register.  Same arithmetic, same order, same bits as the fp32-table kernel.
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-template <int kSteps>
-__device__ __forceinline__ void load_pass_bf16(u32x4 (&kv)[kSteps], const uint16_t* p)
-{
-#pragma unroll
-    for (int i = 0; i < kSteps; ++i) {
-        kv[i] = *reinterpret_cast<const u32x4*>(p + 16 * i);
-    }
-}
-
-template <int kSteps>
-__device__ __forceinline__ float pair_dot(const f32x4 (&qlo)[kSteps], const f32x4 (&qhi)[kSteps],
-                                          const u32x4 (&kv)[kSteps])
+// `q` is the thread's part of the staged query (16 values per step: eight of them its own); the lower four of a step come
+// in registers, the upper four are read from LDS here, one group of steps at a time.
+template <int kSteps, int kGroup, int kKept>
+__device__ __forceinline__ float pair_dot(const f32x4 (&qlo)[kKept], const float* q, u32x4 (&kv)[kSteps])
 {
     float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int i = 0; i < kSteps; ++i) {
-        a[0] = __builtin_fmaf(qlo[i].x, __uint_as_float(kv[i].x << 16), a[0]);
-        a[1] = __builtin_fmaf(qlo[i].y, __uint_as_float(kv[i].x & 0xffff0000u), a[1]);
-        a[2] = __builtin_fmaf(qlo[i].z, __uint_as_float(kv[i].y << 16), a[2]);
-        a[3] = __builtin_fmaf(qlo[i].w, __uint_as_float(kv[i].y & 0xffff0000u), a[3]);
-        a[4] = __builtin_fmaf(qhi[i].x, __uint_as_float(kv[i].z << 16), a[4]);
-        a[5] = __builtin_fmaf(qhi[i].y, __uint_as_float(kv[i].z & 0xffff0000u), a[5]);
-        a[6] = __builtin_fmaf(qhi[i].z, __uint_as_float(kv[i].w << 16), a[6]);
-        a[7] = __builtin_fmaf(qhi[i].w, __uint_as_float(kv[i].w & 0xffff0000u), a[7]);
+    for (int g = 0; g < kSteps; g += kGroup) {
+        f32x4 qhi[kGroup], qlow[kGroup];
+#pragma unroll
+        for (int i = 0; i < kGroup; ++i) {
+            qlow[i] = g + i < kKept ? qlo[g + i < kKept ? g + i : 0] : *reinterpret_cast<const f32x4*>(q + 16 * (g + i));
+            qhi[i] = *reinterpret_cast<const f32x4*>(q + 16 * (g + i) + 4);
+        }
+        own_vectors<kGroup>(&kv[g]);
+#pragma unroll
+        for (int i = 0; i < kGroup; ++i) {
+            const u32x4 k = kv[g + i];
+            const f32x4 lo = qlow[i], hi = qhi[i];
+            a[0] = __builtin_fmaf(lo.x, __uint_as_float(k.x << 16), a[0]);
+            a[1] = __builtin_fmaf(lo.y, __uint_as_float(k.x & 0xffff0000u), a[1]);
+            a[2] = __builtin_fmaf(lo.z, __uint_as_float(k.y << 16), a[2]);
+            a[3] = __builtin_fmaf(lo.w, __uint_as_float(k.y & 0xffff0000u), a[3]);
+            a[4] = __builtin_fmaf(hi.x, __uint_as_float(k.z << 16), a[4]);
+            a[5] = __builtin_fmaf(hi.y, __uint_as_float(k.z & 0xffff0000u), a[5]);
+            a[6] = __builtin_fmaf(hi.z, __uint_as_float(k.w << 16), a[6]);
+            a[7] = __builtin_fmaf(hi.w, __uint_as_float(k.w & 0xffff0000u), a[7]);
+        }
+        asm volatile("" ::: "memory");                   // the next group's LDS reads stay behind this group
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) { a[c] = quad_perm<kQuadXor1>(a[c]) + a[c]; }   // lanes j and j+8: the other thread
@@ -395,16 +478,18 @@ __device__ __forceinline__ float pair_dot(const f32x4 (&qlo)[kSteps], const f32x
 }
 
 template <int kD, typename QT>
-__global__ __launch_bounds__(kThreads) void score_kernel_bf16(const ScoreArgs a, const ucm::SelectArgs sel)
+__global__ __launch_bounds__(kThreads, kD <= 128 ? 4 : 2) void score_kernel_bf16(const ScoreArgs a, const ucm::SelectArgs sel)
 {
     constexpr int kSteps = kD / 16;
+    constexpr int kGroup = kSteps % 4 == 0 ? 4 : 2;
+    constexpr int kKept = kSteps / 2;
     __shared__ __attribute__((aligned(16))) float qbar[kMaxRow];
+    __shared__ float tile_scores[kMaxTile];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l = blockIdx.x;
-    const bool fused = a.tickets != nullptr;
     TileInfo t;
-    if (!locate<kD>(a, lane, t)) { return; }
+    if (!locate<kD>(a, sel.topk_len, lane, t)) { return; }
     const int tile0 = t.tile * a.tile_blocks;
     const int tile_end = min(tile0 + a.tile_blocks, t.n);
     if (t.ok && tile0 < tile_end) {                                  // (uniform over the workgroup)
@@ -419,9 +504,7 @@ __global__ __launch_bounds__(kThreads) void score_kernel_bf16(const ScoreArgs a,
         const int h = vb / a.num_repre;
         const int stride = kWaves * blocks_per_pass;
 
-        const uint16_t* rbase = static_cast<const uint16_t*>(a.repre) + static_cast<int64_t>(l) * a.repre_layer_stride +
-                                t.seg0 * row + vb * kD + 8 * p;
-        float* sout = a.scores + static_cast<int64_t>(l) * a.scores_layer_stride + t.seg0;
+        const uint16_t* rbase = static_cast<const uint16_t*>(a.repre) + static_cast<int64_t>(l) * a.repre_layer_stride + t.seg0 * row;
 
         // Loads and the store below are unconditional (rows and the output index are clamped to the tile's last
         // block, whose score is then written more than once): an operation skipped on some path would make the
@@ -429,45 +512,39 @@ __global__ __launch_bounds__(kThreads) void score_kernel_bf16(const ScoreArgs a,
         // sinking a prefetch down to its use.
         int b0 = tile0 + wave * blocks_per_pass;
         u32x4 kv_a[kSteps], kv_b[kSteps];
-        load_pass_bf16<kSteps>(kv_a, rbase + static_cast<int64_t>(min(b0 + bl, tile_end - 1)) * row);
+        auto load_pass = [&](u32x4 (&kv)[kSteps], int base) { load_vectors<kSteps, kGroup, 2>(kv, rbase, base, tile_end - 1, vecs, lane); };
+        load_pass(kv_a, b0);
         asm volatile("" ::: "memory");
 
         stage_query<kD, QT>(a, l, t.q_row, qbar);
         __syncthreads();
 
-        // Half of the thread's query values stay in registers, the other half is read from LDS again in every pass
-        // (broadcast reads, after the memory clobber that follows the prefetch): with all of them in registers the
-        // kernel needs 158 VGPRs and runs three waves per SIMD, with half it needs 126 and runs four, which is worth
-        // 8 % on long requests (80 layers x 8 requests x 523-981 blocks: 239 -> 220 us) and costs the ragged batch
-        // of 16 short requests nothing; all of them from LDS (97 VGPRs, still four waves) was 211 us there but 56
-        // instead of 51 us on the ragged batch, whose workgroups make only a few passes.
+        // A quarter of the thread's query values stay in registers (the lower half of the first steps), the others are read
+        // from LDS in every pass: 125 VGPRs and four waves per SIMD.  With half of them in registers it is 137, three waves.
         const float* qmine = &qbar[h * kD + 8 * p];
-        f32x4 ql[kSteps];
+        f32x4 ql[kKept];
 #pragma unroll
-        for (int i = 0; i < kSteps; ++i) { ql[i] = *reinterpret_cast<const f32x4*>(qmine + 16 * i); }
-        auto finish = [&](const u32x4 (&kv)[kSteps], int base) {
-            f32x4 qh[kSteps];
-#pragma unroll
-            for (int i = 0; i < kSteps; ++i) { qh[i] = *reinterpret_cast<const f32x4*>(qmine + 16 * i + 4); }
-            const float dot = pair_dot<kSteps>(ql, qh, kv);
+        for (int i = 0; i < kKept; ++i) { ql[i] = *reinterpret_cast<const f32x4*>(qmine + 16 * i); }
+        auto finish = [&](u32x4 (&kv)[kSteps], int base) {
+            const float dot = pair_dot<kSteps, kGroup, kKept>(ql, qmine, kv);
             const float s = head_sum(dot, bl * vecs * 2, 2, a.kv_heads, a.num_repre);
             // the lanes of a block all hold its score; a scale of 1 changes no bit
-            store_score(sout + min(base + bl, tile_end - 1), s * a.scale, fused);
+            tile_scores[min(base + bl, tile_end - 1) - tile0] = s * a.scale;
         };
         while (b0 < tile_end) {
             const int b1 = b0 + stride;
-            load_pass_bf16<kSteps>(kv_b, rbase + static_cast<int64_t>(min(b1 + bl, tile_end - 1)) * row);
+            load_pass(kv_b, b1);
             asm volatile("" ::: "memory");
             finish(kv_a, b0);
             if (b1 >= tile_end) { break; }
             const int b2 = b1 + stride;
-            load_pass_bf16<kSteps>(kv_a, rbase + static_cast<int64_t>(min(b2 + bl, tile_end - 1)) * row);
+            load_pass(kv_a, b2);
             asm volatile("" ::: "memory");
             finish(kv_b, b1);
             b0 = b2;
         }
     }
-    if (fused) { select_if_last(a, sel, t, l); }
+    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores);
 }
 
 template <int kD, typename QT>
@@ -519,7 +596,7 @@ int score_launch(const char* name, const void* q, int q_dtype, int64_t q_layer_s
     if (n_req == 0 || (max_seg_len == 0 && !sel)) { return UCM_OK; }
     // upper bound of sum(ceil(seg_len / tile)): exact to within n_req when the host knows the total
     const int row_bytes = vecs * head_dim * es;
-    int tile_blocks = tile_blocks_arg > 0 ? tile_blocks_arg : std::max(8, (128 * 1024) / row_bytes);
+    int tile_blocks = tile_blocks_arg > 0 ? std::min(tile_blocks_arg, kMaxTile) : std::max(8, (128 * 1024) / row_bytes);
     if (tile_blocks_arg <= 0) {
         // a launch over one layer or few short requests: smaller tiles until about half the chip's CUs have a
         // workgroup (one layer of 16 requests x 240 blocks: 16.0 us with 77 workgroups, 14.2 us with 137)

@@ -15,7 +15,8 @@ using ucm::ordered_key;
 template <int kEpl, bool kHeapTies>
 __global__ __launch_bounds__(64) void topk_windows_kernel(const ucm::SelectArgs a)
 {
-    ucm::select_wave<kEpl, kHeapTies>(a, blockIdx.x, blockIdx.y, threadIdx.x);
+    const int r = blockIdx.x;
+    ucm::select_wave<kEpl, kHeapTies>(a, r, blockIdx.y, threadIdx.x, a.seg_len[r], a.seg_off[r], a.topk_len[r]);
 }
 
 template <bool kHeapTies>

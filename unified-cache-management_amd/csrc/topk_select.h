@@ -70,22 +70,23 @@ struct SelectArgs {
 // Called by all 64 lanes of one wave for request r of layer l; kEpl * 64 is the
 // longest request the instance holds (longer ones are cut there: host checked).
 //
+// The request's own descriptors (length, first row, how many to keep) come from the caller, which may have fetched them
+// long before.
+//
 // kCoherent: the scores were written by other workgroups of the SAME launch (device-scope stores that went through
 // to memory); they are read with device-scope loads, which do not take a line that an L2 of another part of the
-// chip may still hold in an older state.
+// chip may still hold in an older state - or they are all in this workgroup's LDS (`lds`, not null).
 template <int kEpl, bool kHeapTies, bool kCoherent = false>
-__device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, int lane)
+__device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, int lane, int n, int64_t seg0, int k,
+                                            const float* lds = nullptr)
 {
     const int start_w = a.start_w, end_w = a.end_w, out_stride = a.out_stride;
     const int64_t lr = static_cast<int64_t>(l) * a.cnt_layer_stride + r;
     const int64_t row_at = static_cast<int64_t>(l) * a.idx_layer_stride + static_cast<int64_t>(r) * out_stride;
-    int n = a.seg_len[r];
     n = min(min(n, a.max_seg_len), min(out_stride, 64 * kEpl));  // host checked; clamp so nothing can run past a row
     if (a.block_tables) { n = min(n, a.bt_stride); }
-    const int64_t seg0 = a.seg_off[r];
     // a descriptor that came from device memory is followed only inside the scores of a layer
     if (seg0 < 0 || seg0 + max(n, 0) > a.scores_rows) { n = 0; }
-    const int k = a.topk_len[r];
     int32_t* out = a.idx_out + row_at;
     int32_t* pout = a.phys_out ? a.phys_out + row_at : nullptr;
     const int32_t* bt = a.block_tables ? a.block_tables + static_cast<size_t>(r) * a.bt_stride : nullptr;
@@ -120,8 +121,11 @@ __device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, i
         for (int j = 0; j < kEpl; ++j) {
             const int i = j * 64 + lane;
             const bool cand = i >= start_w && i < hi;
-            const float* sp = s + (cand ? i : 0);
-            const float sv = kCoherent ? __hip_atomic_load(sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *sp;
+            const int at = cand ? i : 0;
+            float sv;
+            if (kCoherent && lds) { sv = lds[at]; }
+            else if (kCoherent) { sv = __hip_atomic_load(s + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+            else { sv = s[at]; }
             key[j] = cand ? ordered_key(sv) : 0u;
             phys[j] = bt ? bt[min(i, n - 1)] : 0;
         }
@@ -135,6 +139,8 @@ __device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, i
 #pragma unroll
                 for (int j = 0; j < kEpl; ++j) { cnt += __popcll(__ballot(key[j] >= c)); }
                 if (cnt >= m) { T = c; }
+                // exactly m keys at or above c: they are the selection, and no lower bit can change that
+                if (cnt == m) { T = c - 1u; break; }
             }
             int greater = 0;
 #pragma unroll
