@@ -551,6 +551,7 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
     constexpr unsigned kEntrySub = kM < static_cast<int>(kSpan) ? kM : kSpan;   // kLds: sub-blocks per plane entry
     constexpr unsigned kEntryTiles = kEntrySub > kTileSub ? kEntrySub / kTileSub : 1;
     constexpr unsigned kEntriesPerBlock = kM / kEntrySub;
+    constexpr bool kWholeLines = kM >= 4;                // see load_keys
 
     extern __shared__ __attribute__((aligned(16))) unsigned short q_s[];   // [row_pad][kQStride]
     // kLds: [entry][row_pad] floats from byte plane_offset on (0 with one row tile: the queries then live in
@@ -582,6 +583,11 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
 
     // A span's keys: for each of its tiles, kSteps 16-byte loads per lane, piece 2*ks + half of the lane's
     // sub-block; the lanes of one instruction cover M*16 contiguous bytes per block and lane half.
+    // From four sub-blocks on, the two halves' pieces of a block are whole 128-byte lines in one instruction, which are
+    // then read with the non-temporal hint; with fewer an instruction takes 32 or 64 bytes of a line and the hint would
+    // lose the line before the instructions that take the rest.  512 tasks of the ragged batch, without and with the
+    // hint: 64 x 32 channels 1006 and 896 us (6.4 TB/s), 16 x 128 972 and 871, 4 x 128 268 and 241, 4 x 32 136 and 129;
+    // 2 x 128 172 and 198, 1 x 128 139 and 178 us.
     // Everything is unconditional - MFMA steps past d_pad reload piece 0 and are multiplied with a zero
     // query fragment, lanes and tiles past the workgroup's end reload its last vector and are masked or
     // never used.
@@ -599,7 +605,8 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
             const unsigned short* krow = tbase + static_cast<int64_t>(s_mine / kM) * row_stride + (s_mine % kM) * 8;
 #pragma unroll
             for (int ks = 0; ks < kSteps; ++ks) {
-                kf[t * kSteps + ks] = ucm::gload16(krow + (static_cast<unsigned>(ks) < ksteps ? ks : 0) * (16 * kM));
+                const unsigned short* piece = krow + (static_cast<unsigned>(ks) < ksteps ? ks : 0) * (16 * kM);
+                kf[t * kSteps + ks] = kWholeLines ? ucm::gload16_nt(piece) : ucm::gload16(piece);
             }
         }
         asm volatile("" ::: "memory");
