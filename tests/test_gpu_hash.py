@@ -270,6 +270,42 @@ def test_hash_query_codes_near_zero_projections_and_scales(ucm, dev):
         assert want_q[3].any() and want_q[4].any()
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("hq", [8, 40])
+@pytest.mark.parametrize("n_cols", [1, 8, 9, 32])
+def test_hash_query_few_and_many_doubtful_results_per_wave(ucm, dev, n_cols, hq, dtype):
+    """`n_cols` of a wave's 32 weight columns project every row to one term of 2^-6 .. 2^-50 of the others' size or to
+    exactly zero: up to sixteen lanes' doubtful results are redone by the whole wave and, where its sum does not settle
+    the sign, by a lane in order; more lanes redo their own (sixteen lanes are eight columns of a tile of eight rows)."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(900 + n_cols)
+    narrow = (lambda a: synth.bf16_widen(synth.bf16_round_bits(a.astype(np.float32)))) if dtype == "bf16" else \
+        (lambda a: a.astype(np.float16).astype(np.float32))
+    n_req, hkv = 6, 8
+    w = narrow(rng.standard_normal((128, 128)) * 2)
+    cols = np.concatenate([b * 32 + rng.permutation(32)[:n_cols] for b in range(4)])
+    w[1:126:2, cols] = -w[0:125:2, cols]                       # pairs that cancel, dims 0 .. 125
+    w[126, cols], w[127, cols] = 1.0, 0.0
+    q = rng.standard_normal((1, n_req, hq, 128))
+    q[..., 1:126:2] = q[..., 0:125:2]
+    e = rng.integers(6, 51 if dtype == "bf16" else 25, (1, n_req, hq))     # (float16: down to its smallest subnormals)
+    q[..., 126] = rng.choice([-1.0, 0.0, 1.0], (1, n_req, hq)) * 2.0 ** -e
+    q = narrow(q)
+    to = (lambda a: torch.from_numpy(a).to(dev).to(torch.bfloat16 if dtype == "bf16" else torch.float16))
+    q_codes = torch.full((1, n_req, hq, 16), 0xEE, dtype=torch.uint8, device=dev)
+    q_sum = torch.full((1, n_req, 128), 77, dtype=torch.int16, device=dev)
+    qbar = torch.full((1, n_req, hkv, 16), 0xEE, dtype=torch.uint8, device=dev)
+    ops.hash_encode_queries(to(q), to(w), hkv, q_codes, q_sum, qbar, n_req)
+    torch.cuda.synchronize()
+    want = O.hash_encode_f32(q[0], w)
+    assert np.array_equal(q_codes[0].cpu().numpy(), want)
+    bits = np.unpackbits(want, axis=-1, bitorder="little")
+    assert np.array_equal(bits[..., cols], np.broadcast_to((q[0, :, :, 126] > 0)[..., None], bits[..., cols].shape))
+    means = np.stack([O.q_head_mean(q[0, r], hkv) for r in range(n_req)])
+    assert np.array_equal(qbar[0].cpu().numpy(), O.hash_encode_f32(means, w))
+
+
 def test_hash_query_rows_outside_the_layer_are_skipped(ucm, dev):
     """A request whose q_rows entry is negative or past the layer's queries leaves its outputs untouched."""
     from ucm_amd import ops
