@@ -423,7 +423,8 @@ int ucm_prefetch_plan(const int32_t* map_block, const int32_t* map_len, int32_t*
  *   block_codes  dev u8 [n_layers][rows][kv_heads][16]: majority vote of each bit
  *                (colsum > 0; an exact tie gives 0), layer stride in BYTES
  *   workgroups   persistent workgroups launched over all layers, each of whose
- *                waves steps through the list of blocks; 0 = the default (4096)
+ *                waves steps through the list of blocks; 0 = the default (256 or 1024, or,
+ *                for a short list, teams of waves that share a block)
  * A block is encoded in tiles of 32 key vectors: block_size * kv_heads must be
  * a multiple of 32 (UCM_ENOTSUP otherwise; 16-token blocks need two kv heads
  * or more), kv_heads one of 1, 2, 4, 8 and block_size at most 16383.

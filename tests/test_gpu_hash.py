@@ -73,6 +73,37 @@ def test_hash_encode_blocks(ucm, dev, hkv, bs):
                        colsum[:, torch.from_numpy(slots.astype(np.int64)).to(dev)])
 
 
+@pytest.mark.parametrize("n", [1, 256, 257, 512, 513, 1024, 1025])
+@pytest.mark.parametrize("hkv,bs", [(8, 4), (8, 12), (4, 72), (1, 512)])
+def test_hash_encode_short_lists_share_blocks(ucm, dev, hkv, bs, n):
+    """A list of up to 256, 512 or 1024 blocks goes to teams of eight, four or two waves that share a block (never more waves
+    than it has tiles: 1, 3, 9 and 16 here), a longer one to single waves; bad ids, block codes and column sums of all."""
+    from ucm_amd import ops
+
+    nb = 5
+    w_bits, w_f32 = make_weights(836)
+    keys = synth.normal_bf16_bits(837, (nb, bs, hkv, 128))
+    keys[3, bs // 2:] = 0
+    ids = (np.arange(n) * 3 % nb).astype(np.int32)
+    slots = synth.permutation(838, n).astype(np.int32)
+    if n > 2:
+        ids[n // 2], slots[n - 1] = nb, -1
+    live = np.array([i for i in range(n) if ids[i] < nb and slots[i] >= 0])
+    colsum = torch.full((1, n, hkv, 128), 77, dtype=torch.int16, device=dev)
+    bcodes = torch.full((1, n, hkv, 16), 0xEE, dtype=torch.uint8, device=dev)
+    tcodes = torch.full((1, n, bs, hkv, 16), 0xEE, dtype=torch.uint8, device=dev)
+    lp = ops.LayerPointers([bf16_dev(keys, dev)])
+    ops.hash_encode_blocks(lp, i32(ids, dev), i32(slots, dev), n, bf16_dev(w_bits, dev), bs, hkv, nb, colsum, bcodes, token_codes=tcodes)
+    torch.cuda.synchronize()
+    want_t = O.hash_encode(keys, w_f32)
+    want_s, want_b = O.hash_colsum(want_t), O.hash_majority(want_t)
+    assert np.array_equal(tcodes[0].cpu().numpy()[slots[live]], want_t[ids[live]])
+    assert np.array_equal(colsum[0].cpu().numpy()[slots[live]], want_s[ids[live]])
+    assert np.array_equal(bcodes[0].cpu().numpy()[slots[live]], want_b[ids[live]])
+    rest = np.setdiff1d(np.arange(n), slots[live])
+    assert (tcodes[0].cpu().numpy()[rest] == 0xEE).all() and (colsum[0].cpu().numpy()[rest] == 77).all()
+
+
 @pytest.mark.parametrize("hkv,bs", [(8, 128), (2, 48), (1, 160), (4, 8)])
 def test_hash_encode_persistent_waves_and_queue_overflow(ucm, dev, hkv, bs):
     """One workgroup per layer walks the whole list (every wave takes several blocks, the

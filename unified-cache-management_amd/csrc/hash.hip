@@ -40,8 +40,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDim = 128;           // head_dim
 constexpr int kBits = 128;          // code length
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
 constexpr int kWtStride = kDim + 8; // bf16 elements per transposed weight row (272 B: spreads LDS banks)
 constexpr int kQueueCap = 256;
 constexpr int kMaxHeads = 8;
@@ -62,9 +60,12 @@ __device__ __forceinline__ int row_of_col(int col)
     return (col & ~31) + (i >> 2) * 8 + h * 4 + (i & 3);
 }
 
+// Ones counts of the block being encoded, per head: columns 2k and 2k+1 are the halves of word k (a block has at most
+// 16383 tokens).  Everything is added to whole words, so a correction of -1 that comes before its count borrows from the
+// neighbour only until the count is there.
 struct __attribute__((aligned(16))) WaveScratch {
     unsigned queue[kQueueCap];
-    int colsum[kMaxHeads][kBits];   // per-head ones counts of the block being encoded
+    unsigned colsum[kMaxHeads][kBits / 2];
 };
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -167,7 +168,7 @@ __device__ __attribute__((noinline)) void drain_exact(WaveScratch& ws, int qlen,
             const bool pos = exact_positive<kF16>(blk + static_cast<size_t>(v) * kDim, &neg_wt[row_of_col(col) * kWtStride]);
             if (static_cast<unsigned>(pos) != prov) {
                 if (tc_out) { atomicXor(&tc_out[v * 4 + (col >> 5)], 1u << (col & 31)); }
-                atomicAdd(&ws.colsum[v % kv_heads][col], pos ? 1 : -1);
+                atomicAdd(&ws.colsum[v % kv_heads][col >> 1], (pos ? 1u : ~0u) << (16 * (col & 1)));
             }
         }
     }
@@ -190,15 +191,15 @@ __device__ __forceinline__ void planes_add(unsigned (&pl)[kPlanes], unsigned x)
 
 // Adds the 32 counts of a plane set to the per-head column sums in LDS and clears
 // it.  Bit b of word pair `wp` is column (2*wp + b/16)*32 + half*16 + b%16.
-__device__ __forceinline__ void planes_flush(unsigned (&pl)[kPlanes], int* __restrict__ head_row, int wp, int half)
+__device__ __forceinline__ void planes_flush(unsigned (&pl)[kPlanes], unsigned* __restrict__ head_row, int wp, int half)
 {
 #pragma unroll 4
-    for (int b = 0; b < 32; ++b) {
-        int cnt = 0;
+    for (int b = 0; b < 32; b += 2) {
+        unsigned cnt = 0u;
 #pragma unroll
-        for (int p = 0; p < kPlanes; ++p) { cnt |= static_cast<int>((pl[p] >> b) & 1u) << p; }
+        for (int p = 0; p < kPlanes; ++p) { cnt |= (((pl[p] >> b) & 1u) | ((pl[p] >> (b + 1)) & 1u) << 16) << p; }
         const int col = (2 * wp + (b >> 4)) * 32 + half * 16 + (b & 15);
-        if (cnt) { atomicAdd(&head_row[col], cnt); }
+        if (cnt) { atomicAdd(&head_row[col / 2], cnt); }
     }
 #pragma unroll
     for (int p = 0; p < kPlanes; ++p) { pl[p] = 0u; }
@@ -225,9 +226,9 @@ __device__ __forceinline__ unsigned coset_add(unsigned x)
 }
 
 template <int kHeads>
-__device__ __forceinline__ void planes_flush_owner(unsigned (&pl)[kPlanes], int* __restrict__ colsum, int wp, int half, int lr)
+__device__ __forceinline__ void planes_flush_owner(unsigned (&pl)[kPlanes], unsigned* __restrict__ colsum, int wp, int half, int lr)
 {
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int j = 0; j < 8; ++j) {                        // bits 4j .. 4j+3: columns (2*wp + j/4)*32 + half*16 + 4*(j%4) + 0..3
         unsigned c = 0u;                                 // byte k: count of bit 4j + k
@@ -243,13 +244,11 @@ __device__ __forceinline__ void planes_flush_owner(unsigned (&pl)[kPlanes], int*
         if constexpr (kHeads <= 2) { even = coset_add<8>(even); odd = coset_add<8>(odd); }
         if constexpr (kHeads <= 4) { even = coset_add<16>(even); odd = coset_add<16>(odd); }
         if (lr < kHeads) {
-            int* dst = colsum + lr * kBits + (2 * wp + (j >> 2)) * 32 + half * 16 + 4 * (j & 3);
-            i32x4 v = *reinterpret_cast<i32x4*>(dst);
-            v.x += static_cast<int>(even & 0xffffu);
-            v.y += static_cast<int>(odd & 0xffffu);
-            v.z += static_cast<int>(even >> 16);
-            v.w += static_cast<int>(odd >> 16);
-            *reinterpret_cast<i32x4*>(dst) = v;
+            unsigned* dst = colsum + (lr * kBits + (2 * wp + (j >> 2)) * 32 + half * 16 + 4 * (j & 3)) / 2;
+            u32x2 v = *reinterpret_cast<u32x2*>(dst);
+            v.x += (even & 0xffffu) | (odd << 16);
+            v.y += (even >> 16) | (odd & 0xffff0000u);
+            *reinterpret_cast<u32x2*>(dst) = v;
         }
     }
 #pragma unroll
@@ -273,22 +272,117 @@ __device__ __forceinline__ void planes_flush_owner(unsigned (&pl)[kPlanes], int*
 // one kv head because kv_heads divides 32) that are added to LDS once per block.
 // Workgroups are persistent over the list of blocks so that staging the weight
 // matrix is paid once per workgroup, not once per four blocks.
-// grid: x = workgroup (wave w of workgroup g takes items g*kWaves + w, then steps by the grid), y = layer
+//
+// The keys go from memory straight to LDS (global_load_lds: sixteen bytes per lane, no registers), half a tile at a time (32
+// vectors x 64 dims = 4 KiB: whole 128-byte lines, eight adjacent lanes each), and each wave reads them back as MFMA
+// operands from a ring of three halves of its own; no barrier is involved.  Lane i of load n writes sixteen bytes at
+// n * 1024 + i * 16, so the order of the pieces inside a vector's 128 bytes is chosen on the source side: piece p of vector v
+// sits at place p ^ ((v / 2) % 8), which spreads the sixteen lanes that read the same piece of sixteen vectors over all banks.
+// That leaves room for the whole weight matrix in registers (128 of them), in the layout the A operand wants; it is fetched
+// from its LDS copy, which the exact redo uses too, once per block.
+// One workgroup of eight waves per compute unit, two waves per SIMD.  (Keys loaded into registers as the operand wants them
+// touch 64 sectors of as many vectors per instruction, and two tiles of them and the accumulators left no room for the
+// weights, which then took 32 KiB of LDS reads per tile.)
+// 32 layers x 1024 blocks of 128 tokens x 8 heads: 1.90 -> 1.85 ms with token codes (4.9 TB/s), 1.71 -> 1.61 ms without
+// (5.3 TB/s).  With the codes it is bound by memory: the same loads and stores without any arithmetic take 1.78 ms,
+// the loads alone 1.45; the arithmetic alone takes 1.28 ms.  Codes are stored with the non-temporal hint (plain: 2 % slower).
+//
+// Waits: a wave's loads complete in order, so `vmcnt(n)` with n no larger than the number of memory operations issued
+// after a half's four loads means that half has landed.  The asm statements carry a memory clobber: LDS reads stay on their
+// side of them.  A half is reloaded only after the reads of it have returned (lgkmcnt(0) in front of the loads).
+// grid: x = workgroup (wave w of workgroup g takes items g + w*gridDim.x of all layers' lists laid end to end, then steps by
+// the grid)
+constexpr int kEncWaves = 8;
+constexpr int kEncThreads = kEncWaves * 64;
+constexpr unsigned kHalfTile = 32 * 64 * 2;
+constexpr unsigned kRing = 3 * kHalfTile;
+
+struct __attribute__((aligned(128))) EncodeLds {
+    unsigned char keys[kEncWaves][kRing];
+    unsigned short wt[kBits * kWtStride];                // wt[row_of_col(col)][d] = -W[d][col]
+    WaveScratch scratch[kEncWaves];
+    float w_norm2[kBits];                                // by row of wt
+};
+static_assert(sizeof(EncodeLds) <= 160 * 1024, "LDS of a compute unit");
+
+// sixteen bytes per lane from base + offset (per lane) to LDS byte address `lds` + 16 * lane
+__device__ __forceinline__ void load_to_lds(unsigned lds, const unsigned char* base, unsigned offset)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base) : "memory", "m0");
+}
+
 template <bool kTokenCodes, bool kF16>
-__global__ __launch_bounds__(kThreads, 2) void hash_encode_blocks_kernel(
+__global__ __launch_bounds__(kEncThreads, 2) void hash_encode_blocks_kernel(
     const void* const* __restrict__ k_layers, const int32_t* __restrict__ block_ids,
-    const int32_t* __restrict__ slots, unsigned num_blocks, unsigned n_items, unsigned rows,
+    const int32_t* __restrict__ slots, unsigned num_blocks, unsigned n_items, unsigned n_layers, unsigned rows,
     unsigned tokens, unsigned kv_heads, const unsigned short* __restrict__ w,
     unsigned* __restrict__ token_codes, int64_t tc_layer_stride,
     short* __restrict__ colsum_out, int64_t cs_layer_stride,
-    unsigned* __restrict__ block_codes, int64_t bc_layer_stride)
+    unsigned* __restrict__ block_codes, int64_t bc_layer_stride, unsigned parts)
 {
-    __shared__ __attribute__((aligned(16))) unsigned short wt[kBits * kWtStride];  // wt[row_of_col(col)][d] = -W[d][col]
-    __shared__ float w_norm2[kBits];                     // by row of wt
-    __shared__ WaveScratch scratch[kWaves];
+    extern __shared__ __attribute__((aligned(128))) unsigned char encode_lds[];
+    EncodeLds& s = *reinterpret_cast<EncodeLds*>(encode_lds);
+    unsigned short* wt = s.wt;
+
+    // the wave index through readfirstlane: the item a wave works on is then known to be the same for all lanes,
+    // and its block id and slot are read with scalar loads, which do not queue behind the key loads in flight
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = lane >> 5, lr = lane & 31;
+    const unsigned n_vec = tokens * kv_heads;            // vectors of kDim bf16 in a block
+    const unsigned n_tiles = n_vec / 32;
+    // this wave's tiles of a block: all of them, or the part of a team of `parts` waves
+    const unsigned part = wave & (parts - 1);
+    const unsigned tile_begin = n_tiles * part / parts, tile_end = n_tiles * (part + 1) / parts;
+
+    // keys of an item (entry i of layer l: l * n_items + i), or null when its block id or slot is out of range (never dereferenced)
+    const unsigned all_items = n_items * n_layers;
+    auto item_keys = [&](unsigned item, unsigned& l, unsigned& slot_out) -> const unsigned short* {
+        if (item >= all_items) { return nullptr; }
+        l = item / n_items;
+        const unsigned i = item - l * n_items;
+        const unsigned id = block_ids ? static_cast<unsigned>(block_ids[i]) : i;
+        slot_out = slots ? static_cast<unsigned>(slots[i]) : i;
+        if (id >= num_blocks || slot_out >= rows) { return nullptr; }
+        return static_cast<const unsigned short*>(k_layers[l]) + static_cast<size_t>(id) * n_vec * kDim;
+    };
+
+    // ---- the ring of key halves
+    unsigned char* ring = s.keys[wave];
+    const unsigned ring_lds = __builtin_amdgcn_readfirstlane(
+        static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring)));
+    // load n of a half: lane i brings piece (i % 8) ^ (v / 2 % 8) of vector v = 8 n + i / 8 (the +4 n of v / 2 flips bit 2)
+    const unsigned from_even = (lane >> 3) * (kDim * 2) + (((lane & 7) ^ (lane >> 4)) << 4), from_odd = from_even ^ 64u;
+    auto load_half = [&](const unsigned short* blk, unsigned tile, unsigned h, unsigned at) {
+        const unsigned char* base = reinterpret_cast<const unsigned char*>(blk) + static_cast<size_t>(tile) * (2 * kHalfTile) + h * 128;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (unsigned n = 0; n < 4; ++n) { load_to_lds(ring_lds + at + n * 1024, base + n * 2048, n & 1 ? from_odd : from_even); }
+    };
+    // MFMA step ks of lane (vector lr, k-half `half`) takes dims ks*16 + half*8 .. +8, the instruction's own order: piece
+    // 2*(ks%4) + half of the vector's 128 bytes in half ks/4
+    const unsigned mine = lr * 128 + ((half ^ ((lr >> 1) & 7)) << 4);
+    auto key_piece = [&](unsigned at, int ks) { return *reinterpret_cast<const u32x4*>(ring + ((at + mine) ^ ((ks & 3) << 5))); };
+    auto next_place = [](unsigned at) { return at == 2 * kHalfTile ? 0u : at + kHalfTile; };
+    unsigned at0 = 0;                                    // where the current tile's first half is
+    bool prefetched = false;                             // the ring already holds (or awaits) this item's first three halves
+    u32x4 first_piece = {0u, 0u, 0u, 0u};                // step 0 of the next tile
+
+    // (a team takes one item, and the grid has a team for every item)
+    const unsigned item_step = gridDim.x * kEncWaves;
+    const unsigned first_item = blockIdx.x + wave / parts * gridDim.x;
+    unsigned carried_layer = 0, carried_slot = 0;        // the item looked up as the one before's successor
+    const unsigned short* carried_blk = item_keys(first_item, carried_layer, carried_slot);
+    auto load_first_halves = [&](const unsigned short* blk) {
+        load_half(blk, tile_begin, 0, at0);
+        load_half(blk, tile_begin, 1, next_place(at0));
+        load_half(blk, min(tile_begin + 1, tile_end - 1), 0, next_place(next_place(at0)));
+    };
+    // (on their way while the weights are staged: a short list is all latency)
+    bool awaited = carried_blk != nullptr;
+    if (awaited) { load_first_halves(carried_blk); }
 
     // ---- weights: global [d][col] -> LDS [col][d], sign flipped
-    for (int e8 = threadIdx.x; e8 < kDim * kBits / 8; e8 += kThreads) {
+    for (int e8 = threadIdx.x; e8 < kDim * kBits / 8; e8 += kEncThreads) {
         const int d = e8 / (kBits / 8), c0 = (e8 % (kBits / 8)) * 8;
         const u32x4 v = *reinterpret_cast<const u32x4*>(w + d * kBits + c0);
 #pragma unroll
@@ -299,86 +393,78 @@ __global__ __launch_bounds__(kThreads, 2) void hash_encode_blocks_kernel(
     }
     __syncthreads();
     {
-        const int c = threadIdx.x >> 1, part = threadIdx.x & 1;   // two threads per column, 64 dims each
-        float s = 0.0f;
+        const int c = threadIdx.x >> 2, part = threadIdx.x & 3;   // four threads per column, 32 dims each
+        float n2 = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            s = norm2_acc<kF16>(*reinterpret_cast<const u32x4*>(&wt[c * kWtStride + part * 64 + k * 8]), s);
+        for (int k = 0; k < 4; ++k) {
+            n2 = norm2_acc<kF16>(*reinterpret_cast<const u32x4*>(&wt[c * kWtStride + part * 32 + k * 8]), n2);
         }
-        s += __shfl_xor(s, 1, 64);
-        if (part == 0) { w_norm2[c] = s; }
+        n2 += __shfl_xor(n2, 1, 64);
+        n2 += __shfl_xor(n2, 2, 64);
+        if (part == 0) { s.w_norm2[c] = n2; }
     }
     __syncthreads();
 
-    // the wave index through readfirstlane: the item a wave works on is then known to be the same for all lanes,
-    // and its block id and slot are read with scalar loads, which do not queue behind the key loads in flight
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int half = lane >> 5, lr = lane & 31;
-    const unsigned l = blockIdx.y;
-    const unsigned n_vec = tokens * kv_heads;            // vectors of kDim bf16 in a block
-    const unsigned n_tiles = n_vec / 32;
-    WaveScratch& ws = scratch[wave];
-    int* head_row = &ws.colsum[lr % kv_heads][0];        // vector tile*32 + lr is a row of head lr % kv_heads
+    WaveScratch& ws = s.scratch[wave];
+    unsigned* head_row = &ws.colsum[lr % kv_heads][0];   // vector tile*32 + lr is a row of head lr % kv_heads
 
     float sw[4];                                         // tau * largest ||w_col|| of each 32-column block
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
-        float m = w_norm2[nb * 32 + lr];
+        float m = s.w_norm2[nb * 32 + lr];
 #pragma unroll
         for (int d = 16; d >= 1; d >>= 1) { m = fmaxf(m, __shfl_xor(m, d, 64)); }
-        sw[nb] = sqrtf(kTauBlocks2 * m) * 1.0001f;
+        // (the same in all lanes: a scalar register)
+        sw[nb] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sqrtf(kTauBlocks2 * m) * 1.0001f)));
     }
 
-    // keys of item i, or null when its block id or slot is out of range (never dereferenced)
-    auto item_keys = [&](unsigned i, unsigned& slot_out) -> const unsigned short* {
-        if (i >= n_items) { return nullptr; }
-        const unsigned id = block_ids ? static_cast<unsigned>(block_ids[i]) : i;
-        slot_out = slots ? static_cast<unsigned>(slots[i]) : i;
-        if (id >= num_blocks || slot_out >= rows) { return nullptr; }
-        return static_cast<const unsigned short*>(k_layers[l]) + static_cast<size_t>(id) * n_vec * kDim;
-    };
-
-    // B fragments (keys).  MFMA step ks of lane (vector lr, k-half `half`) takes dims
-    // ks*16 + half*8 .. +8, the instruction's own order: the two lanes of a vector then
-    // read neighbouring 16-byte pieces of one 32-byte sector in every load instruction, so
-    // an instruction touches 32 cache lines, not 64.  (With a lane reading its own
-    // contiguous 128-byte line over the eight steps instead - half*64 + ks*8, any order
-    // of the contraction index being fine as long as both operands agree - the kernel
-    // took 12 % more cycles with the keys from HBM and the same with the keys in cache.)
-    u32x4 k_a[8], k_b[8];
-    auto load_tile = [&](u32x4 (&kf)[8], const unsigned short* from, unsigned tile) {
-        const unsigned short* xrow = from + (static_cast<size_t>(tile) * 32 + lr) * kDim + half * 8;
+    // ---- block summaries from the counts in LDS: a wave's own, or those of its team, whose waves take turns at the heads
+    // (LDS operations of one wave complete in order; no barrier is needed inside the wave)
+    auto write_summaries = [&](unsigned l, unsigned slot) {
+        short* cs = colsum_out + (static_cast<int64_t>(l) * cs_layer_stride + static_cast<int64_t>(slot) * kv_heads * kBits);
+        unsigned* bc = block_codes + (static_cast<int64_t>(l) * bc_layer_stride + static_cast<int64_t>(slot) * kv_heads * 4);
+        const WaveScratch* team = &s.scratch[wave - part];
+        for (unsigned h = part; h < kv_heads; h += parts) {
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) { kf[ks] = ucm::gload16(xrow + ks * 16); }
+            for (int piece = 0; piece < 2; ++piece) {
+                const int col = piece * 64 + lane;
+                int n_ones = 0;
+                for (unsigned t = 0; t < parts; ++t) { n_ones += reinterpret_cast<const unsigned short*>(team[t].colsum[h])[col]; }
+                const int sgn = 2 * n_ones - static_cast<int>(tokens);
+                cs[h * kBits + col] = static_cast<short>(sgn);
+                const unsigned long long m = __ballot(sgn > 0);
+                if (lane == 0) {
+                    bc[h * 4 + piece * 2] = static_cast<unsigned>(m);
+                    bc[h * 4 + piece * 2 + 1] = static_cast<unsigned>(m >> 32);
+                }
+            }
+        }
     };
-    bool prefetched = false;                             // k_a / k_b already hold (or await) this item's first tiles
-
-    const unsigned item_step = gridDim.x * kWaves;
-    const unsigned first_item = blockIdx.x * kWaves + wave;
-    unsigned carried_slot = 0;                           // the item looked up as the one before's successor
-    const unsigned short* carried_blk = item_keys(first_item, carried_slot);
-    for (unsigned item = first_item; item < n_items; item += item_step) {
-        unsigned next_slot = 0;
-        const unsigned slot = carried_slot;
+    unsigned team_layer = 0, team_slot = 0;
+    bool has_counts = false;
+    for (unsigned item = first_item; item < all_items; item += item_step) {
+        unsigned next_layer = 0, next_slot = 0;
+        const unsigned l = carried_layer, slot = carried_slot;
         const unsigned short* blk = carried_blk;
         // the tiles after this item's last one come from the next item of this wave, so its
         // first keys are on their way while this item's summaries are written
-        const unsigned short* next_blk = item_keys(item + item_step, next_slot);
+        const unsigned short* next_blk = item_keys(item + item_step, next_layer, next_slot);
         carried_blk = next_blk;
+        carried_layer = next_layer;
         carried_slot = next_slot;
         if (!blk) { prefetched = false; continue; }
-        const bool chain = next_blk != nullptr && n_tiles >= 2;
+        const bool chain = next_blk != nullptr && n_tiles >= 2 && parts == 1;
         if (!chain) { next_blk = blk; }
         unsigned* tc_out = kTokenCodes ? token_codes + (static_cast<int64_t>(l) * tc_layer_stride +
                                                         static_cast<int64_t>(slot) * n_vec * 4) : nullptr;
-        for (int e = lane; e < kMaxHeads * kBits; e += 64) { (&ws.colsum[0][0])[e] = 0; }
+        for (int e = lane; e < kMaxHeads * kBits / 2; e += 64) { (&ws.colsum[0][0])[e] = 0u; }
 
         unsigned planes01[kPlanes], planes23[kPlanes];
 #pragma unroll
         for (int p = 0; p < kPlanes; ++p) { planes01[p] = 0u; planes23[p] = 0u; }
         unsigned pending = 0;                            // tiles counted in the planes
         int qlen = 0;
-        // inside a block of more than 63 tiles (once per 63 tiles; the three copies of the tile code each hold one)
+        // inside a block of more than 63 tiles (once per 63 tiles)
         auto flush_planes = [&]() {
             if (kv_heads == 8) {                         // (uniform)
                 planes_flush_owner<8>(planes01, &ws.colsum[0][0], 0, half, lr);
@@ -400,16 +486,25 @@ __global__ __launch_bounds__(kThreads, 2) void hash_encode_blocks_kernel(
 
         // A tile's code words are stored one trip late, at the start of the next tile's work:
         // a store issued just before the wait for the next keys would be waited for as well.
-        // The store is unconditional (a branch around it would make the compiler's wait-count
-        // bookkeeping pessimistic): the first trip writes zeros to tile 0's slot, which the
+        // The first trip writes zeros to the first tile's slot, which the
         // second trip overwrites.  The exact redo patches code words in memory, so what is
         // held here is stored before a drain and read back after it.
         typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
         u32x2 pend_cw = {0u, 0u};
-        unsigned pend_tile = 0;
+        unsigned pend_tile = tile_begin;
         auto store_codes = [&]() {
             if (kTokenCodes) {
-                *reinterpret_cast<u32x2*>(tc_out + (static_cast<size_t>(pend_tile) * 32 + lr) * 4 + half * 2) = pend_cw;
+                __builtin_nontemporal_store(pend_cw, reinterpret_cast<u32x2*>(tc_out + (static_cast<size_t>(pend_tile) * 32 + lr) * 4 + half * 2));
+            }
+        };
+        u32x4 wf[8][4];                                  // the A operand: step ks of column block nb
+        auto load_weights = [&]() {
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) {
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) {
+                    wf[ks][nb] = *reinterpret_cast<const u32x4*>(&wt[(nb * 32 + lr) * kWtStride + half * 8 + ks * 16]);
+                }
             }
         };
         auto drain_queue = [&]() {
@@ -426,77 +521,70 @@ __global__ __launch_bounds__(kThreads, 2) void hash_encode_blocks_kernel(
             }
         };
 
-        // One tile.  `kb` holds its keys; as soon as the matrix cores have consumed them the
-        // same registers are reloaded with the tile after next (of the next item at the end
-        // of this one), so two tiles are in flight per wave for most of the time without a
-        // third buffer.  The reload is unconditional: one skipped on some path would make
-        // the compiler wait for everything outstanding.
-        // Without token codes there are sixteen registers to spare, and the weight fragments of the first step
-        // of a tile stay in them for the whole kernel: no tile then starts with a wait for LDS, and an eighth of
-        // the LDS reads is gone.  With token codes the fragments are requested first thing in a tile, ahead of
-        // the wait for the keys and of their norms.
-        constexpr bool kResidentFirst = !kTokenCodes;
-        u32x4 wf_first[4];
-        if (kResidentFirst) {
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                wf_first[nb] = *reinterpret_cast<const u32x4*>(&wt[(nb * 32 + lr) * kWtStride + half * 8]);
+        if (!prefetched) {
+            if (!awaited) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (halves loaded for nobody)
+                load_first_halves(blk);
             }
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            first_piece = key_piece(at0, 0);
         }
-        auto process = [&](u32x4 (&kb)[8], unsigned tile) {
-            u32x4 wf[2][4];
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                if (kResidentFirst) { wf[0][nb] = wf_first[nb]; }
-                else { wf[0][nb] = *reinterpret_cast<const u32x4*>(&wt[(nb * 32 + lr) * kWtStride + half * 8]); }
-            }
-            __builtin_amdgcn_sched_barrier(0);
+        awaited = false;
+        prefetched = chain;
+        load_weights();
+
+#pragma unroll 1
+        for (unsigned tile = tile_begin; tile < tile_end; ++tile) {
+            const unsigned at1 = next_place(at0), at2 = next_place(at1);
             store_codes();
 
-            // ||x||^2 of vector lr, in four partial sums: one chain of thirty-two dependent dot instructions
-            // would leave the wave waiting on each one's latency
-            float xp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const unsigned e = kb[ks][j];
-                    xp[j] = dot2_self<kF16>(e, xp[j]);
-                }
-            }
-            float xn2 = (xp[0] + xp[1]) + (xp[2] + xp[3]);
-            xn2 += __shfl_xor(xn2, 32, 64);
-            const float sx = sqrtf(xn2);
-
+            // Step ks + 1 is read from LDS while the matrix instructions of step ks run; ||x||^2 of vector lr is added up
+            // between them, in four partial sums (one chain of thirty-two dependent dot instructions would leave the wave
+            // waiting on each one's latency).  A half's place is reloaded once its last step has been read: with
+            // half 1 of the next tile, and half 0 of the one after it (of the next item's at the end of this one).  The
+            // reload is unconditional, so that the waits can count on it.
             f32x16 acc[4];
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) { acc[nb][i] = 0.0f; }
             }
-            // the weight fragments of a step are read from LDS while the matrix instructions of the step before run
+            float xp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            u32x4 kf[2];
+            kf[0] = first_piece;
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks) {
-                const u32x4 kf = kb[ks];
-                if (ks < 7) {
-#pragma unroll
-                    for (int nb = 0; nb < 4; ++nb) {
-                        wf[(ks + 1) & 1][nb] = *reinterpret_cast<const u32x4*>(&wt[(nb * 32 + lr) * kWtStride + half * 8 + (ks + 1) * 16]);
-                    }
-                }
+                if (ks == 3) { asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); }   // (only half 0 of the next tile came later)
+                if (ks < 7) { kf[(ks + 1) & 1] = key_piece(ks < 3 ? at0 : at1, ks + 1); }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int nb = 0; nb < 4; ++nb) {
-                    acc[nb] = mfma_32x32x16<kF16>(wf[ks & 1][nb], kf, acc[nb]);
+                    acc[nb] = mfma_32x32x16<kF16>(wf[ks][nb], kf[ks & 1], acc[nb]);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const unsigned e = kf[ks & 1][j];
+                    xp[j] = dot2_self<kF16>(e, xp[j]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+                if (ks == 3) {
+                    const bool over = tile + 1 >= tile_end;
+                    load_half(over ? next_blk : blk, over ? (chain ? 0u : tile_end - 1) : tile + 1, 1, at0);
+                }
             }
             {
                 const unsigned t2 = tile + 2;
-                const bool over = t2 >= n_tiles;
-                load_tile(kb, over ? next_blk : blk, over ? (chain ? t2 - n_tiles : n_tiles - 1) : t2);
+                const bool over = t2 >= tile_end;
+                load_half(over ? next_blk : blk, over ? (chain ? t2 - tile_end : tile_end - 1) : t2, 0, at1);
             }
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");       // half 0 of the next tile: two halves came after it
+            first_piece = key_piece(at2, 0);
+            at0 = at2;
             __builtin_amdgcn_sched_barrier(0);
+            float xn2 = (xp[0] + xp[1]) + (xp[2] + xp[3]);
+            const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(xn2), __float_as_uint(xn2), false, false);
+            xn2 = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+            const float sx = sqrtf(xn2);
 
             // sign bits -> compact words: bit 16*(nb%2) + i of pair nb/2 is accumulator i of block nb
             unsigned pair[2];
@@ -556,7 +644,7 @@ __global__ __launch_bounds__(kThreads, 2) void hash_encode_blocks_kernel(
                         const unsigned signs = pair[nb >> 1] >> (16 * (nb & 1));
                         unsigned long long um = __ballot(mask != 0u);
                         while (um) {
-                            if (qlen + 64 > kQueueCap) { drain_queue(); }
+                            if (qlen + 64 > kQueueCap) { drain_queue(); load_weights(); }
                             if (mask) {
                                 const unsigned i = static_cast<unsigned>(__builtin_ctz(mask));
                                 mask &= mask - 1u;
@@ -575,49 +663,21 @@ __global__ __launch_bounds__(kThreads, 2) void hash_encode_blocks_kernel(
                 flush_planes();
                 pending = 0;
             }
-        };
-
-        if (!prefetched) {
-            load_tile(k_a, blk, 0);
-            load_tile(k_b, blk, min(1u, n_tiles - 1));
-        }
-        prefetched = chain;
-        unsigned tile = 0;
-#pragma unroll 1
-        for (; tile + 1 < n_tiles; tile += 2) {
-            process(k_a, tile);
-            process(k_b, tile + 1);
-        }
-        if (tile < n_tiles) {
-            process(k_a, tile);
-            // an odd tile count leaves the next item's tile 0 in k_b and its tile 1 in k_a
-            if (chain) {
-#pragma unroll
-                for (int ks = 0; ks < 8; ++ks) { const u32x4 t = k_a[ks]; k_a[ks] = k_b[ks]; k_b[ks] = t; }
-            }
         }
         store_codes();
         if (qlen > 0) { drain_exact<kF16>(ws, qlen, lane, blk, wt, tc_out, kv_heads); }
         flush_planes_last();
 
-        // ---- block summaries
-        // (LDS operations of one wave complete in order; no barrier is needed inside the wave)
-        short* cs = colsum_out + (static_cast<int64_t>(l) * cs_layer_stride + static_cast<int64_t>(slot) * kv_heads * kBits);
-        unsigned* bc = block_codes + (static_cast<int64_t>(l) * bc_layer_stride + static_cast<int64_t>(slot) * kv_heads * 4);
-        for (unsigned h = 0; h < kv_heads; ++h) {
-#pragma unroll
-            for (int part = 0; part < 2; ++part) {
-                const int col = part * 64 + lane;
-                const int n_ones = ws.colsum[h][col];
-                const int sgn = 2 * n_ones - static_cast<int>(tokens);
-                cs[h * kBits + col] = static_cast<short>(sgn);
-                const unsigned long long m = __ballot(sgn > 0);
-                if (lane == 0) {
-                    bc[h * 4 + part * 2] = static_cast<unsigned>(m);
-                    bc[h * 4 + part * 2 + 1] = static_cast<unsigned>(m >> 32);
-                }
-            }
-        }
+        team_layer = l;
+        team_slot = slot;
+        has_counts = true;
+        if (parts > 1) { break; }
+        write_summaries(l, slot);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may still be on its way to LDS when the wave ends
+    if (parts > 1) {
+        __syncthreads();                                 // (every wave comes here once)
+        if (has_counts) { write_summaries(team_layer, team_slot); }
     }
 }
 
@@ -1158,7 +1218,6 @@ int hash_encode_blocks(bool f16, const void* const* k_layers, int n_layers, int 
 {
     UCM_REQUIRE(n >= 0, "ucm_hash_encode_blocks: n=%d", n);
     UCM_REQUIRE(workgroups >= 0 && workgroups <= (1 << 20), "ucm_hash_encode_blocks: workgroups=%d", workgroups);
-    const int encode_groups = workgroups > 0 ? workgroups : 4096;
     if (n == 0) { return UCM_OK; }
     UCM_REQUIRE(k_layers && w_bf16 && colsum && block_codes, "ucm_hash_encode_blocks: null pointer");
     UCM_REQUIRE(n_layers > 0 && n_layers <= 65535 && num_blocks > 0 && rows > 0 && block_size > 0,
@@ -1172,22 +1231,52 @@ int hash_encode_blocks(bool f16, const void* const* k_layers, int n_layers, int 
                 "ucm_hash_encode_blocks: token_codes must be 16-byte aligned");
     UCM_REQUIRE(token_codes_layer_stride % 4 == 0 && block_codes_layer_stride % 4 == 0,
                 "ucm_hash_encode_blocks: code strides are in bytes and must be multiples of 4");
-    // persistent workgroups: about 4096 of them over all layers, each wave stepping through the list
-    const int groups = (n + kWaves - 1) / kWaves;
-    const int gx = std::min(groups, std::max(1, (encode_groups + n_layers - 1) / n_layers));
-#define UCM_HASH_ENCODE_ARGS dim3(gx, n_layers), dim3(kThreads), 0, ucm::as_stream(stream), k_layers, block_ids, slots, \
-        static_cast<unsigned>(num_blocks), static_cast<unsigned>(n), static_cast<unsigned>(rows),                        \
-        static_cast<unsigned>(block_size), static_cast<unsigned>(kv_heads), static_cast<const unsigned short*>(w_bf16),  \
-        reinterpret_cast<unsigned*>(token_codes), token_codes_layer_stride / 4, colsum, colsum_layer_stride,             \
-        reinterpret_cast<unsigned*>(block_codes), block_codes_layer_stride / 4
-    if (f16) {
-        if (token_codes) { hipLaunchKernelGGL((hash_encode_blocks_kernel<true, true>), UCM_HASH_ENCODE_ARGS); }
-        else { hipLaunchKernelGGL((hash_encode_blocks_kernel<false, true>), UCM_HASH_ENCODE_ARGS); }
-    } else {
-        if (token_codes) { hipLaunchKernelGGL((hash_encode_blocks_kernel<true, false>), UCM_HASH_ENCODE_ARGS); }
-        else { hipLaunchKernelGGL((hash_encode_blocks_kernel<false, false>), UCM_HASH_ENCODE_ARGS); }
+    const void* kernel = f16 ? (token_codes ? reinterpret_cast<const void*>(hash_encode_blocks_kernel<true, true>)
+                                            : reinterpret_cast<const void*>(hash_encode_blocks_kernel<false, true>))
+                             : (token_codes ? reinterpret_cast<const void*>(hash_encode_blocks_kernel<true, false>)
+                                            : reinterpret_cast<const void*>(hash_encode_blocks_kernel<false, false>));
+    if (int rc = ucm::check_hip(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(EncodeLds)),
+                                "ucm_hash_encode_blocks (LDS size)")) {
+        return rc;
     }
+    // Persistent workgroups, each wave stepping through the list - or, when the list is too short for that to fill the
+    // chip's 2048 waves, teams of two, four or eight waves of a workgroup that share a block: one layer's 8 or 100
+    // blocks of 32 tiles take 21 us with teams of eight and 50 us with lone waves; 300 blocks 33 us, 900 64 us.
+    // A call that names its number of workgroups has that many walk the list.  (Items are numbered in 31 bits: a list longer
+    // than that over all layers goes out a few layers at a time.)
+    const int chunk = std::min(n_layers, std::max(1, 0x7fffffff / n));
+    for (int l0 = 0; l0 < n_layers; l0 += chunk) {
+        const int layers = std::min(chunk, n_layers - l0);
+        const int64_t items = static_cast<int64_t>(n) * layers;
+        int parts = 1;
+        if (workgroups == 0) {
+            while (parts < kEncWaves && parts * 2 <= block_size * kv_heads / 32 && items * parts * 2 <= 256 * kEncWaves) { parts *= 2; }
+        }
+        const int teams = kEncWaves / parts;
+        const int64_t full = (items + teams - 1) / teams;     // workgroups when every one of their teams has an item
+        int64_t gx = std::max(full, std::min<int64_t>(items, 256));
+        if (workgroups > 0) { gx = std::min<int64_t>(full, workgroups); }
+        // One workgroup per compute unit, until the waves have eight items each: from there on four per compute unit even
+        // out how fast the units get through theirs (2700 blocks: 174 us with one, 196 with 339 workgroups; 32768
+        // blocks: 1.87 and 1.85 ms).
+        else if (parts == 1) { gx = std::min<int64_t>(gx, items <= 8 * 256 * kEncWaves ? 256 : 1024); }
+        unsigned* tc = token_codes ? reinterpret_cast<unsigned*>(token_codes + l0 * token_codes_layer_stride) : nullptr;
+#define UCM_HASH_ENCODE_ARGS dim3(static_cast<unsigned>(gx)), dim3(kEncThreads), sizeof(EncodeLds), ucm::as_stream(stream),  \
+        k_layers + l0, block_ids, slots, static_cast<unsigned>(num_blocks), static_cast<unsigned>(n),                     \
+        static_cast<unsigned>(layers), static_cast<unsigned>(rows), static_cast<unsigned>(block_size),                   \
+        static_cast<unsigned>(kv_heads), static_cast<const unsigned short*>(w_bf16), tc, token_codes_layer_stride / 4,   \
+        colsum + l0 * colsum_layer_stride, colsum_layer_stride,                                                          \
+        reinterpret_cast<unsigned*>(block_codes + l0 * block_codes_layer_stride), block_codes_layer_stride / 4,          \
+        static_cast<unsigned>(parts)
+        if (f16) {
+            if (token_codes) { hipLaunchKernelGGL((hash_encode_blocks_kernel<true, true>), UCM_HASH_ENCODE_ARGS); }
+            else { hipLaunchKernelGGL((hash_encode_blocks_kernel<false, true>), UCM_HASH_ENCODE_ARGS); }
+        } else {
+            if (token_codes) { hipLaunchKernelGGL((hash_encode_blocks_kernel<true, false>), UCM_HASH_ENCODE_ARGS); }
+            else { hipLaunchKernelGGL((hash_encode_blocks_kernel<false, false>), UCM_HASH_ENCODE_ARGS); }
+        }
 #undef UCM_HASH_ENCODE_ARGS
+    }
     UCM_LAUNCH_CHECK("ucm_hash_encode_blocks");
 }
 
