@@ -251,28 +251,40 @@ __global__ __launch_bounds__(kPlanThreads) void delta_plan_wide_kernel(
     bool keep[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) { hit_slot[e] = -1; keep[e] = false; }
-    const int res_quads = (n_slots + 3) >> 2, sel_quads = (k + 3) >> 2;
-    for (int q = 0; q < res_quads; ++q) {
-        const int4 v = *reinterpret_cast<const int4*>(&s_res[q * 4]);
+    // sixteen entries per trip, their reads issued together (past the lists the arrays hold -1): a trip of four is one
+    // LDS latency long, and a budget of 153 slots walks two lists of them
+    // (16 requests: 8.8 us that way, 7.3 this way)
+    for (int i0 = 0; i0 < n_slots; i0 += 16) {
+        int4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { v[u] = *reinterpret_cast<const int4*>(&s_res[i0 + u * 4]); }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             if (my_sel[e] >= 0) {   // the last matching slot wins, as in the one-wave kernel
-                if (v.x == my_sel[e]) { hit_slot[e] = q * 4; }
-                if (v.y == my_sel[e]) { hit_slot[e] = q * 4 + 1; }
-                if (v.z == my_sel[e]) { hit_slot[e] = q * 4 + 2; }
-                if (v.w == my_sel[e]) { hit_slot[e] = q * 4 + 3; }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (v[u].x == my_sel[e]) { hit_slot[e] = i0 + u * 4; }
+                    if (v[u].y == my_sel[e]) { hit_slot[e] = i0 + u * 4 + 1; }
+                    if (v[u].z == my_sel[e]) { hit_slot[e] = i0 + u * 4 + 2; }
+                    if (v[u].w == my_sel[e]) { hit_slot[e] = i0 + u * 4 + 3; }
+                }
             }
         }
     }
-    for (int q = 0; q < sel_quads; ++q) {
-        const int4 v = *reinterpret_cast<const int4*>(&s_sel[q * 4]);
+    for (int i0 = 0; i0 < k; i0 += 16) {
+        int4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { v[u] = *reinterpret_cast<const int4*>(&s_sel[i0 + u * 4]); }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            if (my_res[e] >= 0 && (v.x == my_res[e] || v.y == my_res[e] || v.z == my_res[e] || v.w == my_res[e])) {
-                keep[e] = true;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (v[u].x == my_res[e] || v[u].y == my_res[e] || v[u].z == my_res[e] || v[u].w == my_res[e]) { keep[e] = true; }
             }
         }
     }
+#pragma unroll
+    for (int e = 0; e < E; ++e) { keep[e] = keep[e] && my_res[e] >= 0; }
 
     bool miss[E], freed[E];
     int miss_rank[E], free_rank[E];
