@@ -201,41 +201,36 @@ def score_select(q: torch.Tensor, repre: torch.Tensor, seg_off: torch.Tensor, se
                  scale: float = 1.0, num_repre: int = 1, tile_blocks: int = 0, total_blocks: int = 0) -> None:
     """score_blocks and topk_windows as one launch (ucm_score_select): q [L, rows, q_heads, head_dim] whose layer 0
     belongs to ``first_layer``... of the tables; tickets int32 [L, n_req], zero before the first call and left zero."""
-    if q.dim() != 4 or repre.dim() != 3 or scores.dim() != 2:
+    qs, rs, ss, idx_shape, cnt_shape = q.shape, repre.shape, scores.shape, idx_out.shape, count_out.shape
+    if len(qs) != 4 or len(rs) != 3 or len(ss) != 2:
         raise ValueError("q [L,rows,Hq,D], repre [L,rows,Hkv*D], scores [L,rows] expected")
-    head_dim, q_heads = q.shape[3], q.shape[2]
-    if repre.shape[2] != kv_heads * num_repre * head_dim:
+    head_dim, q_heads = qs[3], qs[2]
+    if rs[2] != kv_heads * num_repre * head_dim:
         raise ValueError("repre row does not match kv_heads*num_repre*head_dim")
     n_req = seg_off.numel()
-    n_layers = q.shape[0] if n_layers is None else n_layers
-    if first_layer < 0 or first_layer + n_layers > min(repre.shape[0], scores.shape[0], idx_out.shape[0]) or n_layers > q.shape[0]:
+    n_layers = qs[0] if n_layers is None else n_layers
+    if first_layer < 0 or first_layer + n_layers > min(rs[0], ss[0], idx_shape[0]) or n_layers > qs[0]:
         raise ValueError("layer range outside the tables")
-    if idx_out.dim() != 3 or idx_out.shape[1] != n_req or count_out.shape != idx_out.shape[:2] or tickets.shape != count_out.shape:
+    if len(idx_shape) != 3 or idx_shape[1] != n_req or cnt_shape != idx_shape[:2] or tickets.shape != cnt_shape:
         raise ValueError("idx_out [L,n_req,stride], count_out and tickets [L,n_req] expected")
-    if scores.shape[1] < repre.shape[1]:
+    if ss[1] < rs[1]:
         raise ValueError("scores row shorter than the representative table")
-    if phys_out is not None and phys_out.shape != idx_out.shape:
+    if phys_out is not None and phys_out.shape != idx_shape:
         raise ValueError("phys_out must have idx_out's shape")
-    if sparse_seq_lens is not None and sparse_seq_lens.shape != count_out.shape:
+    if sparse_seq_lens is not None and sparse_seq_lens.shape != cnt_shape:
         raise ValueError("sparse_seq_lens must have count_out's shape")
-    args = _lib.ScoreSelectArgs(
-        q=_dev(q, q.dtype, "q"), q_dtype=_q_code(q), q_heads=q_heads, q_layer_stride=q.stride(0),
-        q_rows=_opt(q_rows, torch.int32, "q_rows"), repre=_dev(repre, repre.dtype, "repre"),
-        repre_dtype=_lib.DTYPE_BF16 if repre.dtype == torch.bfloat16 else _lib.DTYPE_F32,
-        repre_layer_stride=repre.stride(0), repre_rows=repre.shape[1], seg_off=_dev(seg_off, torch.int32, "seg_off"),
-        seg_len=_dev(seg_len, torch.int32, "seg_len"), topk_len=_dev(topk_len, torch.int32, "topk_len"), n_req=n_req,
-        max_seg_len=max_seg_len, first_layer=first_layer, kv_heads=kv_heads, head_dim=head_dim,
-        scores=_dev(scores, torch.float32, "scores"), scores_layer_stride=scores.stride(0), tile_blocks=int(tile_blocks),
-        start_w=start_w, end_w=end_w, idx_out=_dev(idx_out, torch.int32, "idx_out"),
-        count_out=_dev(count_out, torch.int32, "count_out"), out_stride=idx_out.shape[2],
-        bt_stride=0 if block_tables is None else block_tables.shape[1],
-        block_tables=_opt(block_tables, torch.int32, "block_tables"), phys_out=_opt(phys_out, torch.int32, "phys_out"),
-        seq_lens=_opt(seq_lens, torch.int32, "seq_lens"), sparse_seq_lens=_opt(sparse_seq_lens, torch.int32, "sparse_seq_lens"),
-        block_size=block_size, tickets=_dev(tickets, torch.int32, "tickets"))
-    args.n_layers, args.num_repre, args.scale, args.total_blocks = n_layers, num_repre, float(scale), int(total_blocks)
-    import ctypes as C
-
-    _lib.call("ucm_score_select", C.addressof(args), _stream())
+    i32 = torch.int32
+    args = _lib.pack_score_select(
+        _dev(q, q.dtype, "q"), _q_code(q), q_heads, q.stride(0), _opt(q_rows, i32, "q_rows") or 0,
+        _dev(repre, repre.dtype, "repre"), _lib.DTYPE_BF16 if repre.dtype == torch.bfloat16 else _lib.DTYPE_F32, num_repre,
+        repre.stride(0), rs[1], _dev(seg_off, i32, "seg_off"), _dev(seg_len, i32, "seg_len"),
+        _dev(topk_len, i32, "topk_len"), n_req, max_seg_len, first_layer, n_layers, kv_heads, head_dim,
+        _dev(scores, torch.float32, "scores"), scores.stride(0), scale, int(tile_blocks), start_w, end_w,
+        _dev(idx_out, i32, "idx_out"), _dev(count_out, i32, "count_out"), idx_shape[2],
+        0 if block_tables is None else block_tables.shape[1], _opt(block_tables, i32, "block_tables") or 0,
+        _opt(phys_out, i32, "phys_out") or 0, _opt(seq_lens, i32, "seq_lens") or 0,
+        _opt(sparse_seq_lens, i32, "sparse_seq_lens") or 0, block_size, 0, _dev(tickets, i32, "tickets"), 0, 0, int(total_blocks))
+    _lib.call("ucm_score_select", args, _stream())
 
 
 def topk_windows(scores: torch.Tensor, seg_off: torch.Tensor, seg_len: torch.Tensor, topk_len: torch.Tensor,
