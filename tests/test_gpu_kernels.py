@@ -621,6 +621,40 @@ def test_kv_moves_of_one_tensor_parallel_rank(ucm, dev):
         ops.kv_gather_blocks(ops.LayerPointers(ranks[0][1]), nb * bb, bb, nb, i32(ids, dev), staging, rank=4, tp_size=4)
 
 
+@pytest.mark.parametrize("n_slots,bb", [(1, 16), (64, 131072), (65, 131072 + 16), (1023, 48), (1024, 64), (1025, 16400), (40, 262144)])
+def test_planned_loads_of_scattered_slots(ucm, dev, n_slots, bb):
+    """Plans whose entries to load are scattered over a row: rows of up to, exactly and beyond the 1024 slots a workgroup lists
+    at once, slices of less than a piece, one piece, a piece and sixteen bytes, two pieces; entries that are out of range
+    anywhere, an empty row, a full row and a row outside the call's are left alone."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(930 + n_slots)
+    n_layers, rows_n, stored, src_n = 2, 4, 7, 9
+    nb = n_slots + 3
+    pool = rng.integers(0, 256, (stored, n_layers, 2, bb), dtype=np.uint8)
+    load = np.where(rng.random((n_layers, rows_n, n_slots)) < 0.3, rng.integers(0, src_n, (n_layers, rows_n, n_slots)), -1).astype(np.int32)
+    load[:, 1], load[0, 2] = -1, 5
+    load[:, 0, 0] = src_n                                        # past the table of stored blocks
+    src = rng.integers(0, stored, (rows_n, src_n)).astype(np.int32)
+    src[:, 3], src[:, 4] = -1, stored                            # not in the pool
+    dst = np.stack([rng.permutation(nb)[:n_slots] for _ in range(rows_n)]).astype(np.int32)
+    dst[0, n_slots // 2] = nb
+    for use in (np.array([2, -1, 0, 1, rows_n], np.int32), np.array([2], np.int32)):
+        # one request's destinations at a time are distinct, those of several may meet: give each row a cache of its own
+        for r in (use if len(use) == 1 else [2, 0]):
+            caches = [torch.full((2, nb, bb), 0xEE, dtype=torch.uint8, device=dev) for _ in range(n_layers)]
+            only = np.array([x if x in (r, -1, 1, rows_n) else -1 for x in use], np.int32)
+            ops.kv_load_planned(ops.LayerPointers(caches), 0, 0, n_layers, nb * bb, bb, nb, torch.from_numpy(pool).to(dev).view(-1),
+                                n_layers * 2 * bb, i32(load, dev), i32(src, dev), i32(dst, dev), i32(only, dev))
+            for l in range(n_layers):
+                want = np.full((2, nb, bb), 0xEE, np.uint8)
+                for j in range(n_slots):
+                    e = load[l, r, j]
+                    if 0 <= e < src_n and 0 <= src[r, e] < stored and 0 <= dst[r, j] < nb:
+                        want[:, dst[r, j]] = pool[src[r, e], l]
+                assert np.array_equal(caches[l].cpu().numpy(), want), (r, l)
+
+
 def test_copy_batch_pointer_arrays(ucm, dev):
     from ucm_amd import ops
 
