@@ -181,8 +181,11 @@ __global__ __launch_bounds__(kThreads) void kv_load_planned_kernel(
 
 // The same loads when every row says how many of its leading entries are loads (load_count): the work is
 // known exactly, so it is dealt out evenly.  Every workgroup builds the running total of the (layer, request)
-// pairs' counts in LDS (a few hundred integers), and takes the copies w, w + grid, ... of the 2 * total
-// (K and V); which pair a copy belongs to is a binary search in the totals.  grid: x = workgroup.
+// pairs' counts in LDS (a few hundred integers), and takes the pieces w, w + grid, ... of the 2 * total slices
+// (K and V); which pair a slice belongs to is a binary search in the totals.
+// (Pieces of one 128 KiB trip, and a running total by wave scans: 47 loads of one layer 21.4 us with whole slices and a scan
+// of ten barriers, 15.7 so; 116 loads 29.5 and 27.4; 887 loads of 8 layers 170.7 and 169.8.)
+// grid: x = workgroup.
 constexpr unsigned kMaxPlannedPairs = 4096;
 
 __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
     unsigned n_layers, StoredLayout lay)
 {
     __shared__ unsigned s_total[kMaxPlannedPairs + 1];   // s_total[p] = loads of the pairs before p
-    __shared__ unsigned s_part[kThreads];
+    __shared__ unsigned s_part[kThreads / 64];
     const unsigned pairs = n_layers * batch;             // pair p = layer p / batch, request p % batch
     constexpr unsigned kPer = kMaxPlannedPairs / kThreads;
     unsigned mine[kPer], sum = 0;
@@ -212,15 +215,17 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
         mine[i] = c;
         sum += c;
     }
-    s_part[threadIdx.x] = sum;
-    __syncthreads();
-    for (unsigned d = 1; d < kThreads; d <<= 1) {         // inclusive scan of the threads' sums
-        const unsigned v = threadIdx.x >= d ? s_part[threadIdx.x - d] : 0u;
-        __syncthreads();
-        s_part[threadIdx.x] += v;
-        __syncthreads();
+    // running total of the threads' sums: inside a wave, then over the waves before it
+    unsigned incl = sum;
+#pragma unroll
+    for (unsigned d = 1; d < 64; d <<= 1) {
+        const unsigned v = __shfl_up(incl, d, 64);
+        if ((threadIdx.x & 63) >= d) { incl += v; }
     }
-    unsigned run = s_part[threadIdx.x] - sum;
+    if ((threadIdx.x & 63) == 63) { s_part[threadIdx.x >> 6] = incl; }
+    __syncthreads();
+    unsigned run = incl - sum;
+    for (unsigned w = 0; w < kThreads / 64; ++w) { run += w < threadIdx.x >> 6 ? s_part[w] : 0u; }
 #pragma unroll
     for (unsigned i = 0; i < kPer; ++i) {
         s_total[threadIdx.x * kPer + i] = run;
@@ -228,9 +233,11 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
     }
     if (threadIdx.x == kThreads - 1) { s_total[kMaxPlannedPairs] = run; }
     __syncthreads();
-    const unsigned copies = 2u * s_total[kMaxPlannedPairs];
-    for (unsigned w = blockIdx.x; w < copies; w += gridDim.x) {   // (uniform in the workgroup)
-        const unsigned t = w >> 1, kv = w & 1u;
+    const unsigned pieces = static_cast<unsigned>((block_bytes + kLoadPiece - 1) / kLoadPiece);
+    const uint64_t units = static_cast<uint64_t>(2u * s_total[kMaxPlannedPairs]) * pieces;
+    for (uint64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {   // (uniform in the workgroup)
+        const unsigned w = static_cast<unsigned>(unit / pieces), t = w >> 1, kv = w & 1u;
+        const size_t off = static_cast<size_t>(unit - static_cast<uint64_t>(w) * pieces) * kLoadPiece;
         unsigned lo = 0, hi = pairs;                     // last pair whose running total is <= t
         while (hi - lo > 1) {
             const unsigned mid = (lo + hi) >> 1;
@@ -244,9 +251,9 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
         if (src < 0 || static_cast<uint64_t>(src) >= pool_blocks) { continue; }
         const unsigned dst = static_cast<unsigned>(dst_table[l * dst_layer_stride + static_cast<int64_t>(row) * dst_stride + j]);
         if (dst >= num_blocks) { continue; }
-        copy_slice(static_cast<uint8_t*>(layers[l]) + kv * kv_stride + static_cast<size_t>(dst) * block_bytes,
-                   pool + static_cast<size_t>(src) * pool_block_bytes + lay.slice(store_first_layer + l, kv, block_bytes),
-                   block_bytes);
+        copy_slice(static_cast<uint8_t*>(layers[l]) + kv * kv_stride + static_cast<size_t>(dst) * block_bytes + off,
+                   pool + static_cast<size_t>(src) * pool_block_bytes + lay.slice(store_first_layer + l, kv, block_bytes) + off,
+                   min(kLoadPiece, block_bytes - off));
     }
 }
 
