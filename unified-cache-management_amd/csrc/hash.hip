@@ -3,9 +3,9 @@
 //
 // The projection [vectors x 128] . [128 x 128] is the one real contraction on
 // the whole retrieval path (128 flop per byte of key), so it runs on the matrix
-// cores: v_mfma_f32_32x32x16_bf16, one wave per cache block, 32-vector tiles,
-// the weight matrix staged once per workgroup in LDS (transposed, padded rows,
-// sign flipped).
+// cores: v_mfma_f32_32x32x16_bf16, a wave (or a team of waves) per cache block,
+// 32-vector tiles, the keys through LDS and the weight matrix in registers (its
+// transposed, sign-flipped copy in LDS serves the exact redo).
 // Only the SIGN of each projection is kept, and it has to be the sign of the
 // exactly accumulated dot product (the CPU oracle accumulates in fp64), so
 // every result whose magnitude is within the fp32 accumulation error bound
