@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kEncThreads, 2) void hash_encode_blocks_kernel(
             for (int piece = 0; piece < 2; ++piece) {
                 const int col = piece * 64 + lane;
                 int n_ones = 0;
-                for (unsigned t = 0; t < parts; ++t) { n_ones += reinterpret_cast<const unsigned short*>(team[t].colsum[h])[col]; }
+                for (unsigned t = 0; t < parts; ++t) { n_ones += static_cast<int>((team[t].colsum[h][col >> 1] >> (16 * (col & 1))) & 0xffffu); }
                 const int sgn = 2 * n_ones - static_cast<int>(tokens);
                 cs[h * kBits + col] = static_cast<short>(sgn);
                 const unsigned long long m = __ballot(sgn > 0);
