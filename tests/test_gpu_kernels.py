@@ -655,6 +655,46 @@ def test_planned_loads_of_scattered_slots(ucm, dev, n_slots, bb):
                 assert np.array_equal(caches[l].cpu().numpy(), want), (r, l)
 
 
+@pytest.mark.parametrize("counted", [False, True])
+@pytest.mark.parametrize("n_layers,rows_n,n_slots,bb", [
+    (2, 4, 9, 32768 + 16), (1, 3, 5, 32768), (1, 3, 7, 48), (2, 3, 5, 4 * 131072 + 4096),      # small launches, each size of workgroup
+    (8, 9, 60, 65536), (8, 9, 60, 65536 + 16), (8, 9, 60, 131072), (8, 9, 60, 49152),          # large ones: a piece, a piece and a remainder, two
+    (8, 9, 40, 131072 + 16), (4, 8, 40, 262144),                                              # the list: pieces of a longer slice
+    (65, 64, 3, 48), (65, 64, 1, 32768 + 16)])                                                # more rows than the counted kernel's table
+def test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_slots, bb, counted):
+    """The rule that picks how a plan's loads are dealt out, on both sides of its bounds, with and without counts; with
+    them a row's first entries load and what stands behind the count is left alone."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(n_slots + bb)
+    stored, src_n = 5, 6
+    nb = rows_n * n_slots + 2
+    pool = rng.integers(0, 256, (stored, n_layers, 2, bb), dtype=np.uint8)
+    load = np.where(rng.random((n_layers, rows_n, n_slots)) < 0.4, rng.integers(0, src_n, (n_layers, rows_n, n_slots)), -1).astype(np.int32)
+    count = rng.integers(-1, n_slots + 2, (n_layers, rows_n)).astype(np.int32)
+    src = rng.integers(0, stored, (rows_n, src_n)).astype(np.int32)
+    src[:, 2] = stored                                            # not in the pool
+    dst = rng.permutation(nb)[: rows_n * n_slots].reshape(rows_n, n_slots).astype(np.int32)
+    dst[rows_n // 2, 0] = nb
+    caches = torch.full((n_layers, 2, nb, bb), 0xEE, dtype=torch.uint8, device=dev)
+    ops.kv_load_planned(ops.LayerPointers([caches[l] for l in range(n_layers)]), 0, 0, n_layers, nb * bb, bb, nb,
+                        torch.from_numpy(pool).to(dev).view(-1), n_layers * 2 * bb, i32(load, dev), i32(src, dev), i32(dst, dev), None,
+                        load_count=i32(count, dev) if counted else None)
+    pool_d = torch.from_numpy(pool).to(dev)
+    for l in range(n_layers):
+        want = torch.full((2, nb, bb), 0xEE, dtype=torch.uint8, device=dev)
+        at, what = [], []
+        for r in range(rows_n):
+            for j in range(min(n_slots, max(int(count[l, r]), 0)) if counted else n_slots):
+                e = load[l, r, j]
+                if 0 <= e < src_n and src[r, e] < stored and dst[r, j] < nb:
+                    at.append(int(dst[r, j]))
+                    what.append(int(src[r, e]))
+        if at:
+            want[:, at] = pool_d[what, l].transpose(0, 1)
+        assert torch.equal(caches[l], want), l
+
+
 def test_copy_batch_pointer_arrays(ucm, dev):
     from ucm_amd import ops
 

@@ -21,32 +21,34 @@ constexpr size_t kStep = static_cast<size_t>(kThreads) * 16 * kUnroll;  // 128 K
 // kN x 16 KiB of a slice: every load is issued before the first store goes out.  Stores that start as the
 // loads trickle in mix reads and writes on the HBM channels and cost about 6 % of the copy rate (1.64 ms ->
 // 1.75 ms for the 5.1 GB gather), hence the wait for ALL of the trip's loads.
-template <int kN>
+template <int kN, int kT = kThreads>
 __device__ __forceinline__ void copy_trip(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t base)
 {
     u32x4 v[kN];
 #pragma unroll
     for (int u = 0; u < kN; ++u) {
-        v[u] = ucm::gload16_nt(src + base + static_cast<size_t>(u) * kThreads * 16);
+        v[u] = ucm::gload16_nt(src + base + static_cast<size_t>(u) * kT * 16);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int u = 0; u < kN; ++u) {
-        ucm::gstore16_nt(dst + base + static_cast<size_t>(u) * kThreads * 16, v[u]);
+        ucm::gstore16_nt(dst + base + static_cast<size_t>(u) * kT * 16, v[u]);
     }
 }
 
 // One workgroup copies one whole slice (a 256 KiB K or V block = 2 trips of 128 KiB).  size is a multiple of
 // 16.  What is left after the 128 KiB trips goes in trips of 64, 32 and 16 KiB (the slices of 64-, 32- and
-// 16-token blocks), each with all its loads in flight at once, and a last partial one.
+// 16-token blocks), each with all its loads in flight at once, and a last partial one.  (kT threads: a trip is kT * 128 bytes.)
+template <int kT = kThreads>
 __device__ __forceinline__ void copy_slice(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t size)
 {
+    constexpr size_t kTrip = static_cast<size_t>(kT) * 16 * kUnroll;
     size_t o = 0;
     const size_t mine = threadIdx.x * 16u;
-    for (; o + kStep <= size; o += kStep) { copy_trip<kUnroll>(dst, src, o + mine); }
-    if (o + kStep / 2 <= size) { copy_trip<kUnroll / 2>(dst, src, o + mine); o += kStep / 2; }
-    if (o + kStep / 4 <= size) { copy_trip<kUnroll / 4>(dst, src, o + mine); o += kStep / 4; }
-    if (o + kStep / 8 <= size) { copy_trip<kUnroll / 8>(dst, src, o + mine); o += kStep / 8; }
+    for (; o + kTrip <= size; o += kTrip) { copy_trip<kUnroll, kT>(dst, src, o + mine); }
+    if (o + kTrip / 2 <= size) { copy_trip<kUnroll / 2, kT>(dst, src, o + mine); o += kTrip / 2; }
+    if (o + kTrip / 4 <= size) { copy_trip<kUnroll / 4, kT>(dst, src, o + mine); o += kTrip / 4; }
+    if (o + kTrip / 8 <= size) { copy_trip<kUnroll / 8, kT>(dst, src, o + mine); o += kTrip / 8; }
     if (o + mine < size) { ucm::gstore16_nt(dst + o + mine, ucm::gload16_nt(src + o + mine)); }
 }
 
@@ -114,8 +116,54 @@ __global__ __launch_bounds__(kThreads) void kv_gather_selected_kernel(
 
 // Loads planned on the device: slot j of request row `row` receives logical block load_sel[l][row][j] (or
 // nothing, -1) from a pool of stored blocks laid out [block][layer][K|V].
+//
+// A workgroup of kT threads follows one slot, or one piece of it (kT * 128 bytes, a trip), and nothing else: it ends with its
+// stores on their way, and one whose slot loads nothing ends after one read.  The shorter the slice, the fewer threads: what
+// limits short slices is how many of them a compute unit has under way, and what limits a plan that loads little is how
+// fast it gets through idle workgroups (1024 threads: two a unit; 256: eight).  us, 1024 threads for every 16th (or
+// every) slot of a row | a list per row as below, one slice after the other | this:
+//   64 requests x 50 slots, 4 KiB, all load          30.0 | 30.7 | 12.0       a tenth  22.4 | 20.5 | 8.4
+//   8 layers x 16 x 50, 32 KiB                       159  | 158  | 145                 26.2 | 33.0 | 18.7
+//   32 layers x 32 x 153, 32 KiB                     3840 | 4010 | 3810                406  | 403  | 397
+//   8 layers x 64 x 48, 32 KiB                       563  | 606  | 588                 85.1 | 66.6 | 62.7
+//   4 layers x 32 x 60, 64 KiB                       345  | 343  | 352                 41.5 | 55.0 | 39.5
+//   8 layers x 8 x 100, 128 KiB                      594  | 590  | 580                 63.7 | 84.2 | 61.1
+// (A loop over further pieces, for grids that stop short of a row, made an idle workgroup 1.8 times as long.)
+// grid: x = slot * pieces + piece, y = request of the call, z = layer*2 + K|V
+template <int kT>
+__global__ __launch_bounds__(kT) void kv_load_slot_kernel(
+    void* const* __restrict__ layers, size_t kv_stride, size_t block_bytes, unsigned num_blocks,
+    const uint8_t* __restrict__ pool, uint64_t pool_blocks, size_t pool_block_bytes, unsigned store_first_layer,
+    const int32_t* __restrict__ load_sel, unsigned n_slots, const int32_t* __restrict__ src_table, unsigned src_stride,
+    const int32_t* __restrict__ dst_table, unsigned dst_stride, int64_t dst_layer_stride,
+    const int32_t* __restrict__ load_count, const int32_t* __restrict__ rows, unsigned table_rows, unsigned pieces, StoredLayout lay)
+{
+    constexpr size_t kPiece = static_cast<size_t>(kT) * 16 * kUnroll;
+    const unsigned b = blockIdx.y, l = blockIdx.z >> 1, kv = blockIdx.z & 1;
+    unsigned row = b;
+    if (rows) {
+        const int32_t r = rows[b];
+        if (r < 0) { return; }
+        row = static_cast<unsigned>(r);
+    }
+    if (row >= table_rows) { return; }
+    const unsigned j = blockIdx.x / pieces;
+    if (load_count && static_cast<int>(j) >= load_count[static_cast<size_t>(l) * table_rows + row]) { return; }
+    const int32_t sel = load_sel[(static_cast<size_t>(l) * table_rows + row) * n_slots + j];
+    if (sel < 0 || static_cast<unsigned>(sel) >= src_stride) { return; }          // slot keeps what it holds
+    const int32_t src = src_table[static_cast<size_t>(row) * src_stride + sel];
+    const unsigned dst = static_cast<unsigned>(dst_table[l * dst_layer_stride + static_cast<int64_t>(row) * dst_stride + j]);
+    if (src < 0 || static_cast<uint64_t>(src) >= pool_blocks || dst >= num_blocks) { return; }   // not in the pool, or outside the cache
+    const size_t off = (blockIdx.x - j * pieces) * kPiece;
+    copy_slice<kT>(static_cast<uint8_t*>(layers[l]) + kv * kv_stride + static_cast<size_t>(dst) * block_bytes + off,
+                   pool + static_cast<size_t>(src) * pool_block_bytes + lay.slice(store_first_layer + l, kv, block_bytes) + off,
+                   min(kPiece, block_bytes - off));
+}
+
+// The same for slices of more than a 128 KiB trip in launches of many pieces, where a workgroup each costs more in idle ones
+// than it brings (8 layers x 16 requests x 153 slots of 256 KiB, one in fifty loads: 155 us that way, 87 this way).
 // A workgroup looks at all of its row's slots at once, keeps the ones that load something in a list in LDS, and takes its
-// share of their pieces: the row's workgroups deal the pieces (one 128 KiB trip each) out between them.  (Stepping from slot to
+// share of their pieces: the row's workgroups deal the pieces (one trip each) out between them.  (Stepping from slot to
 // slot costs a trip to memory for every slot that has nothing to load, with the copies standing still, and whole
 // slices of 256 KiB leave the chip half empty at the end: 2 layers x 16 requests with 779 blocks to load 181 us, 143 this
 // way; 8 layers x 16 requests, 1875 blocks, 359 and 353 us = 5.6 TB/s.  Pieces of 64 KiB: 148 and 360 us.)
@@ -429,17 +477,38 @@ extern "C" int ucm_kv_load_planned_tp(void* const* layers, int n_layers, size_t 
                            static_cast<unsigned>(dst_stride), dst_layer_stride, load_count, rows,
                            static_cast<unsigned>(table_rows), static_cast<unsigned>(batch), static_cast<unsigned>(n_layers), lay);
     } else {
-        // The entries to load are scattered over a row (or there are too many rows for the counted kernel's table): about
-        // 4096 workgroups over all rows, at least four a row, never more than a row has pieces.
+        // The entries to load are scattered over a row (or there are too many rows for the counted kernel's table).
         const int64_t table = static_cast<int64_t>(batch) * n_layers * 2;
-        const int64_t row_pieces = static_cast<int64_t>(n_slots) * static_cast<int64_t>((block_bytes + kLoadPiece - 1) / kLoadPiece);
-        const unsigned gx = static_cast<unsigned>(std::min(row_pieces, std::max<int64_t>(4, 4096 / table)));
-        hipLaunchKernelGGL(kv_load_planned_kernel, dim3(gx, batch, n_layers * 2), dim3(kThreads), 0,
-                           ucm::as_stream(stream), layers, kv_stride, block_bytes, static_cast<unsigned>(num_blocks),
-                           static_cast<const uint8_t*>(pool), static_cast<uint64_t>(pool_blocks), pool_block_bytes,
-                           static_cast<unsigned>(store_first_layer), load_sel, static_cast<unsigned>(n_slots), src_table,
-                           static_cast<unsigned>(src_stride), dst_table, static_cast<unsigned>(dst_stride), dst_layer_stride,
-                           load_count, rows, static_cast<unsigned>(table_rows), lay);
+        const auto pieces = [&](size_t piece) { return static_cast<int64_t>((block_bytes + piece - 1) / piece); };
+        auto follow_slots = [&](auto kernel, int threads) {
+            const unsigned per_slot = static_cast<unsigned>(pieces(static_cast<size_t>(threads) * 16 * kUnroll));
+            hipLaunchKernelGGL(kernel, dim3(n_slots * per_slot, batch, n_layers * 2), dim3(threads), 0, ucm::as_stream(stream), layers,
+                               kv_stride, block_bytes, static_cast<unsigned>(num_blocks), static_cast<const uint8_t*>(pool),
+                               static_cast<uint64_t>(pool_blocks), pool_block_bytes, static_cast<unsigned>(store_first_layer),
+                               load_sel, static_cast<unsigned>(n_slots), src_table, static_cast<unsigned>(src_stride), dst_table,
+                               static_cast<unsigned>(dst_stride), dst_layer_stride, load_count, rows,
+                               static_cast<unsigned>(table_rows), per_slot, lay);
+        };
+        // (64 KiB slices in small launches: 4 requests x 300 slots 51 us with 1024 threads, 55 with 512; in large ones idle
+        // workgroups count: 8 layers x 8 requests x 100 slots of 128 KiB, one in fifty loads, 29 us with 512 and 32 with 1024.
+        // A row of more than a million slots does not fit the grid; the list takes any number.)
+        const bool fits = n_slots <= 1 << 20;
+        if (fits && block_bytes <= kStep / 4) {
+            follow_slots(kv_load_slot_kernel<256>, 256);
+        } else if (n_slots * pieces(kLoadPiece) * table <= 4096) {
+            follow_slots(kv_load_slot_kernel<kThreads>, kThreads);
+        } else if (fits && block_bytes <= kStep) {
+            follow_slots(kv_load_slot_kernel<512>, 512);
+        } else {
+            // about 4096 workgroups over all rows, at least four a row, never more than a row has pieces
+            const unsigned gx = static_cast<unsigned>(std::min(n_slots * pieces(kLoadPiece), std::max<int64_t>(4, 4096 / table)));
+            hipLaunchKernelGGL(kv_load_planned_kernel, dim3(gx, batch, n_layers * 2), dim3(kThreads), 0,
+                               ucm::as_stream(stream), layers, kv_stride, block_bytes, static_cast<unsigned>(num_blocks),
+                               static_cast<const uint8_t*>(pool), static_cast<uint64_t>(pool_blocks), pool_block_bytes,
+                               static_cast<unsigned>(store_first_layer), load_sel, static_cast<unsigned>(n_slots), src_table,
+                               static_cast<unsigned>(src_stride), dst_table, static_cast<unsigned>(dst_stride), dst_layer_stride,
+                               load_count, rows, static_cast<unsigned>(table_rows), lay);
+        }
     }
     UCM_LAUNCH_CHECK("ucm_kv_load_planned");
 }
