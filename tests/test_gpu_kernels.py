@@ -660,6 +660,7 @@ def test_planned_loads_of_scattered_slots(ucm, dev, n_slots, bb):
     (2, 4, 9, 32768 + 16), (1, 3, 5, 32768), (1, 3, 7, 48), (2, 3, 5, 4 * 131072 + 4096),      # small launches, each size of workgroup
     (8, 9, 60, 65536), (8, 9, 60, 65536 + 16), (8, 9, 60, 131072), (8, 9, 60, 49152),          # large ones: a piece, a piece and a remainder, two
     (8, 9, 40, 131072 + 16), (4, 8, 40, 262144),                                              # the list: pieces of a longer slice
+    (40, 41, 2, 48), (12, 40, 2, 131072 + 16),                                                # counts over several waves of the running total
     (65, 64, 3, 48), (65, 64, 1, 32768 + 16)])                                                # more rows than the counted kernel's table
 def test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_slots, bb, counted):
     """The rule that picks how a plan's loads are dealt out, on both sides of its bounds, with and without counts; with
