@@ -116,11 +116,14 @@ __device__ __forceinline__ void swap_rows(unsigned& a, unsigned& b)
 // One pass of a wave: kSteps 16-byte loads per lane over 64/kLanes vectors, kLanes adjacent lanes per vector and step.
 // Register g*kGroup + n of lane L receives step g*kGroup + (L's top bits) of vector n*(vectors/kGroup) + (L / kLanes);
 // own_vectors then leaves step i of vector L/kLanes in register i.  A block past `last` is read as block `last`.
+// The non-temporal hint only where an instruction takes whole lines: six steps of bf16 (head_dim 96) go two by two, 64 bytes
+// of 192, and with the hint each group of steps fetched its lines anew: 32 layers x 4350 blocks x 8 heads 63.1 us, 47.5 with plain loads.
 template <int kSteps, int kGroup, int kLanes, typename T>
 __device__ __forceinline__ void load_vectors(u32x4 (&kv)[kSteps], const T* __restrict__ rbase, int base, int last, int vecs, int lane)
 {
     constexpr int kPer = 64 / kLanes / kGroup;           // vectors per load instruction
     constexpr int kElems = 16 / kLanes;                  // elements of a 16-byte piece
+    constexpr bool kWholeLines = kGroup == kSteps || kGroup * 16 * sizeof(T) % 128 == 0;
     const int step = lane / (64 / kGroup), mine = (lane / kLanes) & (kPer - 1);
     const int lg = __builtin_ctz(vecs);                  // vecs is a power of two (host checked)
 #pragma unroll
@@ -129,7 +132,9 @@ __device__ __forceinline__ void load_vectors(u32x4 (&kv)[kSteps], const T* __res
         const int vec = (min(base + (v >> lg), last) << lg) + (v & (vecs - 1));
         const T* p = rbase + static_cast<size_t>(static_cast<unsigned>(vec)) * (kSteps * 16) + step * 16 + (lane & (kLanes - 1)) * kElems;
 #pragma unroll
-        for (int g = 0; g < kSteps / kGroup; ++g) { kv[g * kGroup + n] = ucm::gload16_nt(p + g * kGroup * 16); }
+        for (int g = 0; g < kSteps / kGroup; ++g) {
+            kv[g * kGroup + n] = kWholeLines ? ucm::gload16_nt(p + g * kGroup * 16) : ucm::gload16(p + g * kGroup * 16);
+        }
     }
 }
 
