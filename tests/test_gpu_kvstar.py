@@ -174,6 +174,27 @@ def test_kvstar_votes_match_oracle(ucm, dev, x, hq, hkv, d, M):
             assert abs(got[off[t] : off[t] + n].sum() - x * hq) < 1e-3 * x * hq
 
 
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 80, 96, 112, 128])
+@pytest.mark.parametrize("M", [2, 4, 32])
+@pytest.mark.parametrize("hq", [8, 24])                       # up to 32 query rows per kv head, and more
+def test_kvstar_votes_of_every_vector_length(ucm, dev, hq, M, d):
+    """Vectors that fill the kernel's steps and vectors that end one, two or three steps earlier, read plainly (M = 2, d = 16)
+    and in whole lines, on both paths."""
+    from ucm_amd import ops
+
+    x, hkv, lens = 4, 2, [19, 0, 70]
+    rows = int(np.sum(lens))
+    scale = np.float32(0.25)
+    repre = f16_bits(synth.normal_f32(1300 + d, (rows, M, hkv, d)) * scale)
+    qs = [f16_bits(synth.normal_f32(1301 + t, (x, hq, d)) * scale) for t in range(len(lens))]
+    for tiles_per_wave in (0, -1):
+        got, off = run_votes(ops, dev, qs, repre, lens, x, hq, tiles_per_wave=tiles_per_wave)
+        for t, n in enumerate(lens):
+            if n:
+                want = O.kvstar_retrieve(qs[t], repre[off[t] : off[t] + n], topk=1)[1]
+                assert np.allclose(got[off[t] : off[t] + n], want, rtol=VOTE_RTOL, atol=VOTE_ATOL), (tiles_per_wave, t)
+
+
 def test_kvstar_many_short_tasks_take_the_in_lds_path(ucm, dev):
     """Enough (task, kv head) pairs that the automatic choice is one workgroup per pair with the task's
     per-block sums in LDS; ragged lengths including empty tasks."""

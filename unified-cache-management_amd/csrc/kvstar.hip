@@ -509,6 +509,11 @@ __device__ __forceinline__ unsigned task_blocks(const int32_t* __restrict__ seg_
     return ok ? static_cast<unsigned>(n) : 0u;
 }
 
+// How the score kernel reads keys: plainly; whole lines, with the non-temporal hint; the same for vectors that end before
+// the last of kSteps steps, which then read kNoKeys instead of a piece.  Why: see load_keys.
+enum class KeyReads { kPlain, kLines, kLinesShort };
+__device__ const unsigned short kNoKeys[8] __attribute__((aligned(16))) = {0, 0, 0, 0, 0, 0, 0, 0};
+
 // grid: x = chunk of sub-blocks, y = kv head, z = task.  The table is head-major and piece-interleaved
 // inside a block (see above), so what one workgroup streams is one contiguous run read in whole lines
 // (in the reference's [row][sub-block][kv head][d] order each vector of a head sits kv_heads*d*2 bytes
@@ -529,7 +534,7 @@ __device__ __forceinline__ unsigned task_blocks(const int32_t* __restrict__ seg_
 // itself reduces every row's maximum and denominator when it is through, and only this head's share of
 // the votes ([task][kv head][max_blocks], in ws_part) goes to memory: 1/32 of the other path's stores,
 // whose number per compute unit - not their bytes - is what that path pays for.
-template <int kM, int kSteps, bool kTwoRowTiles, bool kLds>
+template <int kM, int kSteps, bool kTwoRowTiles, bool kLds, KeyReads kReads>
 __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
     const unsigned short* __restrict__ q, const int64_t* __restrict__ q_off, unsigned n_tokens, unsigned q_heads,
     unsigned d_orig, const int32_t* __restrict__ pruned, const int32_t* __restrict__ pruned_sel,
@@ -551,7 +556,7 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
     constexpr unsigned kEntrySub = kM < static_cast<int>(kSpan) ? kM : kSpan;   // kLds: sub-blocks per plane entry
     constexpr unsigned kEntryTiles = kEntrySub > kTileSub ? kEntrySub / kTileSub : 1;
     constexpr unsigned kEntriesPerBlock = kM / kEntrySub;
-    constexpr bool kWholeLines = kM >= 4;                // see load_keys
+    static_assert(kReads == KeyReads::kPlain || kM >= 4, "an instruction reads whole lines");
 
     extern __shared__ __attribute__((aligned(16))) unsigned short q_s[];   // [row_pad][kQStride]
     // kLds: [entry][row_pad] floats from byte plane_offset on (0 with one row tile: the queries then live in
@@ -583,14 +588,18 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
 
     // A span's keys: for each of its tiles, kSteps 16-byte loads per lane, piece 2*ks + half of the lane's
     // sub-block; the lanes of one instruction cover M*16 contiguous bytes per block and lane half.
-    // From four sub-blocks on, the two halves' pieces of a block are whole 128-byte lines in one instruction, which are
-    // then read with the non-temporal hint; with fewer an instruction takes 32 or 64 bytes of a line and the hint would
+    // From four sub-blocks on, the two halves' pieces of a block are whole 128-byte lines in one instruction, and
+    // they are read with the non-temporal hint; with fewer an instruction takes 32 or 64 bytes of a line and the hint would
     // lose the line before the instructions that take the rest.  512 tasks of the ragged batch, without and with the
     // hint: 64 x 32 channels 1006 and 896 us (6.4 TB/s), 16 x 128 972 and 871, 4 x 128 268 and 241, 4 x 32 136 and 129;
     // 2 x 128 172 and 198, 1 x 128 139 and 178 us.
-    // Everything is unconditional - MFMA steps past d_pad reload piece 0 and are multiplied with a zero
-    // query fragment, lanes and tiles past the workgroup's end reload its last vector and are masked or
-    // never used.
+    // Everything is unconditional - lanes and tiles past the workgroup's end reload its last vector and are masked or
+    // never used, MFMA steps past d_pad are multiplied with a zero query fragment.  What these steps load has to be near:
+    // piece 0 once more where lines stay in the L1, one piece of zeros where they do not (16 layers x 16 requests, 16 and 8
+    // sub-blocks x 80 channels: 345 and 194 us reading plainly, 357 and 201 with the hint and piece 0, 309 and 175 with the zeros;
+    // an instance of its own, because choosing the address costs vectors without a missing step 1 to 3 %).  With one
+    // step of four missing the hint wins all the same (16 x 48 channels 222 and 212 us); with one of two it does not, and
+    // these are read plainly (64 x 16 channels 361 us, 372 with the hint).
     //
     // Three key buffers rotate, so two spans are in flight while one is worked on.  Every group of loads is
     // followed by a compiler barrier (an empty asm that may touch memory): left to itself the compiler sinks
@@ -606,7 +615,10 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
 #pragma unroll
             for (int ks = 0; ks < kSteps; ++ks) {
                 const unsigned short* piece = krow + (static_cast<unsigned>(ks) < ksteps ? ks : 0) * (16 * kM);
-                kf[t * kSteps + ks] = kWholeLines ? ucm::gload16_nt(piece) : ucm::gload16(piece);
+                if constexpr (kReads == KeyReads::kLinesShort) {
+                    piece = ks <= kSteps / 2 || static_cast<unsigned>(ks) < ksteps ? krow + ks * (16 * kM) : kNoKeys;
+                }
+                kf[t * kSteps + ks] = kReads == KeyReads::kPlain ? ucm::gload16(piece) : ucm::gload16_nt(piece);
             }
         }
         asm volatile("" ::: "memory");
@@ -1316,28 +1328,34 @@ int kvstar_votes(const void* q_f16, int64_t q_elems, const int64_t* q_off, int n
         static_cast<unsigned>(kv_heads),                                                                                      \
         static_cast<unsigned>(d_pruned), static_cast<unsigned>(d_pad), repre_head_stride, repre_row_stride, ws_max, ws_part, \
         static_cast<unsigned>(max_blocks), max_tiles, spans_per_wave, row_pad, plane_offset, q_full_ok, tb
-#define UCM_KVSTAR_LAUNCH4(M, STEPS, TWO, LDS)                                                                        \
+#define UCM_KVSTAR_LAUNCH4(M, STEPS, TWO, LDS, READS)                                                                 \
     do {                                                                                                             \
         if (lds_bytes > 48u * 1024u) {                                                                               \
             const hipError_t ea = hipFuncSetAttribute(                                                               \
-                reinterpret_cast<const void*>(kvstar_score_kernel<M, STEPS, TWO, LDS>),                              \
+                reinterpret_cast<const void*>(kvstar_score_kernel<M, STEPS, TWO, LDS, READS>),                       \
                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));                           \
             if (ea != hipSuccess) { return ucm::check_hip(ea, "ucm_kvstar_votes (LDS size)"); }                      \
         }                                                                                                            \
-        hipLaunchKernelGGL((kvstar_score_kernel<M, STEPS, TWO, LDS>), UCM_KVSTAR_ARGS);                              \
+        hipLaunchKernelGGL((kvstar_score_kernel<M, STEPS, TWO, LDS, READS>), UCM_KVSTAR_ARGS);                       \
     } while (0)
-#define UCM_KVSTAR_LAUNCH3(M, STEPS, TWO)                                                                             \
+#define UCM_KVSTAR_LAUNCH3(M, STEPS, TWO, READS)                                                                      \
     do {                                                                                                             \
-        if (use_lds) { UCM_KVSTAR_LAUNCH4(M, STEPS, TWO, true); } else { UCM_KVSTAR_LAUNCH4(M, STEPS, TWO, false); } \
+        if (use_lds) { UCM_KVSTAR_LAUNCH4(M, STEPS, TWO, true, READS); }                                             \
+        else { UCM_KVSTAR_LAUNCH4(M, STEPS, TWO, false, READS); }                                                    \
     } while (0)
-#define UCM_KVSTAR_LAUNCH2(M, STEPS)                                                                                  \
+#define UCM_KVSTAR_LAUNCH2(M, STEPS, READS)                                                                           \
     do {                                                                                                             \
-        if (R > 32) { UCM_KVSTAR_LAUNCH3(M, STEPS, true); } else { UCM_KVSTAR_LAUNCH3(M, STEPS, false); }            \
+        if (R > 32) { UCM_KVSTAR_LAUNCH3(M, STEPS, true, READS); } else { UCM_KVSTAR_LAUNCH3(M, STEPS, false, READS); } \
     } while (0)
 #define UCM_KVSTAR_LAUNCH(M)                                                                                          \
     do {                                                                                                             \
-        if (steps == 2) { UCM_KVSTAR_LAUNCH2(M, 2); } else if (steps == 4) { UCM_KVSTAR_LAUNCH2(M, 4); }             \
-        else { UCM_KVSTAR_LAUNCH2(M, 8); }                                                                           \
+        constexpr KeyReads lines = M >= 4 ? KeyReads::kLines : KeyReads::kPlain;                                     \
+        constexpr KeyReads lines_short = M >= 4 ? KeyReads::kLinesShort : KeyReads::kPlain;                          \
+        if (d_pad == 16) { UCM_KVSTAR_LAUNCH2(M, 2, KeyReads::kPlain); }                                             \
+        else if (steps == 2) { UCM_KVSTAR_LAUNCH2(M, 2, lines); }                                                    \
+        else if (steps == 4) { UCM_KVSTAR_LAUNCH2(M, 4, lines); }                                                    \
+        else if (d_pad < 128) { UCM_KVSTAR_LAUNCH2(M, 8, lines_short); }                                             \
+        else { UCM_KVSTAR_LAUNCH2(M, 8, lines); }                                                                    \
     } while (0)
     switch (sub_blocks) {
     case 1: UCM_KVSTAR_LAUNCH(1); break;
