@@ -131,7 +131,9 @@ int ucm_block_mean(const void* const* k_layers, int n_layers, int num_blocks,
  *              variant, the mean over all q heads of TopkCal.cal_topk
  *              (ucm/sparse/gsa/gsa.py:386-412, to the rounding of its own
  *              summation order; the ranking is the same for any positive scale).
- *   tile_blocks  blocks scored per workgroup; 0 sizes a workgroup's share to 128 KiB
+ *   tile_blocks  blocks scored per workgroup, 1..4096, where more than 2048 count as
+ *              2048 (what a workgroup's scores have room for; the scores are the same
+ *              for every value); 0 sizes a workgroup's share to 128 KiB
  *              of representatives (a value for benchmarks and tests, not part of
  *              the reference interface).
  * head_dim must be 32, 64, 96, 128, 192 or 256, kv_heads*num_repre one of 1, 2,

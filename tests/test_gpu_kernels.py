@@ -336,6 +336,24 @@ def test_q_rows_indirection_and_tile_sizes(ucm, dev):
 
 
 @pytest.mark.parametrize("repre_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tile", [2047, 2048, 2049, 4096])
+def test_tiles_around_what_a_workgroup_holds(ucm, dev, tile, repre_dtype):
+    """Requests of one and of several tiles at the largest tile a workgroup's scores have room for, and above it."""
+    from ucm_amd import ops
+
+    hkv, g, d, lens = 1, 2, 32, [2047, 2048, 2049, 4096, 5000, 1]
+    off, rows = np.concatenate([[0], np.cumsum(lens)[:-1]]), int(np.sum(lens))
+    q = synth.normal_bf16_as_f32(43, (len(lens), hkv * g, d))
+    repre = as_bf16_values(synth.normal_f32(44, (rows, hkv * d)))
+    scores = torch.zeros((1, rows), device=dev)
+    ops.score_blocks(torch.from_numpy(q).to(dev)[None], torch.from_numpy(repre).to(dev).to(repre_dtype)[None], i32(off, dev), i32(lens, dev),
+                     max(lens), hkv, scores, tile_blocks=tile)
+    for r, n in enumerate(lens):
+        want = O.kq_scores(O.q_head_mean(q[r], hkv), repre[off[r] : off[r] + n].reshape(n, hkv, 1, d))
+        assert np.array_equal(bits(scores[0, off[r] : off[r] + n].cpu().numpy()), bits(want)), r
+
+
+@pytest.mark.parametrize("repre_dtype", [torch.float32, torch.bfloat16])
 def test_query_rows_outside_the_layer_are_skipped(ucm, dev, repre_dtype):
     """q_rows comes from device memory: a request whose query row is negative or past the layer's block of
     queries is not followed - its scores stay as they were - and the other requests are scored as usual."""
