@@ -98,6 +98,28 @@ def test_ops_need_device_tensors(ucm):
         ops.copy_batch(torch.zeros(2, dtype=torch.int64), torch.zeros(2, dtype=torch.int64), 16)
 
 
+@pytest.mark.parametrize("name,value", [("scale", 0.25), ("scale", 3), ("scale", 1e39), ("scale", float("inf")), ("max_seg_len", 2**32 + 5),
+                                        ("start_w", -1), ("end_w", 2**31), ("total_blocks", 2**64 + 7), ("q_layer_stride", -(2**63)),
+                                        ("kv_heads", True), ("block_size", 2.0), ("n_req", "3")])
+def test_packed_arguments_are_the_structures(ucm, name, value):
+    """The packed form of ucm_score_select's arguments holds, cuts and refuses what the structure's own fields do."""
+    from ucm_amd import _lib
+
+    names = [n for n, _ in _lib.ScoreSelectArgs._fields_[1:]]
+    values = {n: 7 + 3 * i for i, n in enumerate(names)}
+    values["scale"] = 0.5
+    values[name] = value
+    args = _lib.ScoreSelectArgs()
+    try:
+        for n in names:
+            setattr(args, n, values[n])
+    except TypeError:
+        with pytest.raises(TypeError):
+            _lib.pack_score_select(*[values[n] for n in names])
+    else:
+        assert _lib.pack_score_select(*[values[n] for n in names]) == bytes(args)
+
+
 def test_missing_library_is_loud(ucm, monkeypatch):
     from ucm_amd import _lib
 

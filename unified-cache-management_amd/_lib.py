@@ -106,8 +106,16 @@ if _SCORE_SELECT.size != C.sizeof(ScoreSelectArgs):
 
 
 def pack_score_select(*fields) -> bytes:
-    """ucm_score_select_args_t from the values of the fields after struct_size, in order (null pointers are 0)."""
-    return _SCORE_SELECT.pack(_SCORE_SELECT.size, *fields)
+    """ucm_score_select_args_t from the values of the fields after struct_size, in order (null pointers are 0).  A value that
+    its C type does not hold goes through the structure, which cuts integers and
+    refuses, with a TypeError, what is not one."""
+    try:
+        return _SCORE_SELECT.pack(_SCORE_SELECT.size, *fields)
+    except (struct.error, OverflowError):
+        args = ScoreSelectArgs()
+        for (name, _), value in zip(ScoreSelectArgs._fields_[1:], fields):
+            setattr(args, name, value)
+        return bytes(args)
 
 
 class UcmHipError(RuntimeError):

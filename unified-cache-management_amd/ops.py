@@ -225,7 +225,7 @@ def score_select(q: torch.Tensor, repre: torch.Tensor, seg_off: torch.Tensor, se
         _dev(repre, repre.dtype, "repre"), _lib.DTYPE_BF16 if repre.dtype == torch.bfloat16 else _lib.DTYPE_F32, num_repre,
         repre.stride(0), rs[1], _dev(seg_off, i32, "seg_off"), _dev(seg_len, i32, "seg_len"),
         _dev(topk_len, i32, "topk_len"), n_req, max_seg_len, first_layer, n_layers, kv_heads, head_dim,
-        _dev(scores, torch.float32, "scores"), scores.stride(0), scale, int(tile_blocks), start_w, end_w,
+        _dev(scores, torch.float32, "scores"), scores.stride(0), float(scale), int(tile_blocks), start_w, end_w,
         _dev(idx_out, i32, "idx_out"), _dev(count_out, i32, "count_out"), idx_shape[2],
         0 if block_tables is None else block_tables.shape[1], _opt(block_tables, i32, "block_tables") or 0,
         _opt(phys_out, i32, "phys_out") or 0, _opt(seq_lens, i32, "seq_lens") or 0,
