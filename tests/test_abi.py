@@ -120,6 +120,21 @@ def test_packed_arguments_are_the_structures(ucm, name, value):
         assert _lib.pack_score_select(*[values[n] for n in names]) == bytes(args)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "int8", "float64"])
+def test_score_calls_refuse_tables_of_other_types(ucm, dtype):
+    """A table of 16- or 8-bit elements taken for fp32 would be read past its end."""
+    import torch
+    from ucm_amd import ops
+
+    q, repre, scores = torch.zeros(1, 1, 4, 32), torch.zeros(1, 3, 64, dtype=getattr(torch, dtype)), torch.zeros(1, 3)
+    one = torch.zeros(1, dtype=torch.int32)
+    idx, cnt = torch.zeros(1, 1, 3, dtype=torch.int32), torch.zeros(1, 1, dtype=torch.int32)
+    with pytest.raises(ValueError, match="repre must be"):
+        ops.score_select(q, repre, one, one, one, 3, 2, scores, idx, cnt, cnt.clone())
+    with pytest.raises(ValueError, match="repre must be"):
+        ops.score_blocks(q, repre, one, one, 3, 2, scores)
+
+
 def test_missing_library_is_loud(ucm, monkeypatch):
     from ucm_amd import _lib
 

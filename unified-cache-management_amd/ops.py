@@ -207,6 +207,8 @@ def score_select(q: torch.Tensor, repre: torch.Tensor, seg_off: torch.Tensor, se
     head_dim, q_heads = qs[3], qs[2]
     if rs[2] != kv_heads * num_repre * head_dim:
         raise ValueError("repre row does not match kv_heads*num_repre*head_dim")
+    if repre.dtype != torch.bfloat16 and repre.dtype != torch.float32:
+        raise ValueError("repre must be float32 or bfloat16")
     n_req = seg_off.numel()
     n_layers = qs[0] if n_layers is None else n_layers
     if first_layer < 0 or first_layer + n_layers > min(rs[0], ss[0], idx_shape[0]) or n_layers > qs[0]:
