@@ -104,6 +104,32 @@ def test_hash_encode_short_lists_share_blocks(ucm, dev, hkv, bs, n):
     assert (tcodes[0].cpu().numpy()[rest] == 0xEE).all() and (colsum[0].cpu().numpy()[rest] == 77).all()
 
 
+def test_hash_encode_lists_of_more_than_31_bits_over_all_layers(ucm, dev):
+    """Items are numbered over all layers in 31 bits: a longer list goes out a few layers at a time.  Almost all entries
+    are out of range (and skipped); the first, the middle and the last one encode a block in every layer."""
+    from ucm_amd import ops
+
+    L, n, hkv, bs, nb = 33, 1 << 26, 1, 32, 3
+    caches = torch.randn((L, nb, bs, hkv, 128), device=dev, generator=torch.Generator(device=dev).manual_seed(6)).to(torch.bfloat16)
+    layers = ops.LayerPointers([caches[l] for l in range(L)])
+    w = torch.randn((128, 128), device=dev, generator=torch.Generator(device=dev).manual_seed(7)).to(torch.bfloat16)
+    ids = torch.full((n,), -1, dtype=torch.int32, device=dev)
+    slots = ids.clone()
+    at = torch.tensor([0, n // 2, n - 1], device=dev)
+    short_ids, short_slots = torch.tensor([2, 0, 1], dtype=torch.int32, device=dev), torch.tensor([0, 1, 2], dtype=torch.int32, device=dev)
+    ids[at], slots[at] = short_ids, short_slots
+    out = []
+    for i, s, k in ((ids, slots, n), (short_ids, short_slots, 3)):
+        colsum = torch.zeros((L, 3, hkv, 128), dtype=torch.int16, device=dev)
+        codes = torch.zeros((L, 3, hkv, 16), dtype=torch.uint8, device=dev)
+        tokens = torch.zeros((L, 3, bs, hkv, 16), dtype=torch.uint8, device=dev)
+        ops.hash_encode_blocks(layers, i, s, k, w, bs, hkv, nb, colsum, codes, token_codes=tokens)
+        out.append((colsum, codes, tokens))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    assert out[0][1].any()
+
+
 @pytest.mark.parametrize("hkv,bs", [(8, 128), (2, 48), (1, 160), (4, 8)])
 def test_hash_encode_persistent_waves_and_queue_overflow(ucm, dev, hkv, bs):
     """One workgroup per layer walks the whole list (every wave takes several blocks, the
