@@ -306,6 +306,7 @@ struct __attribute__((aligned(128))) EncodeLds {
 static_assert(sizeof(EncodeLds) <= 160 * 1024, "LDS of a compute unit");
 
 // sixteen bytes per lane from base + offset (per lane) to LDS byte address `lds` + 16 * lane
+// (m0 is set and used inside the statement; nothing else in these kernels touches it, the compiler's own code included)
 __device__ __forceinline__ void load_to_lds(unsigned lds, const unsigned char* base, unsigned offset)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base) : "memory", "m0");

@@ -7,7 +7,8 @@
 // shapes tried on MI355X (8 KiB .. 256 KiB per workgroup, 64 .. 1024 threads,
 // 1 .. 16 loads in flight per thread, persistent grids, with and without the
 // non-temporal hint) this one was the fastest; all of them sit between 5.2 and
-// 6.0 TB/s for a 1:1 read/write mix.
+// 6.0 TB/s for a 1:1 read/write mix.  (Planned loads, most of whose workgroups may
+// have nothing to do, take smaller ones for short slices: kv_load_slot_kernel.)
 #include "common.h"
 
 namespace {

@@ -591,7 +591,7 @@ __global__ __launch_bounds__(kThreads, 2) void kvstar_score_kernel(
     // From four sub-blocks on, the two halves' pieces of a block are whole 128-byte lines in one instruction, and
     // they are read with the non-temporal hint; with fewer an instruction takes 32 or 64 bytes of a line and the hint would
     // lose the line before the instructions that take the rest.  512 tasks of the ragged batch, without and with the
-    // hint: 64 x 32 channels 1006 and 896 us (6.4 TB/s), 16 x 128 972 and 871, 4 x 128 268 and 241, 4 x 32 136 and 129;
+    // hint: 64 x 32 channels 1006 and 893-933 us by process (6.1-6.4 TB/s), 16 x 128 972 and 871, 4 x 128 268 and 241, 4 x 32 136 and 129;
     // 2 x 128 172 and 198, 1 x 128 139 and 178 us.
     // Everything is unconditional - lanes and tiles past the workgroup's end reload its last vector and are masked or
     // never used, MFMA steps past d_pad are multiplied with a zero query fragment.  What these steps load has to be near:

@@ -9,17 +9,26 @@
 //   * fold 16->8->4 (x[j] + x[j+8], then x[j] + x[j+4]), then (x0+x2)+(x1+x3);
 //   * kv heads added in order starting from 0.0f.
 // Mapping onto a 64-wide wavefront: four adjacent threads (a DPP quad) own one
-// (block, head) vector; thread m of the quad holds AVX lanes 4m..4m+3 and reads
-// one float4 per 16-dim step, so a wave streams 16 vectors = 8 KiB of
-// contiguous representatives per pass with 16-byte loads, the two folds that
-// cross threads are quad_perm DPP moves, and the last fold is in-register.
-// The request's group-mean query is staged once per workgroup in LDS and then
-// kept in registers (a thread's head never changes because kv_heads divides 16).
+// (block, head) vector; thread m of the quad holds AVX lanes 4m..4m+3.  A wave
+// takes 16 vectors = 8 KiB of contiguous representatives per pass; its loads take
+// whole lines, several steps of a vector per instruction, and the lanes then
+// exchange what they hold of each other's vectors (load_vectors, own_vectors).
+// The two folds that cross threads are quad_perm DPP moves, the last fold is
+// in-register.  The request's group-mean query is staged once per workgroup in
+// LDS; this kernel then keeps it in registers (a thread's head never changes
+// because kv_heads divides 16), the bf16 one a quarter of it.
 //
 // The table is read in whole 128-byte lines with the non-temporal hint: a read-only loop over 1 GiB reaches 7.0 TB/s with
 // the hint and 6.2 TB/s without it.  80 layers x 8 requests x 6399 blocks (bf16 table, 1.06 GB, with the selection): 177 us
 // = 6.0 TB/s, and 161 us = 6.6 TB/s for the scores alone; 192-208 us with plain loads of 32 bytes per vector and
 // instruction (which the hint makes worse: a line then does not stay in the L1 for the other pieces).
+// What the hint costs and brings depends on what the 256 MiB Infinity Cache holds, since such reads leave nothing in it and
+// throw nothing out.  16, 32 and 64 layers of 16 requests with 5425 blocks, bf16, with the hint | the same loads without:
+//   tables read for the first time in a while        178 MB 42.3 | 45.0 us   355 MB 70.2 | 75.7   711 MB 128 | 140
+//   after another kernel has written 600 MB          178 MB 48.1 | 76.4 us   355 MB 81.6 | 124    711 MB 148 | 197
+//   the same table again, nothing in between         178 MB 40.5 | 38.9 us   355 MB 68.4 | 74.4   711 MB 126 | 140
+// A model runs between two retrievals, which is the first and second line; a loop over a table of 150 to 270 MB and nothing else
+// (or only non-temporal copies) is up to 8 us slower than plain loads.
 #include <algorithm>
 #include <cfloat>
 
@@ -95,7 +104,7 @@ __device__ __forceinline__ f32x4 group_mean4_any(const QT* src, int head_stride,
     return acc * inv;
 }
 
-// The 128-byte lines of a vector are loaded whole: an instruction reads `kGroup` steps of 16 dims of a vector with
+// The 128-byte lines of a vector are loaded whole (but for head_dim 96 in bf16): an instruction reads `kGroup` steps of 16 dims of a vector with
 // neighbouring lanes, and what the lanes then hold of each other's vectors is exchanged in registers.  (A lane that loads
 // its own vector's pieces step by step has every instruction touch a piece of each of the wave's vectors, and
 // the L1 looks up one line per lane pair instead of one per eight lanes.)  swap_halves / swap_rows exchange bit 5 / bit 4
@@ -117,7 +126,7 @@ __device__ __forceinline__ void swap_rows(unsigned& a, unsigned& b)
 // Register g*kGroup + n of lane L receives step g*kGroup + (L's top bits) of vector n*(vectors/kGroup) + (L / kLanes);
 // own_vectors then leaves step i of vector L/kLanes in register i.  A block past `last` is read as block `last`.
 // The non-temporal hint only where an instruction takes whole lines: six steps of bf16 (head_dim 96) go two by two, 64 bytes
-// of 192, and with the hint each group of steps fetched its lines anew: 32 layers x 4350 blocks x 8 heads 63.1 us, 47.5 with plain loads.
+// of 192, and with the hint each group of steps fetched its lines anew: 32 layers x 5425 blocks x 8 heads 63.1 us, 47.5 with plain loads.
 template <int kSteps, int kGroup, int kLanes, typename T>
 __device__ __forceinline__ void load_vectors(u32x4 (&kv)[kSteps], const T* __restrict__ rbase, int base, int last, int vecs, int lane)
 {
@@ -442,12 +451,13 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
 // The live reference path stores block means rounded to the model dtype
 // (ucm/sparse/gsa/gsa.py:640-652); keeping them as bf16 halves the bytes this
 // kernel streams and widens to the same fp32 values.  Two adjacent threads own
-// one (block, head) vector: thread p holds AVX lanes 8p..8p+7 and reads eight
-// bf16 (16 bytes) per 16-dim step, a wave covers 32 vectors = 8 KiB per pass;
-// the j/j+8 fold crosses the pair (one DPP), the j/j+4 and final folds are
-// in-register.  Same arithmetic, same order, same bits as the fp32-table kernel.
-// `q` is the thread's part of the staged query (16 values per step: eight of them its own); the lower four of a step come
-// in registers, the upper four are read from LDS here, one group of steps at a time.
+// one (block, head) vector: thread p holds AVX lanes 8p..8p+7, eight bf16 (16
+// bytes) of every 16-dim step once the exchange is done; a wave covers 32 vectors
+// = 8 KiB per pass; the j/j+8 fold crosses the pair (one DPP), the j/j+4 and final
+// folds are in-register.  Same arithmetic, same order, same bits as the fp32-table kernel.
+// `q` is the thread's part of the staged query (16 values per step: eight of them its own).  The lower four of the first
+// kKept steps come in registers; the others, and the upper four of every step, are read from LDS here, one group of steps at
+// a time.
 template <int kSteps, int kGroup, int kKept>
 __device__ __forceinline__ float pair_dot(const f32x4 (&qlo)[kKept], const float* q, u32x4 (&kv)[kSteps])
 {
