@@ -207,7 +207,8 @@ def score_select(q: torch.Tensor, repre: torch.Tensor, seg_off: torch.Tensor, se
     head_dim, q_heads = qs[3], qs[2]
     if rs[2] != kv_heads * num_repre * head_dim:
         raise ValueError("repre row does not match kv_heads*num_repre*head_dim")
-    if repre.dtype != torch.bfloat16 and repre.dtype != torch.float32:
+    table = repre.dtype
+    if table != torch.bfloat16 and table != torch.float32:
         raise ValueError("repre must be float32 or bfloat16")
     n_req = seg_off.numel()
     n_layers = qs[0] if n_layers is None else n_layers
@@ -224,7 +225,7 @@ def score_select(q: torch.Tensor, repre: torch.Tensor, seg_off: torch.Tensor, se
     i32 = torch.int32
     args = _lib.pack_score_select(
         _dev(q, q.dtype, "q"), _q_code(q), q_heads, q.stride(0), _opt(q_rows, i32, "q_rows") or 0,
-        _dev(repre, repre.dtype, "repre"), _lib.DTYPE_BF16 if repre.dtype == torch.bfloat16 else _lib.DTYPE_F32, num_repre,
+        _dev(repre, table, "repre"), _lib.DTYPE_BF16 if table == torch.bfloat16 else _lib.DTYPE_F32, num_repre,
         repre.stride(0), rs[1], _dev(seg_off, i32, "seg_off"), _dev(seg_len, i32, "seg_len"),
         _dev(topk_len, i32, "topk_len"), n_req, max_seg_len, first_layer, n_layers, kv_heads, head_dim,
         _dev(scores, torch.float32, "scores"), scores.stride(0), float(scale), int(tile_blocks), start_w, end_w,
