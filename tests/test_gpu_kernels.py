@@ -98,6 +98,47 @@ def test_block_mean_of_fp16_caches(ucm, dev, hkv, d, bs):
                        bs, hkv, d, nb)
 
 
+@pytest.mark.parametrize("hkv,d,bs,keys,table", [
+    (8, 128, 16, "bfloat16", "bfloat16"),     # two list entries side by side
+    (8, 128, 128, "float16", "float32"),      # more groups per workgroup than LDS holds: written out on the way
+    (1, 8, 16, "bfloat16", "float32"),        # 256 entries side by side, several to a wave
+    (1, 64, 32, "bfloat16", "bfloat16"),
+    (3, 96, 48, "bfloat16", "float32"),       # a row that does not divide the workgroup
+    (16, 256, 16, "bfloat16", "bfloat16"),    # two column groups
+])
+def test_block_mean_of_large_launches(ucm, dev, hkv, d, bs, keys, table):
+    """256 MiB of keys and more (by repeated blocks) take persistent workgroups: every entry like the oracle's mean of its
+    block, bad ids and slots skipped."""
+    from ucm_amd import ops
+
+    nb, L, row = 37, 3, hkv * d
+    n = (256 << 20) // (L * bs * row * 2) + 333
+    rows = n + 5
+    f16 = keys == "float16"
+    host = np.stack([synth.normal_f32(140 + l, (nb, bs, hkv, d)) for l in range(L)])
+    caches = torch.from_numpy(host).to(torch.float16 if f16 else torch.bfloat16)
+    caches_h = caches.view(torch.int16).numpy().view(np.uint16)
+    caches = caches.to(dev)
+    rng = np.random.default_rng(11)
+    ids, slots = rng.integers(0, nb, n).astype(np.int32), rng.permutation(rows)[:n].astype(np.int32)
+    bad = rng.permutation(n)[:9]
+    good = np.ones(n, bool)
+    good[bad] = False
+    ids[bad[:5]] = [-1, nb, nb + 7, 2 ** 31 - 1, -2 ** 31]
+    slots[bad[5:]] = [-1, rows, rows + 100, -2 ** 31]
+    tdt = torch.float32 if table == "float32" else torch.bfloat16
+    repre = torch.full((L, rows, row), 7.0, dtype=tdt, device=dev)
+    ops.block_mean(ops.LayerPointers([caches[l] for l in range(L)]), i32(ids, dev), i32(slots, dev), repre, bs, hkv, d, nb,
+                   mode=ops.MEAN_BF16_ROUND)
+    for l in range(L):
+        of_block = np.zeros((nb, row), np.float32)
+        O.block_mean_paged(caches_h[l], np.arange(nb), np.arange(nb), of_block, round_bf16=True, keys_f16=f16)
+        want = torch.full((rows, row), 7.0, dtype=tdt, device=dev)
+        at = torch.from_numpy(slots[good].astype(np.int64)).to(dev)
+        want[at] = torch.from_numpy(of_block).to(dev)[torch.from_numpy(ids[good].astype(np.int64)).to(dev)].to(tdt)
+        assert torch.equal(repre[l], want), l
+
+
 def test_block_mean_skips_bad_ids_and_layer_range(ucm, dev):
     from ucm_amd import ops
 
