@@ -101,6 +101,52 @@ def test_kvstar_block_repre_of_fp16_keys(ucm, dev, merge, hkv, d, bs):
     assert torch.allclose(mine.float(), t.float(), rtol=2 ** -10, atol=1e-6)
 
 
+@pytest.mark.parametrize("merge,hkv,d,bs,kept,keys", [
+    (1, 8, 128, 128, 128, "bfloat16"),     # all channels; a block's means do not fit LDS at once
+    (2, 8, 128, 128, 37, "bfloat16"),      # pieces that do not divide the workgroup, a padded last one
+    (2, 4, 128, 128, 32, "float16"),       # a block is one unit of loads
+    (4, 8, 128, 64, 32, "bfloat16"),
+    (8, 16, 128, 64, 64, "float16"),
+    (2, 1, 64, 1024, 16, "bfloat16"),
+])
+def test_kvstar_block_repre_of_blocks_in_whole_units(ucm, dev, merge, hkv, d, bs, kept, keys):
+    """Blocks of 128 KiB and multiples go through the workgroups of sixteen waves, several entries to each, with channel
+    lists named per entry (and layer): like the oracle's, bad blocks, rows and lists skipped."""
+    from ucm_amd import ops
+
+    L, nb, n, M, n_lists = 3, 5, 203, bs // merge, 2
+    rows, d_pad, f16 = n + 4, (kept + 15) // 16 * 16, keys == "float16"
+    caches = [torch.from_numpy(synth.normal_f32(1700 + l, (nb, bs, hkv, d))).to(torch.float16 if f16 else torch.bfloat16) for l in range(L)]
+    caches_h = [c.view(torch.int16).numpy().view(np.uint16) for c in caches]
+    rng = np.random.default_rng(1710 + merge)
+    ids, slots = rng.integers(0, nb, n).astype(np.int32), rng.permutation(rows)[:n].astype(np.int32)
+    sel = rng.integers(0, n_lists, n).astype(np.int32)
+    good = np.ones(n, bool)
+    bad = rng.permutation(n)[:6]
+    good[bad] = False
+    ids[bad[:2]], slots[bad[2:4]] = [-1, nb], [-1, rows]
+    pruned = None
+    if kept < d:
+        sel[bad[4:]] = [-1, n_lists]
+        pruned = np.stack([[[np.sort(rng.permutation(d)[:kept]) for _ in range(hkv)] for _ in range(n_lists)] for _ in range(L)]).astype(np.int32)
+    else:
+        good[bad[4:]] = True
+    i32 = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    repre = ops.kvstar_table(L, hkv, rows, M, d_pad, dev).fill_(3.0)
+    ops.kvstar_block_repre(ops.LayerPointers([c.to(dev) for c in caches]), i32(ids), i32(slots), repre, bs, hkv, d, nb, merge,
+                           pruned=None if pruned is None else i32(pruned), pruned_sel=None if pruned is None else i32(sel))
+    got = ops.kvstar_table_to_reference(repre).contiguous().view(torch.int16).cpu().numpy().view(np.uint16)
+    for l in range(L):
+        want = np.full((rows, M, hkv, d_pad), np.float16(3.0).view(np.uint16), np.uint16)
+        for s in range(n_lists if pruned is not None else 1):
+            of_block = np.zeros((nb, M, hkv, d_pad), np.uint16)
+            O.kvstar_block_repre(caches_h[l], np.arange(nb, dtype=np.int32), np.arange(nb, dtype=np.int32), merge, of_block,
+                                 pruned=None if pruned is None else pruned[l, s], keys_f16=f16)
+            mine = good & ((sel == s) if pruned is not None else True)
+            want[slots[mine]] = of_block[ids[mine]]
+        assert np.array_equal(got[l], want), l
+
+
 @pytest.mark.parametrize("merge", [2, 16, 3])      # the persistent kernel, and the one for other sub-block sizes (16 and 3)
 def test_kvstar_block_repre_channel_lists_per_layer(ucm, dev, merge):
     """One launch over all layers with a different set of kept channels in each (the reference picks them per layer

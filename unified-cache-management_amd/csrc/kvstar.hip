@@ -62,14 +62,23 @@ __device__ __forceinline__ unsigned short f32_to_f16_bits(float f)
 // Phase 2 gathers the kept channels from LDS and writes the pieces, consecutive threads to consecutive
 // 16 bytes.
 constexpr int kRepreUnroll = 16;
+constexpr unsigned kWideThreads = 1024;  // of kvstar_repre_wide_kernel,
+constexpr int kWideUnroll = 8;
+constexpr unsigned kWideLds = 158 * 1024;
+constexpr unsigned kWideGroups = 256;    // one workgroup on each compute unit
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// (v_cvt_pk_bf16_f32 and v_cvt_pk_f16_f32: round to nearest even, subnormals kept; the two are checked against the same
+// rounding in integers for every fp32 value that is no NaN)
 __device__ __forceinline__ unsigned mean_to_f16x2(float lo, float hi, float inv)
 {
-    unsigned a = __float_as_uint(lo * inv), b = __float_as_uint(hi * inv);
-    a += 0x7fffu + ((a >> 16) & 1u);
-    b += 0x7fffu + ((b >> 16) & 1u);
-    return static_cast<unsigned>(f32_to_f16_bits(__uint_as_float(a & 0xffff0000u))) |
-           (static_cast<unsigned>(f32_to_f16_bits(__uint_as_float(b & 0xffff0000u))) << 16);
+    const f32x2 mean = {lo * inv, hi * inv};
+    const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector(mean, bf16x2));
+    const f32x2 wide = {__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(wide, f16x2));
 }
 
 __device__ __forceinline__ void add_bf16x8(float (&acc)[8], const u32x4 v)
@@ -86,7 +95,8 @@ __device__ __forceinline__ unsigned mean_f16keys_to_f16x2(float lo, float hi, fl
 {
     float a = lo * inv, b = hi * inv;
     asm volatile("" : "+v"(a), "+v"(b));     // the product is rounded to fp32 first, as torch's mean is, then converted
-    return static_cast<unsigned>(f32_to_f16_bits(a)) | (static_cast<unsigned>(f32_to_f16_bits(b)) << 16);
+    const f32x2 mean = {a, b};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(mean, f16x2));
 }
 
 __device__ __forceinline__ void add_f16x8(float (&acc)[8], const u32x4 v)
@@ -122,13 +132,14 @@ struct PieceMap {
     int d[8];
 };
 
+template <unsigned kT>
 __device__ __forceinline__ PieceMap make_piece_map(const int32_t* __restrict__ lists, unsigned kv_heads, unsigned head_dim,
                                                    unsigned d_pruned, unsigned pieces)
 {
     PieceMap m;
     const unsigned pairs = kv_heads * pieces;
-    m.fixed = lists != nullptr && pairs <= static_cast<unsigned>(kThreads) && (kThreads % pairs) == 0;
-    m.tpp = m.fixed ? kThreads / pairs : 1u;
+    m.fixed = lists != nullptr && pairs <= kT && (kT % pairs) == 0;
+    m.tpp = m.fixed ? kT / pairs : 1u;
     const unsigned pair = threadIdx.x / m.tpp;
     m.sub = threadIdx.x - pair * m.tpp;
     m.h = m.fixed ? pair / pieces : 0u;
@@ -151,6 +162,7 @@ __device__ __forceinline__ PieceMap make_piece_map(const int32_t* __restrict__ l
 // The stores are non-temporal: the table is not read again by this kernel, and one byte written per eight read
 // costs less that way (a plain streaming kernel with the same mix of 32.4 GB read and 4 GB written measures
 // 6.6 ms with non-temporal stores and 7.0 ms with plain ones; this kernel 7.2 against 7.4).
+template <unsigned kT>
 __device__ __forceinline__ void repre_write_pieces(const unsigned short* __restrict__ stage, const int32_t* __restrict__ kept,
                                                    bool pruned, unsigned kv_heads, unsigned head_dim, unsigned d_pruned,
                                                    unsigned pieces, unsigned srow_stride, unsigned M, unsigned m0, unsigned mc,
@@ -173,7 +185,7 @@ __device__ __forceinline__ void repre_write_pieces(const unsigned short* __restr
         }
         return;
     }
-    for (unsigned e = threadIdx.x; e < kv_heads * pieces * mc; e += kThreads) {
+    for (unsigned e = threadIdx.x; e < kv_heads * pieces * mc; e += kT) {
         const unsigned h = e / (pieces * mc), rem = e - h * (pieces * mc);
         const unsigned piece = rem / mc, ml = rem - piece * mc;
         const unsigned short* srow = stage + ml * srow_stride + h * head_dim;
@@ -230,7 +242,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_repre_kernel(
     if (pruned) {   // this layer's lists (a stride of 0: one set of lists for every layer)
         for (unsigned e = threadIdx.x; e < kv_heads * d_pruned; e += kThreads) { kept[e] = my_lists[e]; }
     }
-    PieceMap pm = make_piece_map(my_lists, kv_heads, head_dim, d_pruned, pieces);
+    PieceMap pm = make_piece_map<kThreads>(my_lists, kv_heads, head_dim, d_pruned, pieces);
     // list_sel: every listed block names the list of the layer's n_lists it is pruned by (the blocks of several
     // requests in one launch, each request with channels of its own); the list in use is replaced when a block
     // names another one, which is once per request and workgroup
@@ -328,12 +340,12 @@ __global__ __launch_bounds__(kThreads) void kvstar_repre_kernel(
                 const int32_t* lists = my_lists + static_cast<size_t>(cur_list) * kv_heads * d_pruned;
                 __syncthreads();                         // nobody reads the old list any more
                 for (unsigned e = threadIdx.x; e < kv_heads * d_pruned; e += kThreads) { kept[e] = lists[e]; }
-                pm = make_piece_map(lists, kv_heads, head_dim, d_pruned, pieces);
+                pm = make_piece_map<kThreads>(lists, kv_heads, head_dim, d_pruned, pieces);
             }
             __syncthreads();
             unsigned short* out = repre + static_cast<int64_t>(blockIdx.y) * layer_stride +
                                   static_cast<int64_t>(static_cast<unsigned>(slots[u.item])) * row_stride;
-            repre_write_pieces(stage, kept, pruned != nullptr, kv_heads, head_dim, d_pruned, pieces, srow_stride, M, u.m0, mc,
+            repre_write_pieces<kThreads>(stage, kept, pruned != nullptr, kv_heads, head_dim, d_pruned, pieces, srow_stride, M, u.m0, mc,
                                out, head_stride, pm);
             __syncthreads();                             // the next chunk overwrites the staged means
         }
@@ -355,6 +367,125 @@ __global__ __launch_bounds__(kThreads) void kvstar_repre_kernel(
         load_unit(va, c.valid ? c : a);
         finish_unit(vb, b.valid ? b : a, b.valid);
         if (!c.valid) { break; }
+        a = c;
+    }
+}
+
+// Blocks that are whole 128 KiB units (kWideThreads x kWideUnroll loads of 16 bytes), whose rows divide the workgroup.  One
+// workgroup of sixteen waves per compute unit, persistent over the (layer, list entry) pairs.  What bounds it is HBM's rate for
+// reads with writes among them, which depends on how the writes come: a streaming loop with one 4 KiB run written per 32 KiB read
+// takes 1730 us for 8.6 GB of keys when two workgroups of four waves per compute unit write at times of their own, 1610 when
+// sixteen waves write a block's pieces together, 1200 without writes.  And on how little else the waves do: a thread's column
+// group never changes and its items lie at the same places of every unit, so a load is a scalar base and an offset kept in
+// a register.  32 layers x 1024 blocks of 128 tokens x 8 heads, a quarter of the channels kept, against kvstar_repre_kernel:
+// merge 2 1892 -> 1702 us, 4 1727 -> 1639; half the blocks: merge 8 817 -> 748, merge 2 with all channels 1280 -> 1171; 64-token
+// blocks 950 -> 849, 4 heads 944 -> 853; one layer, 600 blocks 43.4 -> 35.4, 64 blocks 13.6 -> 11.7, 16 blocks 12.0 -> 11.8.
+template <int kMerge, bool kF16>
+__global__ __launch_bounds__(kWideThreads) void kvstar_repre_wide_kernel(
+    const void* const* __restrict__ k_layers, const int32_t* __restrict__ block_ids,
+    const int32_t* __restrict__ slots, unsigned num_blocks, unsigned n_items, unsigned rows, unsigned block_size,
+    unsigned kv_heads, unsigned head_dim, const int32_t* __restrict__ pruned, int64_t pruned_layer_stride,
+    const int32_t* __restrict__ list_sel, unsigned n_lists,
+    unsigned d_pruned, unsigned d_pad, unsigned short* __restrict__ repre, int64_t layer_stride, int64_t head_stride,
+    int64_t row_stride, unsigned m_chunk, unsigned total)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned short stage[];   // [m_chunk][row + 8], then the channel lists in use
+    constexpr unsigned kItems = kWideUnroll / kMerge;                        // (sub-block, 8 columns) items of a thread and unit
+    const unsigned M = block_size / kMerge, row = kv_heads * head_dim, ncg = row / 8, srow_stride = row + 8, pieces = d_pad / 8;
+    const unsigned item_subs = kWideThreads / ncg, unit_subs = item_subs * kItems;
+    const unsigned tq = threadIdx.x / ncg, tr = threadIdx.x - tq * ncg;
+    const unsigned mine = tq * kMerge * row + tr * 8;
+    const float inv = 1.0f / static_cast<float>(kMerge);
+    int32_t* kept = reinterpret_cast<int32_t*>(stage + static_cast<size_t>(m_chunk) * srow_stride);
+
+    struct Unit {
+        unsigned g, layer, m0, slot, list;               // slot: kNoRow if the entry names no block, row or list
+        const unsigned short* blk;
+    };
+    constexpr unsigned kNoRow = 0xffffffffu;
+    auto open = [&](Unit& u, unsigned g) {
+        u.g = g;
+        u.layer = g / n_items;
+        u.m0 = 0;
+        const unsigned i = g - u.layer * n_items, id = static_cast<unsigned>(block_ids[i]), slot = static_cast<unsigned>(slots[i]);
+        u.list = list_sel ? static_cast<unsigned>(list_sel[i]) : 0u;
+        // (loads are unconditional: a bad id is never followed, the layer's first block is read in its place)
+        u.slot = id < num_blocks && slot < rows && u.list < n_lists ? slot : kNoRow;
+        u.blk = static_cast<const unsigned short*>(k_layers[u.layer]) + static_cast<size_t>(id < num_blocks ? id : 0u) * block_size * row;
+    };
+    auto next_of = [&](const Unit& u, bool& exists) -> Unit {
+        Unit n = u;
+        n.m0 = u.m0 + unit_subs;
+        if (n.m0 >= M) {
+            exists = u.g + gridDim.x < total;
+            if (exists) { open(n, u.g + gridDim.x); }
+        }
+        return n;
+    };
+    auto load_unit = [&](u32x4 (&v)[kWideUnroll], const Unit& u) {
+        const unsigned short* src = u.blk + static_cast<size_t>(u.m0) * kMerge * row;
+#pragma unroll
+        for (unsigned j = 0; j < kItems; ++j) {
+#pragma unroll
+            for (unsigned t = 0; t < kMerge; ++t) { v[j * kMerge + t] = ucm::gload16_nt(src + (j * item_subs * kMerge + t) * row + mine); }
+        }
+        // keeps the compiler from sinking the loads to their use, and from forming the other unit's means before they are issued
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    PieceMap pm = {};
+    unsigned cur_layer = kNoRow, cur_list = 0;
+    auto finish_unit = [&](const u32x4 (&v)[kWideUnroll], const Unit& u, bool exists) {
+        const unsigned chunk0 = u.m0 / m_chunk * m_chunk;
+#pragma unroll
+        for (unsigned j = 0; j < kItems; ++j) {
+            float acc[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) { acc[c] = -0.0f; }   // -0 + x == x for every x, signed zeros included
+#pragma unroll
+            for (unsigned t = 0; t < kMerge; ++t) { add_keys8<kF16>(acc, v[j * kMerge + t]); }
+            u32x4 o;
+            o.x = mean_pair<kF16>(acc[0], acc[1], inv);
+            o.y = mean_pair<kF16>(acc[2], acc[3], inv);
+            o.z = mean_pair<kF16>(acc[4], acc[5], inv);
+            o.w = mean_pair<kF16>(acc[6], acc[7], inv);
+            *reinterpret_cast<u32x4*>(&stage[(u.m0 - chunk0 + j * item_subs + tq) * srow_stride + tr * 8]) = o;
+        }
+        const unsigned end = u.m0 + unit_subs;
+        if (end != M && end != chunk0 + m_chunk) { return; }
+        // the chunk is staged: write its pieces (all conditions here are the same for all threads)
+        const bool live = exists && u.slot != kNoRow;
+        if (live && pruned && (u.layer != cur_layer || u.list != cur_list)) {
+            cur_layer = u.layer;
+            cur_list = u.list;
+            const int32_t* lists = pruned + static_cast<int64_t>(cur_layer) * pruned_layer_stride + static_cast<size_t>(cur_list) * kv_heads * d_pruned;
+            // (nobody reads the old lists any more: a barrier has followed the last chunk's pieces)
+            for (unsigned e = threadIdx.x; e < kv_heads * d_pruned; e += kWideThreads) { kept[e] = lists[e]; }
+            pm = make_piece_map<kWideThreads>(lists, kv_heads, head_dim, d_pruned, pieces);
+        }
+        __syncthreads();
+        if (live) {
+            unsigned short* out = repre + static_cast<int64_t>(u.layer) * layer_stride + static_cast<int64_t>(u.slot) * row_stride;
+            repre_write_pieces<kWideThreads>(stage, kept, pruned != nullptr, kv_heads, head_dim, d_pruned, pieces, srow_stride, M, chunk0,
+                                             end - chunk0, out, head_stride, pm);
+        }
+        __syncthreads();                                 // the next chunk overwrites the staged means
+    };
+
+    Unit a;
+    open(a, blockIdx.x);
+    u32x4 va[kWideUnroll], vb[kWideUnroll];
+    load_unit(va, a);
+    for (;;) {                                           // one way out, at the end: see kvstar_repre_kernel
+        bool has_b = true, has_c = true;
+        const Unit b = next_of(a, has_b);
+        load_unit(vb, has_b ? b : a);
+        finish_unit(va, a, true);
+        const Unit c = has_b ? next_of(b, has_c) : b;
+        has_c = has_c && has_b;
+        load_unit(va, has_c ? c : a);
+        finish_unit(vb, has_b ? b : a, has_b);
+        if (!has_c) { break; }
         a = c;
     }
 }
@@ -388,7 +519,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_repre_any_kernel(
     if (pruned) {
         for (unsigned e = threadIdx.x; e < kv_heads * d_pruned; e += kThreads) { kept[e] = my_lists[e]; }
     }
-    const PieceMap pm = make_piece_map(my_lists, kv_heads, head_dim, d_pruned, pieces);
+    const PieceMap pm = make_piece_map<kThreads>(my_lists, kv_heads, head_dim, d_pruned, pieces);
     for (unsigned m0 = 0; m0 < M; m0 += m_chunk) {       // m_chunk sub-blocks at a time: what fits LDS
         const unsigned mc = min(m_chunk, M - m0);
         for (unsigned w = threadIdx.x; w < mc * ncg; w += kThreads) {
@@ -414,7 +545,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_repre_any_kernel(
             *reinterpret_cast<u32x4*>(&stage[ml * srow_stride + cg * 8]) = o;
         }
         __syncthreads();
-        repre_write_pieces(stage, kept, pruned != nullptr, kv_heads, head_dim, d_pruned, pieces, srow_stride, M, m0, mc, out,
+        repre_write_pieces<kThreads>(stage, kept, pruned != nullptr, kv_heads, head_dim, d_pruned, pieces, srow_stride, M, m0, mc, out,
                            head_stride, pm);
         __syncthreads();                                 // the next chunk overwrites the staged means
     }
@@ -1121,11 +1252,44 @@ extern "C" int ucm_kvstar_block_repre_keys(const void* const* k_layers, int key_
     UCM_SUPPORTED(row % 8 == 0 && d_pad % 8 == 0, "ucm_kvstar_block_repre: kv_heads*head_dim=%u and d_pad=%d must be multiples of 8",
                   row, d_pad);
     UCM_SUPPORTED(row <= 32768u && head_dim % 8 == 0, "ucm_kvstar_block_repre: kv_heads*head_dim=%u (at most 32768), head_dim=%d (a multiple of 8)", row, head_dim);
-    const unsigned m_chunk = std::min<unsigned>(static_cast<unsigned>(M), 33280u / (row + 8));   // sub-blocks staged at a time: 65 KiB of LDS
-    const size_t lds_bytes = static_cast<size_t>(m_chunk) * (row + 8) * 2 + (pruned ? static_cast<size_t>(kv_heads) * d_pruned * 4 : 0);
+    // sub-blocks staged at a time, and what the channel lists take: 65 KiB of LDS, or what the wide kernel has
+    const unsigned list_bytes = pruned ? static_cast<unsigned>(kv_heads) * d_pruned * 4 : 0u;
+    unsigned m_chunk = std::min<unsigned>(static_cast<unsigned>(M), 33280u / (row + 8));
+    const unsigned ncg = row / 8;
+    bool wide = (merge == 1 || merge == 2 || merge == 4 || merge == 8) && ncg <= kWideThreads && kWideThreads % ncg == 0 &&
+                static_cast<uint64_t>(n) * n_layers <= 0x7fffffffull;
+    if (wide) {
+        const unsigned unit_subs = kWideThreads / ncg * (kWideUnroll / merge);
+        const unsigned fit = kWideLds > list_bytes ? (kWideLds - list_bytes) / ((row + 8) * 2) / unit_subs * unit_subs : 0u;
+        wide = M % unit_subs == 0 && fit > 0;
+        if (wide) { m_chunk = std::min<unsigned>(static_cast<unsigned>(M), fit); }
+    }
+    const size_t lds_bytes = static_cast<size_t>(m_chunk) * (row + 8) * 2 + list_bytes;
     UCM_REQUIRE(ucm::aligned16(repre_f16) && repre_layer_stride % 8 == 0 && repre_head_stride % 8 == 0 &&
                     repre_row_stride % 8 == 0, "ucm_kvstar_block_repre: table not 16-byte aligned");
     hipStream_t hs = ucm::as_stream(stream);
+    if (wide) {
+        const unsigned total = static_cast<unsigned>(n) * static_cast<unsigned>(n_layers);
+        const unsigned each = (total + kWideGroups - 1) / kWideGroups, wgs = (total + each - 1) / each;
+        auto launch = [&](auto kernel) -> int {
+            const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                      static_cast<int>(lds_bytes));
+            if (ea != hipSuccess) { return ucm::check_hip(ea, "ucm_kvstar_block_repre (LDS size)"); }
+            hipLaunchKernelGGL(kernel, dim3(wgs), dim3(kWideThreads), lds_bytes, hs, k_layers, block_ids, slots,
+                               static_cast<unsigned>(num_blocks), static_cast<unsigned>(n), static_cast<unsigned>(repre_rows),
+                               static_cast<unsigned>(block_size), static_cast<unsigned>(kv_heads), static_cast<unsigned>(head_dim),
+                               pruned, pruned_layer_stride, pruned_sel, static_cast<unsigned>(lists_per_layer),
+                               static_cast<unsigned>(d_pruned), static_cast<unsigned>(d_pad), static_cast<unsigned short*>(repre_f16),
+                               repre_layer_stride, repre_head_stride, repre_row_stride, m_chunk, total);
+            return ucm::check_hip(hipGetLastError(), "ucm_kvstar_block_repre");
+        };
+        switch (merge) {
+        case 1: return f16 ? launch(kvstar_repre_wide_kernel<1, true>) : launch(kvstar_repre_wide_kernel<1, false>);
+        case 2: return f16 ? launch(kvstar_repre_wide_kernel<2, true>) : launch(kvstar_repre_wide_kernel<2, false>);
+        case 4: return f16 ? launch(kvstar_repre_wide_kernel<4, true>) : launch(kvstar_repre_wide_kernel<4, false>);
+        default: return f16 ? launch(kvstar_repre_wide_kernel<8, true>) : launch(kvstar_repre_wide_kernel<8, false>);
+        }
+    }
     // persistent workgroups for the common sub-block sizes: about 1024 over all layers (two fit a compute unit)
     const unsigned gx = static_cast<unsigned>(std::min(n, std::max(1, (1024 + n_layers - 1) / n_layers)));
 #define UCM_KVSTAR_REPRE(MERGE)                                                                                        \
