@@ -79,6 +79,31 @@ def test_retrieval_worker_protocol_and_errors(ucm, dev):
     assert list(worker.get_result(rid)["indices"][0]) == [7, 3]
 
 
+@pytest.mark.parametrize("dim", [4, 124, 128, 132, 256, 260, 640, 1028])    # columns come in tiles of 128
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 33])                            # slots in groups of 16
+def test_esa_scores_at_tile_edges(ucm, dev, m, dim):
+    """Scores bit for bit and the order of the best ones, with entries that name no row among the candidates."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(1000 * m + dim)
+    data_h, q_h = rng.standard_normal((60, dim)).astype(np.float32), rng.standard_normal((2, dim)).astype(np.float32)
+    lists = np.stack([rng.permutation(60)[:m], rng.permutation(60)[:m]]).astype(np.int32)
+    lists[1, m // 2] = -1
+    lists[1, m // 3] = 60
+    k = m
+    ws, oi = torch.empty(2 * m, device=dev), torch.full((2, k), -7, dtype=torch.int32, device=dev)
+    os_, oc = torch.full((2, k), -7.0, device=dev), torch.zeros(2, dtype=torch.int32, device=dev)
+    ops.esa_retrieve(torch.from_numpy(data_h).to(dev), torch.from_numpy(q_h).to(dev), torch.from_numpy(lists).to(dev), k, ws, oi, os_, oc)
+    for r in range(2):
+        live = lists[r][(lists[r] >= 0) & (lists[r] < 60)]
+        n = int(oc[r])
+        assert n == len(live)
+        if n:
+            wi, wsc = O.esa_retrieve(data_h, q_h[r], live, n)
+            assert np.array_equal(oi[r, :n].cpu().numpy(), wi)
+            assert np.array_equal(os_[r, :n].cpu().numpy().view(np.uint32), np.asarray(wsc, np.float32).view(np.uint32))
+
+
 def test_esa_retrieve_wide_and_ragged_rows(ucm, dev):
     """Batch of requests, -1 padding in the middle, out-of-range slots, dims that are not a multiple of the tile."""
     from ucm_amd import ops

@@ -3,16 +3,21 @@
 //
 // The reference scores each slot with a strictly sequential
 //     score = score + q[d] * data[slot][d]        (separate multiply and add)
-// The products do not depend on the order, the additions do: 256 threads of a
+// The products do not depend on the order, the additions do: four waves of a
 // workgroup multiply the 16-byte pieces they fetch (coalesced, rows are 4 KiB
-// apart) by the query and park the products in LDS, column-major with an odd
-// column stride, and one wave then adds its slot's products in order - per
-// dimension one LDS read at a constant offset and one dependent add, nothing
-// else.  That is all this wave does: two product tiles alternate, the four other
-// waves fill the next tile while the chain of the current one runs, and the loads
-// of the tile after that are in flight.  Latency-bound by design (a chain of `dim`
-// dependent adds): 16 requests of up to 512 slots x 1024 dims take 12.4 us, 13.2
-// when the wave that adds multiplied a quarter of every tile as well.
+// apart) by the query and park the products in LDS, a piece of four columns at a
+// time, and one wave then adds its slot's products in order - one LDS read and
+// four dependent adds per piece.  That is all this wave does: two product tiles
+// alternate, the four other waves fill the next tile while the chain of the
+// current one runs, and the loads of the tile after that are in flight.
+// Latency-bound by design: an add waits 8 cycles for the one before it, 4.1 us
+// for 1024 dims, after the trips to memory for the slots and the first rows.
+// Hence few slots per workgroup, so that every compute unit has rows to fetch: 16
+// requests of up to 512 slots x 1024 dims 10.5 us (64 slots per workgroup and one
+// LDS read per column: 14.0).  With the selection: 1 x 64 slots 16.4 -> 12.4 us,
+// 32 x 1000 32.6 -> 25.6, 8 x 4000 of 512 dims 33.4 -> 29.0, 16 x 512 of 4096
+// dims 43.8 -> 32.9; 32 slots per workgroup or four or eight tiles in flight are
+// 2 to 40 % slower, 8 slots 3 to 10 %.
 //
 // Selection ranks 64-bit keys (order-preserving score bits, then position
 // ascending) by counting the keys above each, spread over workgroups.
@@ -25,12 +30,13 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kSlots = 64;          // slots (rows) per workgroup
+constexpr int kSlots = 16;          // slots (rows) per workgroup
 constexpr int kCols = 128;          // columns per tile
-constexpr int kColStride = kSlots + 1;  // odd: lane r reading column d hits bank (r + d) % 64
+constexpr int kPieces = kCols / 4;  // 16-byte pieces of a row in a tile
+constexpr int kPieceStride = kSlots + 1;    // pieces: an odd stride, so the 32 pieces of a row land on different banks
 constexpr int kScoreThreads = 256;  // that multiply; one more wave adds
-constexpr int kRowsPerLoad = kScoreThreads / (kCols / 4);  // 8 rows per 16-byte load instruction
-constexpr int kLoads = kSlots / kRowsPerLoad;              // 8 loads per thread per tile
+constexpr int kRowsPerLoad = kScoreThreads / kPieces;      // 8 rows per 16-byte load instruction
+constexpr int kLoads = kSlots / kRowsPerLoad;              // loads per thread per tile
 constexpr int kDepth = 2;                                  // tiles in flight per thread (an even number: two LDS buffers)
 
 // Row of the index matrix (and of every per-request output) that request b uses: b itself, or rows[b] when the
@@ -44,90 +50,83 @@ __device__ __forceinline__ bool request_row(const int32_t* __restrict__ rows, un
     return r >= 0 && row < n_rows;
 }
 
-// grid: x = group of 64 entries of the index row, y = request
+// grid: x = group of kSlots entries of the index row, y = request
 __global__ __launch_bounds__(kScoreThreads + 64) void esa_score_kernel(
     const float* __restrict__ data, unsigned n_items, unsigned dim, const float* __restrict__ q,
     const int32_t* __restrict__ indexes, unsigned m, float* __restrict__ scores,
     const int32_t* __restrict__ rows, unsigned n_rows, unsigned idx_stride)
 {
-    __shared__ float tile[2][kCols * kColStride];       // products, [column][slot]
-    __shared__ int32_t slot_of[kSlots];
+    __shared__ f32x4 tile[2][kPieces * kPieceStride];   // products, [piece of four columns][slot]
 
     const unsigned b = blockIdx.y, first = blockIdx.x * kSlots;
     unsigned row;
     if (!request_row(rows, n_rows, b, row)) { return; }   // (uniform)
-    const int32_t* idx_row = indexes + static_cast<size_t>(row) * idx_stride;
-    int32_t my_slot = -1;
-    if (threadIdx.x < kSlots) {
-        const unsigned e = first + threadIdx.x;
-        const int32_t s = e < m ? idx_row[e] : -1;
-        my_slot = (s >= 0 && static_cast<unsigned>(s) < n_items) ? s : -1;
-        slot_of[threadIdx.x] = my_slot;
-    }
+    // every wave looks at the group's entries by itself: no barrier stands before the first loads of rows
+    const unsigned lane = threadIdx.x & 63, mine_of = lane & (kSlots - 1);
+    int32_t slot = -1;
+    if (first + mine_of < m) { slot = indexes[static_cast<size_t>(row) * idx_stride + first + mine_of]; }
+    if (slot < 0 || static_cast<unsigned>(slot) >= n_items) { slot = -1; }
     // a group of padding only (short requests in a wide table) has nothing to score: the selection ignores the
     // scores of entries without a slot
-    if (!__syncthreads_or(my_slot >= 0)) { return; }
+    if (!__any(slot >= 0)) { return; }                   // (the same in all waves)
 
-    const bool adds = threadIdx.x >= kScoreThreads;      // (uniform in a wave)
-    const unsigned mine_of = threadIdx.x & (kSlots - 1);
-    // a multiplying thread's part of a tile: column group c4 (4 floats) of rows r0, r0+8, ...
-    const unsigned c4 = threadIdx.x % (kCols / 4), r0 = threadIdx.x / (kCols / 4) % kRowsPerLoad;
+    // Tiles alternate between two buffers; a buffer is rewritten two tiles later, after the barrier of the tile in between,
+    // which the chain wave only reaches when its chain is done.
+    const unsigned n_tiles = (dim + kCols - 1) / kCols;
+    if (threadIdx.x >= kScoreThreads) {                  // the wave that adds
+        float score = 0.0f;
+        auto add = [&](const f32x4 p) { score = score + p.x; score = score + p.y; score = score + p.z; score = score + p.w; };
+        for (unsigned t = 0; t < n_tiles; ++t) {
+            __syncthreads();
+            const f32x4* mine = &tile[t & 1][mine_of];
+            if ((t + 1) * kCols <= dim) {
+#pragma unroll
+                for (int d = 0; d < kPieces; ++d) { add(mine[d * kPieceStride]); }
+            } else {
+                for (unsigned d = 0; d < (dim - t * kCols) / 4; ++d) { add(mine[d * kPieceStride]); }
+            }
+        }
+        if (lane < kSlots && first + lane < m) { scores[static_cast<size_t>(b) * m + first + lane] = score; }
+        return;
+    }
+    // a multiplying thread's part of a tile: piece c4 (4 floats) of rows r0, r0+8, ...
+    const unsigned c4 = threadIdx.x % kPieces, r0 = threadIdx.x / kPieces;
     const float* row_ptr[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-        const int32_t s = slot_of[r0 + i * kRowsPerLoad];
-        row_ptr[i] = data + static_cast<size_t>(s < 0 ? 0 : s) * dim + c4 * 4;
+        const int32_t s = __shfl(slot, r0 + i * kRowsPerLoad, 64);
+        row_ptr[i] = data + static_cast<size_t>(s < 0 ? 0 : s) * dim;
     }
-    const float* qb = q + static_cast<size_t>(b) * dim + c4 * 4;
-
-    // kDepth tiles of loads are in flight per thread: a tile's chain (128 dependent adds) is several times
-    // shorter than a trip to memory, so the chain of tile t runs while tiles t+1 .. t+kDepth-1 are on their way
+    const float* qb = q + static_cast<size_t>(b) * dim;
+    // Loads are unconditional (pieces past the row's end reload its last one, and nothing adds them): a load that some path
+    // skips would make the compiler wait for all that are outstanding.
     f32x4 regs[kDepth][kLoads], qv[kDepth];
-    auto fetch = [&](int stage, unsigned col0) {
-        if (!adds && col0 + c4 * 4 < dim) {
-            qv[stage] = *reinterpret_cast<const f32x4*>(qb + col0);
+    auto fetch = [&](int stage, unsigned t) {
+        const unsigned col = min(t * kCols + c4 * 4, dim - 4);
+        qv[stage] = *reinterpret_cast<const f32x4*>(qb + col);
 #pragma unroll
-            for (int i = 0; i < kLoads; ++i) { regs[stage][i] = *reinterpret_cast<const f32x4*>(row_ptr[i] + col0); }
-        }
+        for (int i = 0; i < kLoads; ++i) { regs[stage][i] = *reinterpret_cast<const f32x4*>(row_ptr[i] + col); }
+        asm volatile("" ::: "memory");
+    };
+    auto multiply = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) { tile[stage & 1][c4 * kPieceStride + r0 + i * kRowsPerLoad] = qv[stage] * regs[stage][i]; }
+        __syncthreads();
     };
 #pragma unroll
-    for (int u = 0; u < kDepth; ++u) {
-        if (u * kCols < dim) { fetch(u, u * kCols); }
-    }
-    float score = 0.0f;
-    for (unsigned base = 0; base < dim; base += kDepth * kCols) {
+    for (int u = 0; u < kDepth; ++u) { fetch(u, u); }
+    unsigned t = 0;
+    for (; t + kDepth < n_tiles; t += kDepth) {
 #pragma unroll
         for (int u = 0; u < kDepth; ++u) {
-            const unsigned col0 = base + u * kCols;
-            if (col0 >= dim) { break; }                  // (uniform)
-            // (tiles alternate between two buffers; a buffer is rewritten two tiles later, after the barrier
-            // of the tile in between, which the chain wave only reaches when its chain is done)
-            float* tb = tile[u & 1];
-            if (!adds) {
-#pragma unroll
-                for (int i = 0; i < kLoads; ++i) {
-                    float* t = &tb[(c4 * 4) * kColStride + r0 + i * kRowsPerLoad];
-                    t[0] = qv[u].x * regs[u][i].x;
-                    t[kColStride] = qv[u].y * regs[u][i].y;
-                    t[2 * kColStride] = qv[u].z * regs[u][i].z;
-                    t[3 * kColStride] = qv[u].w * regs[u][i].w;
-                }
-            }
-            __syncthreads();
-            if (col0 + kDepth * kCols < dim) { fetch(u, col0 + kDepth * kCols); }
-            if (adds) {
-                const float* mine = &tb[mine_of];
-                if (col0 + kCols <= dim) {
-#pragma unroll 32
-                    for (int d = 0; d < kCols; ++d) { score = score + mine[d * kColStride]; }
-                } else {
-                    for (unsigned d = 0; d < dim - col0; ++d) { score = score + mine[d * kColStride]; }
-                }
-            }
+            multiply(u);
+            fetch(u, t + kDepth + u);
         }
     }
-    if (adds && first + mine_of < m) {
-        scores[static_cast<size_t>(b) * m + first + mine_of] = score;
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+        if (t + u >= n_tiles) { return; }                // (uniform)
+        multiply(u);
     }
 }
 
@@ -165,6 +164,10 @@ __global__ __launch_bounds__(kRankThreads) void esa_rank_kernel(
     const float* s_row = scores + static_cast<size_t>(b) * m;
     const int32_t* idx_row = indexes + static_cast<size_t>(row) * idx_stride;
     if (threadIdx.x == 0) { valid_total = 0; }
+    // what a candidate writes if it is selected, requested with everything else
+    const unsigned cand = blockIdx.x * (kRankThreads / kLanes) + threadIdx.x / kLanes, sub = threadIdx.x % kLanes;
+    const int32_t my_slot = cand < m ? idx_row[cand] : -1;
+    const float my_score = cand < m ? s_row[cand] : 0.0f;
     __syncthreads();
     unsigned mine = 0;
     for (unsigned e0 = threadIdx.x; e0 < n_pad; e0 += 8 * kRankThreads) {
@@ -191,7 +194,6 @@ __global__ __launch_bounds__(kRankThreads) void esa_rank_kernel(
     __syncthreads();
     if (blockIdx.x == 0 && threadIdx.x == 0) { out_count[row] = max(0, min(static_cast<int>(valid_total), topk)); }
 
-    const unsigned cand = blockIdx.x * (kRankThreads / kLanes) + threadIdx.x / kLanes, sub = threadIdx.x % kLanes;
     const unsigned long long my = cand < m ? keys[cand] : 0ull;
     // two keys per 16-byte read, eight reads in flight; n_pad is a multiple of 16 * kLanes
     typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
@@ -207,8 +209,8 @@ __global__ __launch_bounds__(kRankThreads) void esa_rank_kernel(
 #pragma unroll
     for (int d = 1; d < kLanes; d <<= 1) { above += __shfl_xor(above, d, 64); }
     if (sub == 0 && my != 0ull && static_cast<int>(above) < topk) {      // (a valid key is never zero)
-        out_idx[static_cast<size_t>(row) * out_stride + above] = idx_row[cand];
-        out_scores[static_cast<size_t>(row) * out_stride + above] = s_row[cand];
+        out_idx[static_cast<size_t>(row) * out_stride + above] = my_slot;
+        out_scores[static_cast<size_t>(row) * out_stride + above] = my_score;
         if (out_pos) { out_pos[static_cast<size_t>(row) * out_stride + above] = static_cast<int32_t>(cand); }
     }
 }
