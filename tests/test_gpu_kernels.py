@@ -638,6 +638,48 @@ def test_kv_dump_load_round_trip(ucm, dev, bb):
     assert np.array_equal(staging.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("bb", [16, 8192 - 16, 8192, 8192 + 16, 131072, 131072 + 16, 3 * 131072 + 8192 + 48])
+def test_kv_moves_at_the_sizes_of_pieces(ucm, dev, bb):
+    """Slices around what 256 threads take and around pieces of 128 KiB: dumps, loads and gathers of selected blocks, byte
+    for byte, unusable ids and slots past the staging area left alone."""
+    from ucm_amd import ops
+
+    L, nb, n, n_req, stride = 2, 9, 5, 2, 4
+    rng = np.random.default_rng(bb)
+    host = rng.integers(0, 256, (L, 2, nb, bb), dtype=np.uint8)
+    caches = [torch.from_numpy(host[l]).to(dev) for l in range(L)]
+    lp, ids = ops.LayerPointers(caches), np.array([3, nb, 0, -1, 8], np.int32)
+    staging = torch.full((n, L, 2, bb), 0xAB, dtype=torch.uint8, device=dev)
+    ops.kv_gather_blocks(lp, nb * bb, bb, nb, i32(ids, dev), staging)
+    want = np.full((n, L, 2, bb), 0xAB, np.uint8)
+    for i in (0, 2, 4):
+        want[i] = host[:, :, ids[i]]
+    assert np.array_equal(staging.cpu().numpy(), want)
+    to = np.array([1, nb, 7, -1, 2], np.int32)
+    ops.kv_scatter_blocks(lp, nb * bb, bb, nb, i32(to, dev), staging)
+    for i in (0, 2, 4):
+        host[:, :, to[i]] = want[i]
+    assert all(np.array_equal(caches[l].cpu().numpy(), host[l]) for l in range(L))
+    phys = rng.integers(0, nb, (L, n_req, stride)).astype(np.int32)
+    phys[0, 1, 1] = nb
+    count = np.array([[3, 2], [4, 0]], np.int32)
+    region = np.array([4, 2], np.int32)
+    off = np.array([0, 4 * L * 2], np.int64)
+    blocks = 6 * L * 2 - 1                                    # the last slot lies past the staging area
+    out = torch.full((blocks + 1, bb), 0xCD, dtype=torch.uint8, device=dev)
+    ops.kv_gather_selected(lp, nb * bb, bb, nb, i32(phys, dev), i32(count, dev), torch.from_numpy(off).to(dev), i32(region, dev),
+                           stride, out, blocks)
+    want = np.full((blocks + 1, bb), 0xCD, np.uint8)
+    for l in range(L):
+        for r in range(n_req):
+            for kv in range(2):
+                for j in range(count[l, r]):
+                    slot = off[r] + (l * 2 + kv) * region[r] + j
+                    if phys[l, r, j] < nb and slot < blocks:
+                        want[slot] = host[l, kv, phys[l, r, j]]
+    assert np.array_equal(out.cpu().numpy(), want)
+
+
 def test_kv_moves_of_one_tensor_parallel_rank(ucm, dev):
     """Four ranks share the stored block; each moves its own K and V slices to where get_offset (esa.py:124-135) puts
     them, leaves the others' bytes alone, and reads them back - through the block moves and through the planned load."""

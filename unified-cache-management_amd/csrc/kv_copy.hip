@@ -2,13 +2,12 @@
 // the stored-block layout, and the gather of selected blocks from a device
 // block table.  Pure HBM traffic: every byte is read once and written once, so
 // the kernels are 16-byte vector copies with non-temporal hints, one
-// 1024-thread workgroup per slice (a 256 KiB K or V block = 2 trips of 128 KiB
-// in flight), launched with far more workgroups than the 256 CUs.  Of the
+// 1024-thread workgroup per 128 KiB of a slice (a 256 KiB K or V block is two),
+// launched with far more workgroups than the 256 CUs.  Of the
 // shapes tried on MI355X (8 KiB .. 256 KiB per workgroup, 64 .. 1024 threads,
 // 1 .. 16 loads in flight per thread, persistent grids, with and without the
 // non-temporal hint) this one was the fastest; all of them sit between 5.2 and
-// 6.0 TB/s for a 1:1 read/write mix.  (Planned loads, most of whose workgroups may
-// have nothing to do, take smaller ones for short slices: kv_load_slot_kernel.)
+// 6.1 TB/s for a 1:1 read/write mix.  (Short slices take smaller ones.)
 #include "common.h"
 
 namespace {
@@ -18,6 +17,14 @@ using ucm::u32x4;
 constexpr int kThreads = 1024;
 constexpr int kUnroll = 8;
 constexpr size_t kStep = static_cast<size_t>(kThreads) * 16 * kUnroll;  // 128 KiB per trip
+
+// Gathers, dumps and loads by block list: a workgroup moves one trip (128 KiB) of a slice and ends with its stores on their
+// way.  (Both trips of a 256 KiB slice in one workgroup, us: 32 layers x 256 blocks out and back 2845 to 2911 by process, 2769 to 2828
+// this way; 5.1 GB gathered 1751 to 1821, 1707 to 1730; one layer of 20 blocks out and back 23.4, 14.2.)
+// Slices of up to 8 KiB, the blocks of one or two kv heads, take 256 threads: a compute unit has eight of them under way and only
+// two of 1024 (32 layers x 1024 blocks out and back, 4 KiB 299 -> 175 us = 6.1 TB/s, 8 KiB 435 -> 377; 16 KiB 730 -> 760, so no more).
+constexpr int kShortThreads = 256;
+constexpr size_t kShortSlice = 8 * 1024;
 
 // kN x 16 KiB of a slice: every load is issued before the first store goes out.  Stores that start as the
 // loads trickle in mix reads and writes on the HBM channels and cost about 6 % of the copy rate (1.64 ms ->
@@ -37,8 +44,7 @@ __device__ __forceinline__ void copy_trip(uint8_t* __restrict__ dst, const uint8
     }
 }
 
-// One workgroup copies one whole slice (a 256 KiB K or V block = 2 trips of 128 KiB).  size is a multiple of
-// 16.  What is left after the 128 KiB trips goes in trips of 64, 32 and 16 KiB (the slices of 64-, 32- and
+// A workgroup's share of a slice; size is a multiple of 16.  What is left after the 128 KiB trips goes in trips of 64, 32 and 16 KiB (the slices of 64-, 32- and
 // 16-token blocks), each with all its loads in flight at once, and a last partial one.  (kT threads: a trip is kT * 128 bytes.)
 template <int kT = kThreads>
 __device__ __forceinline__ void copy_slice(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t size)
@@ -76,32 +82,35 @@ struct StoredLayout {
     }
 };
 
-// grid: x = index into block_ids, y = layer, z = K|V
-template <bool kToStaging>
-__global__ __launch_bounds__(kThreads) void kv_blocks_kernel(void* const* __restrict__ layers,
+// grid: x = index into block_ids * pieces + piece, y = layer, z = K|V
+template <bool kToStaging, int kT>
+__global__ __launch_bounds__(kT) void kv_blocks_kernel(void* const* __restrict__ layers,
                                                              size_t kv_stride, size_t block_bytes,
                                                              const int32_t* __restrict__ block_ids,
                                                              unsigned num_blocks,
-                                                             uint8_t* __restrict__ staging, StoredLayout lay)
+                                                             uint8_t* __restrict__ staging, unsigned pieces, size_t piece, StoredLayout lay)
 {
-    const unsigned i = blockIdx.x, l = blockIdx.y, kv = blockIdx.z, n_layers = gridDim.y;
+    const unsigned i = pieces == 1 ? blockIdx.x : blockIdx.x / pieces, l = blockIdx.y, kv = blockIdx.z, n_layers = gridDim.y;
+    const size_t off = (blockIdx.x - i * pieces) * piece;
     const unsigned id = static_cast<unsigned>(block_ids[i]);
     if (id >= num_blocks) { return; }  // ids outside the cache are skipped, never dereferenced
     uint8_t* cache = static_cast<uint8_t*>(layers[l]) + kv * kv_stride +
-                     static_cast<size_t>(id) * block_bytes;
-    uint8_t* stage = staging + static_cast<size_t>(i) * n_layers * lay.layer_pitch + lay.slice(l, kv, block_bytes);
-    if (kToStaging) { copy_slice(stage, cache, block_bytes); }
-    else { copy_slice(cache, stage, block_bytes); }
+                     static_cast<size_t>(id) * block_bytes + off;
+    uint8_t* stage = staging + static_cast<size_t>(i) * n_layers * lay.layer_pitch + lay.slice(l, kv, block_bytes) + off;
+    const size_t size = min(piece, block_bytes - off);
+    if (kToStaging) { copy_slice<kT>(stage, cache, size); }
+    else { copy_slice<kT>(cache, stage, size); }
 }
 
-// grid: x = position in the request's selection, y = request, z = layer*2 + K|V
-__global__ __launch_bounds__(kThreads) void kv_gather_selected_kernel(
+// grid: x = position in the request's selection * pieces + piece, y = request, z = layer*2 + K|V
+template <int kT>
+__global__ __launch_bounds__(kT) void kv_gather_selected_kernel(
     const void* const* __restrict__ layers, size_t kv_stride, size_t block_bytes,
     const int32_t* __restrict__ phys, const int32_t* __restrict__ count, unsigned num_blocks,
     unsigned n_req, unsigned phys_stride, const int64_t* __restrict__ dst_off,
-    const int32_t* __restrict__ region_k, uint8_t* __restrict__ staging, uint64_t staging_blocks)
+    const int32_t* __restrict__ region_k, uint8_t* __restrict__ staging, uint64_t staging_blocks, unsigned pieces, size_t piece)
 {
-    const unsigned j = blockIdx.x, r = blockIdx.y, l = blockIdx.z >> 1, kv = blockIdx.z & 1;
+    const unsigned j = pieces == 1 ? blockIdx.x : blockIdx.x / pieces, r = blockIdx.y, l = blockIdx.z >> 1, kv = blockIdx.z & 1;
     const size_t lr = static_cast<size_t>(l) * n_req + r;
     if (static_cast<int32_t>(j) >= count[lr]) { return; }
     const unsigned id = static_cast<unsigned>(phys[lr * phys_stride + j]);
@@ -112,7 +121,8 @@ __global__ __launch_bounds__(kThreads) void kv_gather_selected_kernel(
     if (off < 0 || region < 0) { return; }
     const uint64_t slot = static_cast<uint64_t>(off) + (static_cast<uint64_t>(l) * 2 + kv) * static_cast<uint64_t>(region) + j;
     if (slot >= staging_blocks) { return; }              // never write outside the staging buffer
-    copy_slice(staging + slot * block_bytes, src, block_bytes);
+    const size_t at = (blockIdx.x - j * pieces) * piece;
+    copy_slice<kT>(staging + slot * block_bytes + at, src + at, min(piece, block_bytes - at));
 }
 
 // Loads planned on the device: slot j of request row `row` receives logical block load_sel[l][row][j] (or
@@ -341,6 +351,33 @@ int stored_layout(const char* name, size_t block_bytes, int rank, int tp_size, S
     return UCM_OK;
 }
 
+// Pieces of a slice, a trip each; a list so long that its pieces would not fit one launch is moved slice by slice.
+struct Pieces {
+    unsigned count;
+    size_t bytes;
+};
+Pieces pieces_of(size_t block_bytes, int n, int threads)
+{
+    const size_t trip = static_cast<size_t>(threads) * 16 * kUnroll, count = (block_bytes + trip - 1) / trip;
+    if (static_cast<uint64_t>(n) * count > 0xffffffffu / static_cast<unsigned>(threads)) { return {1u, block_bytes}; }
+    return {static_cast<unsigned>(count), trip};
+}
+
+template <bool kToStaging>
+int move_blocks(const char* name, const void* const* layers, int n_layers, size_t kv_stride, size_t block_bytes, int num_blocks,
+                const int32_t* block_ids, int n, void* staging, const StoredLayout& lay, ucm_stream_t stream)
+{
+    auto launch = [&](auto kernel, int threads) -> int {
+        const Pieces p = pieces_of(block_bytes, n, threads);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n) * p.count, n_layers, 2), dim3(threads), 0, ucm::as_stream(stream),
+                           const_cast<void* const*>(layers), kv_stride, block_bytes, block_ids, static_cast<unsigned>(num_blocks),
+                           static_cast<uint8_t*>(staging), p.count, p.bytes, lay);
+        return ucm::check_hip(hipGetLastError(), name);
+    };
+    return block_bytes <= kShortSlice ? launch(kv_blocks_kernel<kToStaging, kShortThreads>, kShortThreads)
+                                      : launch(kv_blocks_kernel<kToStaging, kThreads>, kThreads);
+}
+
 // dst row dst_idx[i] = src row src_idx[i]: one 256-thread workgroup per pair (a step's query rows are a few KiB each,
 // so the launch is all latency: every thread has its loads in flight before its first store)
 constexpr int kRowThreads = 256;
@@ -392,11 +429,7 @@ extern "C" int ucm_kv_gather_blocks_tp(const void* const* layers, int n_layers, 
     StoredLayout lay;
     if (int rc = stored_layout("ucm_kv_gather_blocks", block_bytes, rank, tp_size, &lay)) { return rc; }
     if (n == 0) { return UCM_OK; }
-    hipLaunchKernelGGL(kv_blocks_kernel<true>, dim3(static_cast<unsigned>(n), n_layers, 2),
-                       dim3(kThreads), 0, ucm::as_stream(stream), const_cast<void* const*>(layers),
-                       kv_stride, block_bytes, block_ids, static_cast<unsigned>(num_blocks),
-                       static_cast<uint8_t*>(staging), lay);
-    UCM_LAUNCH_CHECK("ucm_kv_gather_blocks");
+    return move_blocks<true>("ucm_kv_gather_blocks", layers, n_layers, kv_stride, block_bytes, num_blocks, block_ids, n, staging, lay, stream);
 }
 
 extern "C" int ucm_kv_gather_blocks(const void* const* layers, int n_layers, size_t kv_stride,
@@ -414,11 +447,7 @@ extern "C" int ucm_kv_scatter_blocks_tp(void* const* layers, int n_layers, size_
     StoredLayout lay;
     if (int rc = stored_layout("ucm_kv_scatter_blocks", block_bytes, rank, tp_size, &lay)) { return rc; }
     if (n == 0) { return UCM_OK; }
-    hipLaunchKernelGGL(kv_blocks_kernel<false>, dim3(static_cast<unsigned>(n), n_layers, 2),
-                       dim3(kThreads), 0, ucm::as_stream(stream), layers, kv_stride, block_bytes,
-                       block_ids, static_cast<unsigned>(num_blocks),
-                       static_cast<uint8_t*>(const_cast<void*>(staging)), lay);
-    UCM_LAUNCH_CHECK("ucm_kv_scatter_blocks");
+    return move_blocks<false>("ucm_kv_scatter_blocks", layers, n_layers, kv_stride, block_bytes, num_blocks, block_ids, n, const_cast<void*>(staging), lay, stream);
 }
 
 extern "C" int ucm_kv_scatter_blocks(void* const* layers, int n_layers, size_t kv_stride,
@@ -446,12 +475,16 @@ extern "C" int ucm_kv_gather_selected(const void* const* layers, int n_layers, s
     UCM_REQUIRE(block_bytes > 0 && block_bytes % 16 == 0 && kv_stride % 16 == 0 && ucm::aligned16(staging),
                 "ucm_kv_gather_selected: sizes and staging must be multiples of 16");
     if (n_req == 0 || max_count == 0) { return UCM_OK; }
-    hipLaunchKernelGGL(kv_gather_selected_kernel,
-                       dim3(static_cast<unsigned>(max_count), n_req, n_layers * 2),
-                       dim3(kThreads), 0, ucm::as_stream(stream), layers, kv_stride, block_bytes, phys,
-                       count, static_cast<unsigned>(num_blocks), static_cast<unsigned>(n_req), static_cast<unsigned>(phys_stride), dst_off,
-                       region_k, static_cast<uint8_t*>(staging), static_cast<uint64_t>(staging_blocks));
-    UCM_LAUNCH_CHECK("ucm_kv_gather_selected");
+    auto launch = [&](auto kernel, int threads) -> int {
+        const Pieces p = pieces_of(block_bytes, max_count, threads);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(max_count) * p.count, n_req, n_layers * 2), dim3(threads), 0,
+                           ucm::as_stream(stream), layers, kv_stride, block_bytes, phys, count, static_cast<unsigned>(num_blocks),
+                           static_cast<unsigned>(n_req), static_cast<unsigned>(phys_stride), dst_off, region_k,
+                           static_cast<uint8_t*>(staging), static_cast<uint64_t>(staging_blocks), p.count, p.bytes);
+        return ucm::check_hip(hipGetLastError(), "ucm_kv_gather_selected");
+    };
+    return block_bytes <= kShortSlice ? launch(kv_gather_selected_kernel<kShortThreads>, kShortThreads)
+                                      : launch(kv_gather_selected_kernel<kThreads>, kThreads);
 }
 
 extern "C" int ucm_kv_load_planned_tp(void* const* layers, int n_layers, size_t kv_stride, size_t block_bytes,
