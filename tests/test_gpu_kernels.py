@@ -611,6 +611,41 @@ def make_caches(dev, n_layers, nb, bb, seed):
     return hs, ds
 
 
+@pytest.mark.parametrize("n", [5, 64, 128, 129, 256, 300, 512, 1000, 1024, 2048, 4096])
+@pytest.mark.parametrize("kind", ["ties", "one value", "extremes", "all largest"])
+def test_topk_windows_of_hard_scores(ucm, dev, n, kind):
+    """Every tier of the selection where the threshold is shared: ties in index order, infinities, zeros of both signs, and
+    NaNs up to the bit patterns whose keys are the smallest and the largest there are; none, one and most picks free."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(n)
+    pool = {"ties": np.array([0.5, -0.5, 1.5, 2.0], np.float32).view(np.uint32),
+            "one value": np.array([0x3f800000], np.uint32),
+            "extremes": np.array([0x7fffffff, 0xffffffff, 0x7f800000, 0xff800000, 0, 0x80000000, 0x3f800000], np.uint32),
+            "all largest": np.array([0x7fffffff], np.uint32)}[kind]
+    raw = rng.choice(pool, n).astype(np.uint32)
+    u = np.where(raw == 0x80000000, 0, raw).astype(np.uint64)
+    key = np.where(u >> 31, 0xffffffff - u, u | 0x80000000)
+    sw, ew = 1, 2
+    ks = [k for k in (sw + ew, sw + ew + 1, n // 3, n - 1) if sw + ew <= k < n]
+    table = rng.permutation(n).astype(np.int32)
+    scores = torch.from_numpy(np.tile(raw.view(np.int32), (len(ks), 1))).to(dev).view(torch.float32).contiguous()
+    idx = torch.full((len(ks), 1, n), -7, dtype=torch.int32, device=dev)
+    phys, cnt = idx.clone(), torch.zeros((len(ks), 1), dtype=torch.int32, device=dev)
+    for l, k in enumerate(ks):
+        one = slice(l, l + 1)
+        ops.topk_windows(scores[one], i32([0], dev), i32([n], dev), i32([k], dev), n, idx[one], cnt[one], start_w=sw, end_w=ew,
+                         block_tables=i32(table[None], dev), phys_out=phys[one])
+    for l, k in enumerate(ks):
+        middle = np.arange(sw, n - ew)
+        best = middle[np.argsort(-key[middle].astype(np.int64), kind="stable")][: k - sw - ew]
+        want = np.sort(np.concatenate([np.arange(sw), best, np.arange(n - ew, n)]))
+        assert int(cnt[l, 0]) == k
+        assert np.array_equal(idx[l, 0, :k].cpu().numpy(), want), (k, kind)
+        assert np.array_equal(phys[l, 0, :k].cpu().numpy(), table[want])
+        assert (idx[l, 0, k:] == -7).all()
+
+
 @pytest.mark.parametrize("bb", [262144, 4096, 48, 16 + 32768])
 def test_kv_dump_load_round_trip(ucm, dev, bb):
     """Config-3 shape in small: random block table, scatter staging->cache, gather cache->staging, byte exact."""

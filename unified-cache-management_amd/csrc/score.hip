@@ -45,6 +45,7 @@ using ucm::u32x4;
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxRow = 16 * 128;  // kv_heads * head_dim: what the staged query row may hold
+constexpr int kStaged = std::max(kMaxRow, ucm::select_scratch(16));   // the staged row's place then serves the selection
 constexpr int kMaxTile = 2048;     // blocks of a workgroup: 128 KiB of the narrowest rows (32 bf16)
 
 template <int kCtrl>
@@ -320,14 +321,17 @@ __device__ __forceinline__ float head_sum(float dot, int first, int step, int kv
     return s;
 }
 
-// The request's selection with the smallest tier of key registers that holds it (the host allows at most 1024 blocks here).
-__device__ __forceinline__ void select_tier(const ucm::SelectArgs& sel, const TileInfo& t, int l, int lane, const float* lds)
+// The request's selection with the smallest tier of key registers that holds it (the host allows at most 1024 blocks here); up to
+// kSoloBlocks by the first wave alone, from there on by all four.  scratch: kStaged words of LDS
+constexpr int kSoloBlocks = 128;
+
+__device__ __forceinline__ void select_tier(const ucm::SelectArgs& sel, const TileInfo& t, int l, unsigned* scratch, const float* lds)
 {
-    if (t.n <= 64) { ucm::select_wave<1, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
-    else if (t.n <= 128) { ucm::select_wave<2, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
-    else if (t.n <= 256) { ucm::select_wave<4, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
-    else if (t.n <= 512) { ucm::select_wave<8, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
-    else { ucm::select_wave<16, false, true>(sel, t.r, l, lane, t.n, t.seg0, t.topk, lds); }
+    if (t.n <= 64) { ucm::select_blocks<1, false, 1, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    else if (t.n <= kSoloBlocks) { ucm::select_blocks<2, false, 1, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    else if (t.n <= 256) { ucm::select_blocks<4, false, kWaves, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    else if (t.n <= 512) { ucm::select_blocks<8, false, kWaves, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    else { ucm::select_blocks<16, false, kWaves, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
 }
 
 // A tile's scores on their way out: collected in LDS and written as whole lines when the tile is done.  (One store per
@@ -336,40 +340,48 @@ __device__ __forceinline__ void select_tier(const ucm::SelectArgs& sel, const Ti
 //
 // With the selection fused in, another workgroup of this launch reads the scores.  One wave then stores them at device scope
 // (write-through: no cache of another part of the chip keeps them back), waits until they have reached memory and takes
-// the request's ticket; the others are done before that.  The workgroup that draws the last ticket resets the counter and
-// its wave runs the request's selection (TopkBlockSelector::TopKImpl, select_topk_block.cpp:20-51) on the scores all of
+// the request's ticket.  The workgroup that draws the last ticket resets the counter and
+// runs the request's selection (TopkBlockSelector::TopKImpl, select_topk_block.cpp:20-51) on the scores all of
 // them wrote, which it reads with device-scope loads after it has seen every other ticket.  (A device-scope
 // release/acquire pair would also do, but it writes the whole L2 back per wave: 7x the kernel's time.)
 __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::SelectArgs& sel, const TileInfo& t, int l, int tile0,
-                                            int n_tile, const float* tile_scores)
+                                            int n_tile, const float* tile_scores, float* qbar)
 {
     float* sout = a.scores + static_cast<int64_t>(l) * a.scores_layer_stride + t.seg0 + tile0;
+    __syncthreads();                                             // the tile's scores are complete, and nobody reads the query any more
     if (!a.tickets) {
-        __syncthreads();
         for (int i = threadIdx.x; i < n_tile; i += kThreads) { sout[i] = tile_scores[i]; }
         return;
     }
-    __syncthreads();
-    if (threadIdx.x >= 64) { return; }                           // the other waves are done: their registers are free again
-    const int lane = threadIdx.x;
     const int tiles = max((t.n + a.tile_blocks - 1) / a.tile_blocks, 1);
-    if (tiles == 1 && t.ok) {                                    // all of the request's scores are here: nobody to wait for
-        for (int i = lane; i < n_tile; i += 64) { sout[i] = tile_scores[i]; }
-        select_tier(sel, t, l, lane, tile_scores);
-        return;
+    const bool alone = tiles == 1 && t.ok;                       // all of the request's scores are here: nobody to wait for
+    const bool solo = t.n <= kSoloBlocks;
+    if (threadIdx.x >= 64 && solo) { return; }
+    bool last = true;
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        if (alone) {
+            for (int i = lane; i < n_tile; i += 64) { sout[i] = tile_scores[i]; }
+        } else {
+            for (int i = lane; i < n_tile; i += 64) {
+                __hip_atomic_store(sout + i, tile_scores[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // (the stores are complete when the wave's memory counter is zero)
+            __builtin_amdgcn_s_waitcnt(0);
+            int32_t* ticket = a.tickets + static_cast<int64_t>(l) * sel.cnt_layer_stride + t.r;
+            int drawn = 0;
+            if (lane == 0) { drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+            last = __builtin_amdgcn_readfirstlane(drawn) == tiles - 1;
+            if (last && lane == 0) { __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+        }
     }
-    for (int i = lane; i < n_tile; i += 64) {
-        __hip_atomic_store(sout + i, tile_scores[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!solo && !alone) {
+        __shared__ int draws_last;
+        if (threadIdx.x == 0) { draws_last = last ? 1 : 0; }
+        __syncthreads();
+        last = __builtin_amdgcn_readfirstlane(draws_last) != 0;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");       // (the stores are complete when the wave's memory counter is zero)
-    __builtin_amdgcn_s_waitcnt(0);
-    int drawn = 0;
-    int32_t* ticket = a.tickets + static_cast<int64_t>(l) * sel.cnt_layer_stride + t.r;
-    if (lane == 0) { drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    drawn = __builtin_amdgcn_readfirstlane(drawn);
-    if (drawn != tiles - 1) { return; }
-    if (lane == 0) { __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    select_tier(sel, t, l, lane, nullptr);
+    if (last) { select_tier(sel, t, l, reinterpret_cast<unsigned*>(qbar), alone ? tile_scores : nullptr); }
 }
 
 // grid: x = layer, y = dense tile index over all requests (workgroups past the
@@ -384,7 +396,7 @@ template <int kD, typename QT>
 __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, const ucm::SelectArgs sel)
 {
     constexpr int kSteps = kD / 16;
-    __shared__ __attribute__((aligned(16))) float qbar[kMaxRow];
+    __shared__ __attribute__((aligned(16))) float qbar[kStaged];
     __shared__ float tile_scores[kMaxTile];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -444,7 +456,7 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
             b0 = b2;
         }
     }
-    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores);
+    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores, qbar);
 }
 
 // ---- bf16 representative table ------------------------------------------------
@@ -498,7 +510,7 @@ __global__ __launch_bounds__(kThreads, kD <= 128 ? 4 : 2) void score_kernel_bf16
     constexpr int kSteps = kD / 16;
     constexpr int kGroup = kSteps % 4 == 0 ? 4 : 2;
     constexpr int kKept = kSteps / 2;
-    __shared__ __attribute__((aligned(16))) float qbar[kMaxRow];
+    __shared__ __attribute__((aligned(16))) float qbar[kStaged];
     __shared__ float tile_scores[kMaxTile];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -559,7 +571,7 @@ __global__ __launch_bounds__(kThreads, kD <= 128 ? 4 : 2) void score_kernel_bf16
             b0 = b2;
         }
     }
-    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores);
+    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores, qbar);
 }
 
 template <int kD, typename QT>

@@ -1,7 +1,7 @@
-// Per-request block selection with forced windows: one 64-wide wavefront per
-// (layer, request); the selection itself is ucm::select_wave (topk_select.h).
+// Per-request block selection with forced windows: one workgroup per
+// (layer, request); the selection itself is ucm::select_blocks (topk_select.h).
 //
-// A few KB in, a few hundred bytes out per wave: this kernel is latency-bound,
+// A few KB in, a few hundred bytes out per workgroup: this kernel is latency-bound,
 // not bandwidth-bound; it only has to stay small next to scoring and gather.
 #include "common.h"
 #include "topk_select.h"
@@ -11,19 +11,22 @@ namespace {
 using ucm::lanes_below;
 using ucm::ordered_key;
 
-// grid: x = request, y = layer; block = one wave
+// grid: x = request, y = layer
 template <int kEpl, bool kHeapTies>
-__global__ __launch_bounds__(64) void topk_windows_kernel(const ucm::SelectArgs a)
+__global__ __launch_bounds__(kEpl > 2 ? 256 : 64) void topk_windows_kernel(const ucm::SelectArgs a)
 {
+    __shared__ unsigned scratch[ucm::select_scratch(kEpl)];
     const int r = blockIdx.x;
-    ucm::select_wave<kEpl, kHeapTies>(a, r, blockIdx.y, threadIdx.x, a.seg_len[r], a.seg_off[r], a.topk_len[r]);
+    const int n = a.seg_len[r], off = a.seg_off[r], k = a.topk_len[r];
+    asm volatile("" ::"s"(n), "s"(off), "s"(k));         // all three on their way at once, not each where it is first looked at
+    ucm::select_blocks<kEpl, kHeapTies, (kEpl > 2 ? 4 : 1)>(a, r, blockIdx.y, n, off, k, scratch);
 }
 
 template <bool kHeapTies>
 void launch_select(const ucm::SelectArgs& a, int max_seg_len, int n_layers, hipStream_t s)
 {
-    const dim3 grid(a.n_req, n_layers), block(64);
-#define UCM_TOPK_LAUNCH(EPL) hipLaunchKernelGGL((topk_windows_kernel<EPL, kHeapTies>), grid, block, 0, s, a)
+    const dim3 grid(a.n_req, n_layers);
+#define UCM_TOPK_LAUNCH(EPL) hipLaunchKernelGGL((topk_windows_kernel<EPL, kHeapTies>), grid, dim3(EPL > 2 ? 256 : 64), 0, s, a)
     // registers per lane for the keys: the smallest tier that holds the longest request (the radix steps cost
     // one ballot per register and bit)
     if (max_seg_len <= 64) { UCM_TOPK_LAUNCH(1); }

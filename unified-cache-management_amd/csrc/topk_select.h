@@ -1,17 +1,26 @@
-// Block selection of one (layer, request) by one 64-wide wavefront: the device
+// Block selection of one (layer, request) by a workgroup of one or four waves: the device
 // function behind ucm_topk_windows / ucm_kvstar_topk (topk.hip) and behind the
 // tail of the fused score + select kernel (score.hip).
 //
-// The request's scores are held in registers as order-preserving 32-bit keys
-// (element i lives in lane i%64, register i/64).  Selection is a radix select,
+// The request's scores become order-preserving 32-bit keys; every wave makes its share of
+// them and leaves them in LDS, and one wave then holds all of them in registers (element i
+// in lane i%64, register i/64).  Selection is a radix select,
 // one bit per step from the top: the threshold T is grown greedily while at
-// least m candidates have key >= T, each count being a wave ballot + popcount.
+// least k keys (the forced blocks' are the largest there are) are >= T, each count being a wave ballot + popcount.
 // Candidates with key > T are all taken; of those with key == T the first
-// `m - count(key > T)` in index order are taken, which is exactly where a
+// `k - count(key > T)` in index order are taken, which is exactly where a
 // stable descending sort leaves equal scores.  Output positions are ballot
 // prefix counts in index order, so the result comes out sorted ascending with
 // no sort at all, and the logical->physical block-table lookup is applied on
 // the way out.
+//
+// What bounds it is latency: a wave alone issues an instruction in about ten cycles, and a chain of scalar results takes longer.
+// So all loads stand together without a branch between them (a branch per register had each wait for the one before: 4700 of
+// the 11 100 cycles of a request of 512 blocks), the compares of a step stand before their counts (42 cycles per register and
+// step one after the other, 26 so), and four waves share the loads and the way out.  Alone, of 256, 512 and 1024 blocks: 3.7,
+// 6.3 and 10.2 us as one wave with a register per 64 blocks throughout, 2.9, 4.1 and 5.0 us.  With the scores: 16 requests of up to
+// 512 blocks 14.2 -> 12.6 us (fp32 table), one of 1024 14.3 -> 10.5, one of 256 8.0.  (Halving an interval between the lanes'
+// maxima instead of going bit by bit takes half the steps, each nearly twice as long, and 1000 cycles to begin with.)
 #pragma once
 
 #include "common.h"
@@ -21,14 +30,33 @@ namespace ucm {
 __device__ __forceinline__ unsigned ordered_key(float f)
 {
     f = f + 0.0f;  // -0.0 -> +0.0, so that the two zeros tie like they do under operator>
-    const unsigned u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+    const int u = __float_as_int(f);
+    return static_cast<unsigned>(u ^ ((u >> 31) | static_cast<int>(0x80000000u)));       // negative: all bits, else the sign bit
 }
 
 __device__ __forceinline__ unsigned lanes_below(unsigned long long mask)
 {
     return __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u));
+}
+
+// How many of the wave's keys are at least c: the compares of up to sixteen registers first, then their counts (one after the
+// other, every count would wait for its own compare).
+template <int kEpl>
+__device__ __forceinline__ int count_at_least(const unsigned (&key)[kEpl], unsigned c)
+{
+    constexpr int kGroup = kEpl < 16 ? kEpl : 16;
+    int cnt = 0;
+#pragma unroll
+    for (int g = 0; g < kEpl; g += kGroup) {
+        unsigned long long m[kGroup];
+#pragma unroll
+        for (int j = 0; j < kGroup; ++j) { m[j] = __ballot(key[g + j] >= c); }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kGroup; ++j) { cnt += __popcll(m[j]); }
+    }
+    return cnt;
 }
 
 // What one selection reads and writes; the same for every (layer, request) of a launch.
@@ -67,7 +95,7 @@ struct SelectArgs {
 // the whole list, the ties kept are the ones of P whose rank among the ties is
 // at least g - g_P.  Windows are not used with it (host checked).
 //
-// Called by all 64 lanes of one wave for request r of layer l; kEpl * 64 is the
+// Called by all threads of a workgroup of kWaves waves (1 or 4) for request r of layer l; kEpl * 64 is the
 // longest request the instance holds (longer ones are cut there: host checked).
 //
 // The request's own descriptors (length, first row, how many to keep) come from the caller, which may have fetched them
@@ -76,10 +104,17 @@ struct SelectArgs {
 // kCoherent: the scores were written by other workgroups of the SAME launch (device-scope stores that went through
 // to memory); they are read with device-scope loads, which do not take a line that an L2 of another part of the
 // chip may still hold in an older state - or they are all in this workgroup's LDS (`lds`, not null).
-template <int kEpl, bool kHeapTies, bool kCoherent = false>
-__device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, int lane, int n, int64_t seg0, int k,
-                                            const float* lds = nullptr)
+//
+// scratch: select_scratch(kEpl) words of LDS that nothing else uses any more.
+constexpr int select_scratch(int epl) { return 2 * 64 * epl + 64; }
+
+template <int kEpl, bool kHeapTies, int kWaves, bool kCoherent = false>
+__device__ __forceinline__ void select_blocks(const SelectArgs& a, int r, int l, int n, int64_t seg0, int k, unsigned* scratch,
+                                              const float* lds = nullptr)
 {
+    constexpr int kThreads = kWaves * 64;
+    constexpr int kPer = kEpl > kWaves ? kEpl / kWaves : 1;      // keys a thread makes
+    const int tid = threadIdx.x, lane = tid & 63;
     const int start_w = a.start_w, end_w = a.end_w, out_stride = a.out_stride;
     const int64_t lr = static_cast<int64_t>(l) * a.cnt_layer_stride + r;
     const int64_t row_at = static_cast<int64_t>(l) * a.idx_layer_stride + static_cast<int64_t>(r) * out_stride;
@@ -97,7 +132,7 @@ __device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, i
         count = 0;
         kept_all = true;                         // nothing to drop: the request keeps its length
     } else if (start_w + end_w >= n || k >= n || k <= 0) {
-        for (int i = lane; i < n; i += 64) {
+        for (int i = tid; i < n; i += kThreads) {
             out[i] = i;
             if (pout) { pout[i] = bt[i]; }
         }
@@ -105,98 +140,172 @@ __device__ __forceinline__ void select_wave(const SelectArgs& a, int r, int l, i
         kept_all = true;
     } else if (k < start_w + end_w) {
         // fewer slots than forced blocks: the first k of [0..start_w) ++ [n-end_w..n)
-        for (int j = lane; j < k; j += 64) {
+        for (int j = tid; j < k; j += kThreads) {
             const int idx = j < start_w ? j : n - end_w + (j - start_w);
             out[j] = idx;
             if (pout) { pout[j] = bt[idx]; }
         }
         count = k;
     } else {
-        const int m = k - start_w - end_w;       // free picks among the middle blocks
         const int hi = n - end_w;                // candidates are start_w <= i < hi
         const float* s = a.scores + static_cast<int64_t>(l) * a.scores_layer_stride + seg0;
-        unsigned key[kEpl];
-        int32_t phys[kEpl];                      // the block table's entries, fetched with the scores: a load per
-#pragma unroll                                   // taken element on the way out would cost a memory round trip per register
-        for (int j = 0; j < kEpl; ++j) {
-            const int i = j * 64 + lane;
-            const bool cand = i >= start_w && i < hi;
-            const int at = cand ? i : 0;
-            float sv;
-            if (kCoherent && lds) { sv = lds[at]; }
-            else if (kCoherent) { sv = __hip_atomic_load(s + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-            else { sv = s[at]; }
-            key[j] = cand ? ordered_key(sv) : 0u;
-            phys[j] = bt ? bt[min(i, n - 1)] : 0;
-        }
-        unsigned T = 0;
-        int need = 0;
-        int tie_lo = 0, tie_hi = 0;              // kHeapTies: ranks (among the ties) that are kept
-        if (m > 0) {
-            for (int bit = 31; bit >= 0; --bit) {
-                const unsigned c = T | (1u << bit);
-                int cnt = 0;
+        // the block table's entries are fetched with the scores; without a table the loads read the row of indices
+        // instead, and nothing uses them
+        const int32_t* table = bt ? bt : out;
+        unsigned *keys = scratch, *phys = scratch + 64 * kEpl;
+        unsigned own_key[kPer], pv[kPer];        // (one wave alone goes on from these, without LDS)
+        if (kEpl >= kWaves || tid < 64 * kEpl) {
+            float sv[kPer];
+            if (kCoherent && lds) {
 #pragma unroll
-                for (int j = 0; j < kEpl; ++j) { cnt += __popcll(__ballot(key[j] >= c)); }
-                if (cnt >= m) { T = c; }
-                // exactly m keys at or above c: they are the selection, and no lower bit can change that
-                if (cnt == m) { T = c - 1u; break; }
+                for (int j = 0; j < kPer; ++j) { sv[j] = lds[min(j * kThreads + tid, n - 1)]; }
+            } else {
+#pragma unroll
+                for (int j = 0; j < kPer; ++j) {
+                    const float* p = s + min(j * kThreads + tid, n - 1);
+                    sv[j] = kCoherent ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
+                }
             }
-            int greater = 0;
 #pragma unroll
-            for (int j = 0; j < kEpl; ++j) { greater += __popcll(__ballot(key[j] > T)); }
-            need = m - greater;
-            if (kHeapTies) {
-                // walk the list in index order up to the k-th block with key >= T
-                int seen = 0, g_p = 0;
+            for (int j = 0; j < kPer; ++j) { pv[j] = static_cast<unsigned>(table[min(j * kThreads + tid, n - 1)]); }
+            asm volatile("" ::: "memory");
 #pragma unroll
-                for (int j = 0; j < kEpl; ++j) {
-                    const unsigned long long ge_mask = __ballot(key[j] >= T && key[j] != 0u);
-                    const unsigned long long gt_mask = __ballot(key[j] > T);
-                    const int c = __popcll(ge_mask);
-                    if (seen < m) {
-                        if (seen + c >= m) {
-                            // lane holding the m-th one: the (m - seen)-th set bit of ge_mask
-                            const bool is_pth = ((ge_mask >> lane) & 1ull) && seen + static_cast<int>(lanes_below(ge_mask)) + 1 == m;
-                            const unsigned long long pm = __ballot(is_pth);
-                            const int p_lane = __ffsll(static_cast<long long>(pm)) - 1;
-                            const unsigned long long upto = p_lane >= 63 ? ~0ull : ((2ull << p_lane) - 1ull);
-                            g_p += __popcll(gt_mask & upto);
-                        } else {
-                            g_p += __popcll(gt_mask);
+            for (int j = 0; j < kPer; ++j) {
+                const int i = j * kThreads + tid;
+                const unsigned forced = i < n ? 0xffffffffu : 0u;        // a forced block's key is above all, a place past the end's below
+                own_key[j] = i >= start_w && i < hi ? ordered_key(sv[j]) : forced;
+                keys[i] = own_key[j];
+                if (kWaves > 1) { phys[i] = pv[j]; }
+            }
+        }
+        // One wave finds the threshold; then up to four write out what is above it, each from its share of the elements (a
+        // register's worth takes a wave 240 cycles, the two barriers 300).
+        constexpr int kOutWaves = kWaves < kEpl ? kWaves : kEpl, kOwn = kEpl / kOutWaves;
+        unsigned* shared = scratch + 2 * 64 * kEpl;      // the threshold, then the waves' counts
+        const int wave = kOutWaves > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
+        if (kWaves > 1) {
+            __syncthreads();
+            if (tid >= kOutWaves * 64) { return; }
+        }
+        unsigned T = 0xffffffffu;
+        if (kOutWaves == 1 || wave == 0) {
+            const int m = k - start_w - end_w;           // free picks among the candidates
+            bool exact = false;
+            if (m > 0) {
+                unsigned key[kEpl];
+#pragma unroll
+                for (int j = 0; j < kEpl; ++j) { key[j] = kWaves == 1 ? own_key[kWaves == 1 ? j : 0] : keys[j * 64 + lane]; }
+                T = 0;
+#pragma unroll 1
+                for (int bit = 31; bit >= 0; --bit) {
+                    const unsigned c = T | (1u << bit);
+                    const int cnt = count_at_least<kEpl>(key, c);
+                    if (cnt >= k) { T = c; }
+                    // exactly k keys at or above c: they are the selection, and no lower bit can change that
+                    if (cnt == k) { exact = true; T = c - 1u; break; }
+                }
+            }
+            if (__builtin_expect(!exact, 0)) {
+                // T is the k-th largest key and others hold the same (or no candidate is to be taken at all): the ones that are kept
+                // get the largest key there is, the others the smallest
+                auto candidate = [&](int j, unsigned& key_j) {
+                    const int i = j * 64 + lane;
+                    key_j = keys[i];
+                    return i >= start_w && i < hi;
+                };
+                unsigned key_j;
+                int greater = 0;
+#pragma unroll 1
+                for (int j = 0; j < kEpl; ++j) { greater += __popcll(__ballot(candidate(j, key_j) && key_j > T)); }
+                int tie_lo = 0, tie_hi = m - greater;    // ranks (among the ties) that are kept
+                if (kHeapTies) {
+                    // walk the list in index order up to the m-th block with key >= T
+                    int seen = 0, g_p = 0;
+#pragma unroll 1
+                    for (int j = 0; j < kEpl; ++j) {
+                        const bool cand = candidate(j, key_j);
+                        const unsigned long long ge_mask = __ballot(cand && key_j >= T && key_j != 0u);
+                        const unsigned long long gt_mask = __ballot(cand && key_j > T);
+                        const int c = __popcll(ge_mask);
+                        if (seen < m) {
+                            if (seen + c >= m) {
+                                // lane holding the m-th one: the (m - seen)-th set bit of ge_mask
+                                const bool is_pth = ((ge_mask >> lane) & 1ull) && seen + static_cast<int>(lanes_below(ge_mask)) + 1 == m;
+                                const unsigned long long pm = __ballot(is_pth);
+                                const int p_lane = __ffsll(static_cast<long long>(pm)) - 1;
+                                const unsigned long long upto = p_lane >= 63 ? ~0ull : ((2ull << p_lane) - 1ull);
+                                g_p += __popcll(gt_mask & upto);
+                            } else {
+                                g_p += __popcll(gt_mask);
+                            }
                         }
+                        seen += c;
                     }
-                    seen += c;
+                    tie_lo = greater - g_p;              // one tie left per block above T that came after P
+                    tie_hi = m - g_p;                    // ties inside P
                 }
-                tie_lo = greater - g_p;          // one tie left per block above T that came after P
-                tie_hi = m - g_p;                // ties inside P
-            }
-        }
-        int pos = 0, ties_seen = 0;
+                int ties_seen = 0;
+#pragma unroll 1
+                for (int j = 0; j < kEpl; ++j) {
+                    const bool eq = candidate(j, key_j) && key_j == T;
+                    const unsigned long long eq_mask = __ballot(eq);
+                    const int rank = ties_seen + static_cast<int>(lanes_below(eq_mask));
+                    if (eq) { keys[j * 64 + lane] = rank >= tie_lo && rank < tie_hi ? 0xffffffffu : 0u; }
+                    ties_seen += __popcll(eq_mask);
+                }
+                T = min(T, 0xfffffffeu);
+                if (kWaves == 1) {
 #pragma unroll
-        for (int j = 0; j < kEpl; ++j) {
-            if (j * 64 < n) {
-                const int i = j * 64 + lane;
-                const bool window = i < n && (i < start_w || i >= hi);
-                const bool cand = i >= start_w && i < hi;
-                const bool gt = cand && m > 0 && key[j] > T;
-                const bool eq = cand && m > 0 && key[j] == T;
-                const unsigned long long eq_mask = __ballot(eq);
-                const int tie_rank = ties_seen + static_cast<int>(lanes_below(eq_mask));
-                const bool take = window || gt || (eq && (kHeapTies ? (tie_rank >= tie_lo && tie_rank < tie_hi) : tie_rank < need));
-                ties_seen += __popcll(eq_mask);
-                const unsigned long long take_mask = __ballot(take);
-                if (take) {
-                    const int p = pos + static_cast<int>(lanes_below(take_mask));
-                    out[p] = i;
-                    if (pout) { pout[p] = phys[j]; }
+                    for (int j = 0; j < kPer; ++j) { own_key[j] = keys[j * 64 + lane]; }
                 }
-                pos += __popcll(take_mask);
+            }
+            if (kOutWaves > 1 && lane == 0) { shared[0] = T; }
+        }
+        if (kOutWaves > 1) {
+            __syncthreads();
+            T = __builtin_amdgcn_readfirstlane(shared[0]);
+        }
+        // (a trip takes up to four registers' worth of elements, whose LDS reads then stand together)
+        static_assert(kWaves > 1 || kEpl <= 4, "one wave alone keeps its keys in registers: one trip");
+        constexpr int kTrip = kOwn < 4 ? kOwn : 4;
+        int mine = 0, pos = 0;
+        if (kOutWaves > 1) {
+#pragma unroll 1
+            for (int j0 = 0; j0 < kOwn; j0 += kTrip) {
+#pragma unroll
+                for (int u = 0; u < kTrip; ++u) { mine += __popcll(__ballot(keys[(wave * kOwn + j0 + u) * 64 + lane] > T)); }
+            }
+            if (lane == 0) { shared[1 + wave] = static_cast<unsigned>(mine); }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < kOutWaves; ++w) {
+                const int c = __builtin_amdgcn_readfirstlane(shared[1 + w]);
+                pos += w < wave ? c : 0;
+                count += c;
             }
         }
-        count = pos;
+#pragma unroll 1
+        for (int j0 = 0; j0 < kOwn; j0 += kTrip) {
+            unsigned key_out[kTrip], phys_out[kTrip];
+#pragma unroll
+            for (int u = 0; u < kTrip; ++u) { key_out[u] = kWaves == 1 ? own_key[kWaves == 1 ? u : 0] : keys[(wave * kOwn + j0 + u) * 64 + lane]; }
+#pragma unroll
+            for (int u = 0; u < kTrip; ++u) { phys_out[u] = kWaves == 1 ? pv[kWaves == 1 ? u : 0] : phys[(wave * kOwn + j0 + u) * 64 + lane]; }
+#pragma unroll
+            for (int u = 0; u < kTrip; ++u) {
+                const bool take = key_out[u] > T;
+                const unsigned long long taken = __ballot(take);
+                if (take) {
+                    const int p = pos + static_cast<int>(lanes_below(taken));
+                    out[p] = (wave * kOwn + j0 + u) * 64 + lane;
+                    if (pout) { pout[p] = static_cast<int32_t>(phys_out[u]); }
+                }
+                pos += __popcll(taken);
+            }
+        }
+        if (kOutWaves == 1) { count = pos; }
     }
-    if (lane == 0) {
+    if (tid == 0) {
         a.count_out[lr] = count;
         if (a.sparse_seq_lens && a.seq_lens) {
             const int len = a.seq_lens[r], rem = len % a.block_size;
