@@ -505,6 +505,29 @@ def test_hash_encode_projections_built_to_cancel(ucm, dev, paired):
     assert np.array_equal(bcodes[0].cpu().numpy(), O.hash_majority(want))
 
 
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (1, 1), (33, 1), (28, 4), (40, 8)])     # rows past a tile's end, groups of 1, 4, 5, 7 and 33
+@pytest.mark.parametrize("paired", ["neighbours", "scattered"])
+def test_hash_query_rows_built_to_cancel(ucm, dev, paired, hq, hkv):
+    """The same vectors as query rows, whose bound is the keys' own: every sign, the +-1 sums and the mean codes are the oracle's."""
+    from ucm_amd import ops
+
+    n_req = max(2, 800 // hq)
+    w_bits, w_f32 = make_weights(884)
+    perm = np.arange(128) if paired == "neighbours" else np.random.default_rng(885).permutation(128)
+    x_bits, _ = cancelling_keys(886 + hq, w_f32, n_req * hq, perm)
+    q_h = x_bits.reshape(1, n_req, hq, 128)
+    q_codes = torch.zeros((1, n_req, hq, 16), dtype=torch.uint8, device=dev)
+    q_sum = torch.zeros((1, n_req, 128), dtype=torch.int16, device=dev)
+    qbar = torch.zeros((1, n_req, hkv, 16), dtype=torch.uint8, device=dev)
+    ops.hash_encode_queries(bf16_dev(q_h, dev), bf16_dev(w_bits, dev), hkv, q_codes, q_sum, qbar, n_req)
+    want = O.hash_encode(q_h[0], w_f32)
+    assert np.array_equal(q_codes[0].cpu().numpy(), want)
+    pm = np.unpackbits(want, axis=-1, bitorder="little").astype(np.int32) * 2 - 1
+    assert np.array_equal(q_sum[0].cpu().numpy(), pm.sum(1))
+    qm = np.stack([O.q_head_mean(synth.bf16_widen(q_h[0][r]), hkv) for r in range(n_req)])
+    assert np.array_equal(qbar[0].cpu().numpy(), O.hash_encode_f32(qm, w_f32))
+
+
 def test_hash_encode_keys_beyond_the_fp32_range(ucm, dev):
     """Keys whose fp32 sums overflow on the way (components up to 3e38: the exact sum may be finite and of either
     sign where the matrix cores hold an infinity or a NaN), keys with infinite components and keys with NaN: the

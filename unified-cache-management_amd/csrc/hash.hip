@@ -43,8 +43,8 @@ constexpr int kBits = 128;          // code length
 constexpr int kWtStride = kDim + 8; // bf16 elements per transposed weight row (272 B: spreads LDS banks)
 constexpr int kQueueCap = 256;
 constexpr int kMaxHeads = 8;
-constexpr float kTau2 = 0x1p-30f;   // (2^-15)^2: the query kernel's bound (three bf16 terms per mean, added afterwards)
-constexpr float kTauBlocks2 = 0x1p-32f;   // (2^-16)^2: the block kernel's bound (one chain of 127 additions per result)
+constexpr float kTau2 = 0x1p-30f;   // (2^-15)^2: the bound for the queries' group means (three bf16 terms per mean, added afterwards)
+constexpr float kTauBlocks2 = 0x1p-32f;   // (2^-16)^2: the bound for keys and query rows (one chain of 127 additions per result)
 
 __device__ __forceinline__ unsigned lanes_below(unsigned long long mask)
 {
@@ -688,8 +688,8 @@ __global__ __launch_bounds__(kEncThreads, 2) void hash_encode_blocks_kernel(
 // A mean is an fp32 number, not a bf16 one: it is cut exactly into three bf16 terms (leading 8 bits, the
 // next 8, the rest), which become rows h, 8+h and 16+h of one more tile; those three rows of a column are
 // registers i, i+4, i+8 of the same lane and are added there.  Only signs are kept, and they must be the
-// signs of the exactly accumulated products: a result whose magnitude is below
-// 2^-15 * (largest ||x|| of the tile) * ||w_col|| - more than the fp32 accumulation can be off by - is redone
+// signs of the exactly accumulated products: a result whose magnitude is below 2^-16 (a mean's: 2^-15)
+// * (largest ||x|| of the tile) * ||w_col|| - more than the fp32 accumulation can be off by - is redone
 // in fp64 (a product of an fp32 and a bf16 value is exact in fp64): a few of them by the whole wave, many by their lanes,
 // d ascending, every lane working on one of its own results at a time.  A tile whose vectors are all tiny (norm below 2^-60, where
 // bf16 subnormals and the bound itself lose bits) is redone whole.  Query rows are the A operand and weights
@@ -791,11 +791,13 @@ __device__ __forceinline__ bool mean_f32_exact_positive(const QueryLds& s, unsig
 
 // The redo of a few results, one after the other, by the whole wave: a lane multiplies two of the 128 dims and the products
 // are added in fp64 in whatever order the lanes combine in.  That order's sum and the oracle's (d ascending) each differ from
-// the exact one by less than 127 * 2^-53 * sum|x_d w_d|, so a sum above 2^-44 * sum|x_d w_d| has the oracle's sign; `settled`
+// the exact one by less than 127 * 2^-53 * sum|x_d w_d|, so a sum above `least`, at least 2^-44 * ||x|| ||w|| (from the bound that
+// made the result doubtful: no second sum over the lanes), has the oracle's sign; `settled`
 // is false for any other (cancelling to the last bits, zero, infinite, NaN), which a lane then redoes in order.
-// One lane alone takes four dependent trips to memory and 128 additions per result, and three waves in four of a
-// step had at least one to wait for: 32 requests x 32 layers x 32 heads took 24.0 us that way, 15.4 this way
-// and 11.3 with the redo left out.
+// One lane alone takes four dependent trips to memory and 128 additions per result, and a wave's redo is what its workgroup
+// ends with: 32 requests x 32 layers x 32 heads take 12.7 us, 10.0 with the redo left out, 21.9 by lanes; 13.9 with twice the
+// bound for the rows, a second sum per redo for its size and a branch around every load of a row or a group's head (1 layer x
+// 32 requests 8.1 -> 7.4, 80 layers x 64 requests x 64 heads 76.7 -> 69.8).
 template <int kCtrl>
 __device__ __forceinline__ double add_dpp(double x)
 {
@@ -823,13 +825,12 @@ __device__ __forceinline__ double wave_sum(double x)
 }
 
 template <bool kF16>
-__device__ __forceinline__ bool wave_positive(float x0, float x1, const unsigned short* w_s, unsigned lane, unsigned col, bool& settled)
+__device__ __forceinline__ bool wave_positive(float x0, float x1, const unsigned short* w_s, unsigned lane, unsigned col, double least, bool& settled)
 {
     const float w0 = widen_lo<kF16>(static_cast<unsigned>(w_s[(2 * lane) * kBits + col]));
     const float w1 = widen_lo<kF16>(static_cast<unsigned>(w_s[(2 * lane + 1) * kBits + col]));
-    const double p0 = static_cast<double>(x0) * static_cast<double>(w0), p1 = static_cast<double>(x1) * static_cast<double>(w1);
-    const double sum = wave_sum(p0 + p1), size = wave_sum(__builtin_fabs(p0) + __builtin_fabs(p1));
-    settled = __builtin_fabs(sum) > 0x1p-44 * size && size < __builtin_inf();
+    const double sum = wave_sum(static_cast<double>(x0) * static_cast<double>(w0) + static_cast<double>(x1) * static_cast<double>(w1));
+    settled = __builtin_fabs(sum) > least;               // (not for a bound that is infinite or NaN)
     return sum > 0.0;
 }
 
@@ -870,14 +871,23 @@ __global__ __launch_bounds__(kQueryThreads, 4) void hash_query_kernel(
         float nx2 = 0.0f;
         if (h < kv_heads) {
             const unsigned short* first = qp + (h * g) * kDim + 8 * piece;
+            // four heads of the group per trip to memory (past the last one the last one again), added in order
             float x[8];
-            widen8<kF16>(ucm::gload16(first), x);
-#pragma unroll 4
-            for (unsigned rr = 1; rr < g; ++rr) {
-                float y[8];
-                widen8<kF16>(ucm::gload16(first + rr * kDim), y);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) { x[j] = x[j] + y[j]; }
+            for (int j = 0; j < 8; ++j) { x[j] = -0.0f; }        // -0 + x == x for every x, signed zeros included
+            for (unsigned r0 = 0; r0 < g; r0 += 4) {
+                u32x4 v[4];
+#pragma unroll
+                for (unsigned u = 0; u < 4; ++u) { v[u] = ucm::gload16(first + min(r0 + u, g - 1) * kDim); }
+#pragma unroll
+                for (unsigned u = 0; u < 4; ++u) {
+                    if (r0 + u < g) {                        // (uniform)
+                        float y[8];
+                        widen8<kF16>(v[u], y);
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) { x[j] = x[j] + y[j]; }
+                    }
+                }
             }
             unsigned term[3][8];
             float xmean[8];
@@ -942,19 +952,20 @@ __global__ __launch_bounds__(kQueryThreads, 4) void hash_query_kernel(
     // ---- the query rows, 32 per tile
     int sum = 0;
     for (unsigned t0 = 0; t0 < q_heads; t0 += 32) {
-        const unsigned m_in = t0 + lr32;                 // the row this lane feeds
+        // This lane feeds row t0 + lr32 (past the last one the last one again, whose results nothing looks at).  The loads are
+        // unconditional and stand together: a branch around each had it wait for the one before.
+        const unsigned short* row = qp + min(t0 + lr32, q_heads - 1) * kDim + 8 * half;
         u32x4 xa[8];
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) { xa[ks] = ucm::gload16(row + 16 * ks); }
+        asm volatile("" ::: "memory");
         float nx2 = 0.0f;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            if (m_in < q_heads) { xa[ks] = ucm::gload16(qp + m_in * kDim + 16 * ks + 8 * half); }
-            else { xa[ks] = u32x4{0u, 0u, 0u, 0u}; }
-            nx2 = norm2_acc<kF16>(xa[ks], nx2);
-        }
+        for (int ks = 0; ks < 8; ++ks) { nx2 = norm2_acc<kF16>(xa[ks], nx2); }
         nx2 += __shfl_xor(nx2, 32, 64);
         const float max2 = wave_max32(nx2);
         const bool all_exact = (max2 > 0.0f && !(max2 >= 0x1p-120f)) || !(max2 < __builtin_inff());   // tiny norms, or none that is finite
-        const float bound = sqrtf(kTau2 * max2) * sqrtf(nw2) * 1.01f;
+        const float bound = sqrtf(kTauBlocks2 * max2) * sqrtf(nw2) * 1.01f;
         f32x16 acc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) { acc[i] = 0.0f; }
@@ -976,7 +987,8 @@ __global__ __launch_bounds__(kQueryThreads, 4) void hash_query_kernel(
             const unsigned m = t0 + 8 * (i >> 2) + 4 * (src >> 5) + (i & 3);
             const unsigned x = *reinterpret_cast<const unsigned*>(qp + m * kDim + 2 * lane);
             bool settled;
-            const bool pos = wave_positive<kF16>(widen_lo<kF16>(x), widen_hi<kF16>(x), s.w, lane, wave * 32 + (src & 31), settled);
+            const double least = static_cast<double>(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bound), src))) * 0x1p-28;
+            const bool pos = wave_positive<kF16>(widen_lo<kF16>(x), widen_hi<kF16>(x), s.w, lane, wave * 32 + (src & 31), least, settled);
             if (!settled) { break; }
             if (lane == src) {
                 redo &= redo - 1;
@@ -1049,7 +1061,8 @@ __global__ __launch_bounds__(kQueryThreads, 4) void hash_query_kernel(
             const float x0 = (widen_lo<kF16>(term[0]) + widen_lo<kF16>(term[1])) + widen_lo<kF16>(term[2]);
             const float x1 = (widen_hi<kF16>(term[0]) + widen_hi<kF16>(term[1])) + widen_hi<kF16>(term[2]);
             bool settled;
-            const bool pos = wave_positive<kF16>(x0, x1, s.w, lane, wave * 32 + (src & 31), settled);
+            const double least = static_cast<double>(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bound), src))) * 0x1p-29;
+            const bool pos = wave_positive<kF16>(x0, x1, s.w, lane, wave * 32 + (src & 31), least, settled);
             if (!settled) { break; }
             if (lane == src) {
                 redo &= redo - 1;
