@@ -832,6 +832,13 @@ def test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_
         assert torch.equal(caches[l], want), l
 
 
+@pytest.mark.parametrize("n_layers,rows_n,n_slots,bb", [(32, 32, 2, 8192 + 16), (25, 41, 3, 16384), (40, 41, 2, 8192 + 16),   # a pair a thread, or four
+                                                        (3, 5, 40, 3 * 131072 + 16), (2, 7, 6, 8192)])
+def test_counted_loads_of_many_rows_and_long_slices(ucm, dev, n_layers, rows_n, n_slots, bb):
+    """Running totals of 1024 pairs and more, slices of several pieces each, and the short slices that go by slot instead."""
+    test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_slots, bb, True)
+
+
 def test_copy_batch_pointer_arrays(ucm, dev):
     from ucm_amd import ops
 

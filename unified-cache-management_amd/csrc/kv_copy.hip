@@ -29,14 +29,19 @@ constexpr size_t kShortSlice = 8 * 1024;
 // kN x 16 KiB of a slice: every load is issued before the first store goes out.  Stores that start as the
 // loads trickle in mix reads and writes on the HBM channels and cost about 6 % of the copy rate (1.64 ms ->
 // 1.75 ms for the 5.1 GB gather), hence the wait for ALL of the trip's loads.
-template <int kN, int kT = kThreads>
-__device__ __forceinline__ void copy_trip(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t base)
+// (`meanwhile` runs while the loads are on their way.)
+struct Nothing { __device__ __forceinline__ void operator()() const {} };
+
+template <int kN, int kT = kThreads, typename F = Nothing>
+__device__ __forceinline__ void copy_trip(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t base, F meanwhile = F())
 {
     u32x4 v[kN];
 #pragma unroll
     for (int u = 0; u < kN; ++u) {
         v[u] = ucm::gload16_nt(src + base + static_cast<size_t>(u) * kT * 16);
     }
+    asm volatile("" ::: "memory");
+    meanwhile();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int u = 0; u < kN; ++u) {
@@ -263,20 +268,21 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
     __shared__ unsigned s_part[kThreads / 64];
     const unsigned pairs = n_layers * batch;             // pair p = layer p / batch, request p % batch
     constexpr unsigned kPer = kMaxPlannedPairs / kThreads;
+    // (A thread takes one pair, and four only if there are more pairs than threads; loads of pairs that do not exist read the last
+    // one's.  With four in a row each waited for two trips to memory of its own before the first piece was copied.)
+    const unsigned per = pairs <= kThreads ? 1u : kPer;
     unsigned mine[kPer], sum = 0;
 #pragma unroll
     for (unsigned i = 0; i < kPer; ++i) {
-        const unsigned p = threadIdx.x * kPer + i;
-        unsigned c = 0;
-        if (p < pairs) {
-            const unsigned l = p / batch, b = p - l * batch;
-            const int32_t r = rows ? rows[b] : static_cast<int32_t>(b);
-            if (r >= 0 && static_cast<unsigned>(r) < table_rows) {
-                c = min(n_slots, static_cast<unsigned>(max(load_count[static_cast<size_t>(l) * table_rows + r], 0)));
-            }
-        }
-        mine[i] = c;
-        sum += c;
+        mine[i] = 0;
+        if (i >= per) { break; }                         // (uniform)
+        const unsigned p = threadIdx.x * per + i, pc = min(p, pairs - 1);
+        const unsigned l = pc / batch, b = pc - l * batch;
+        const int32_t r = rows ? rows[b] : static_cast<int32_t>(b);
+        const bool live = r >= 0 && static_cast<unsigned>(r) < table_rows;
+        const int32_t c = load_count[static_cast<size_t>(l) * table_rows + (live ? r : 0)];
+        if (p < pairs && live) { mine[i] = min(n_slots, static_cast<unsigned>(max(c, 0))); }
+        sum += mine[i];
     }
     // running total of the threads' sums: inside a wave, then over the waves before it
     unsigned incl = sum;
@@ -291,7 +297,8 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
     for (unsigned w = 0; w < kThreads / 64; ++w) { run += w < threadIdx.x >> 6 ? s_part[w] : 0u; }
 #pragma unroll
     for (unsigned i = 0; i < kPer; ++i) {
-        s_total[threadIdx.x * kPer + i] = run;
+        if (i >= per) { break; }
+        s_total[threadIdx.x * per + i] = run;
         run += mine[i];
     }
     if (threadIdx.x == kThreads - 1) { s_total[kMaxPlannedPairs] = run; }
@@ -303,14 +310,15 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
     const unsigned pieces = kWhole ? 1u : static_cast<unsigned>((block_bytes + kLoadPiece - 1) / kLoadPiece);
     const unsigned w_step = gridDim.x / pieces, p_step = gridDim.x % pieces;
     // Pieces of 32 KiB and more: the waves start each one together, so that their reads and writes reach HBM in turns (8 layers x 16
-    // x 14 loads of 256 KiB 336 -> 318 us, 8 x 32 x 14 of 64 KiB 178 -> 170; of 8 KiB 35.3 -> 37.4).
-    const bool in_step = block_bytes >= 32 * 1024;
-    unsigned p = blockIdx.x % pieces;
-    for (unsigned w = blockIdx.x / pieces; w < slices; w += w_step, p += p_step) {   // (uniform in the workgroup)
-        if (!kWhole && p >= pieces) {
-            p -= pieces;
-            if (++w >= slices) { break; }
-        }
+    // x 14 loads of 256 KiB 336 -> 325 us, 8 x 32 x 14 of 64 KiB 178 -> 170; of 8 KiB 35.3 -> 37.4).
+    const bool in_step = !kWhole || block_bytes >= 32 * 1024;
+    // The cache and pool address of piece p of slice w, and its size; dst null: nothing to copy
+    struct Piece {
+        const uint8_t* src;
+        uint8_t* dst;
+        size_t size;
+    };
+    auto find = [&](unsigned w, unsigned p) -> Piece {
         const unsigned t = w >> 1, kv = w & 1u;
         const size_t off = kWhole ? 0 : static_cast<size_t>(p) * kLoadPiece;
         unsigned lo = 0, hi = pairs;                     // last pair whose running total is <= t
@@ -321,15 +329,47 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
         const unsigned l = lo / batch, b = lo - l * batch, j = t - s_total[lo];
         const unsigned row = static_cast<unsigned>(rows ? rows[b] : static_cast<int32_t>(b));
         const int32_t sel = load_sel[(static_cast<size_t>(l) * table_rows + row) * n_slots + j];
-        if (sel < 0 || static_cast<unsigned>(sel) >= src_stride) { continue; }
+        if (sel < 0 || static_cast<unsigned>(sel) >= src_stride) { return {nullptr, nullptr, 0}; }
         const int32_t src = src_table[static_cast<size_t>(row) * src_stride + sel];
-        if (src < 0 || static_cast<uint64_t>(src) >= pool_blocks) { continue; }
+        if (src < 0 || static_cast<uint64_t>(src) >= pool_blocks) { return {nullptr, nullptr, 0}; }
         const unsigned dst = static_cast<unsigned>(dst_table[l * dst_layer_stride + static_cast<int64_t>(row) * dst_stride + j]);
-        if (dst >= num_blocks) { continue; }
-        if (in_step) { __syncthreads(); }                // (uniform)
-        copy_slice(static_cast<uint8_t*>(layers[l]) + kv * kv_stride + static_cast<size_t>(dst) * block_bytes + off,
-                   pool + static_cast<size_t>(src) * pool_block_bytes + lay.slice(store_first_layer + l, kv, block_bytes) + off,
-                   kWhole ? block_bytes : min(kLoadPiece, block_bytes - off));
+        if (dst >= num_blocks) { return {nullptr, nullptr, 0}; }
+        return {pool + static_cast<size_t>(src) * pool_block_bytes + lay.slice(store_first_layer + l, kv, block_bytes) + off,
+                static_cast<uint8_t*>(layers[l]) + kv * kv_stride + static_cast<size_t>(dst) * block_bytes + off,
+                kWhole ? block_bytes : min(kLoadPiece, block_bytes - off)};
+    };
+    unsigned p = blockIdx.x % pieces, w = blockIdx.x / pieces;
+    if constexpr (kWhole) {
+        for (; w < slices; w += w_step) {                // (uniform in the workgroup)
+            const Piece cur = find(w, 0);
+            if (!cur.dst) { continue; }
+            if (in_step) { __syncthreads(); }
+            copy_slice(cur.dst, cur.src, cur.size);
+        }
+    } else {
+        // Where the next piece lies is found while this one's loads are on their way (8 layers x 16 x 14 loads of 256 KiB 325 -> 307 us;
+        // short slices, which are copied in less time than it takes to find the next, only lose by it).
+        if (w >= slices) { return; }
+        Piece cur = find(w, p), next = {nullptr, nullptr, 0};
+        for (;;) {
+            w += w_step;
+            p += p_step;
+            if (p >= pieces) {
+                p -= pieces;
+                ++w;
+            }
+            const bool more = w < slices;
+            auto look_ahead = [&]() { if (more) { next = find(w, p); } };
+            __syncthreads();
+            if (cur.dst && cur.size == kStep) {
+                copy_trip<kUnroll>(cur.dst, cur.src, threadIdx.x * 16u, look_ahead);
+            } else {
+                if (cur.dst) { copy_slice(cur.dst, cur.src, cur.size); }
+                look_ahead();
+            }
+            if (!more) { break; }
+            cur = next;
+        }
     }
 }
 
