@@ -384,6 +384,42 @@ def test_hash_query_rows_outside_the_layer_are_skipped(ucm, dev):
                 assert (q_codes[l, r] == 0xEE).all() and (q_sum[l, r] == 77).all() and (qbar[l, r] == 0xEE).all(), (l, r)
 
 
+@pytest.mark.parametrize("n_req", [1, 2, 3, 63, 64, 65, 130])
+@pytest.mark.parametrize("hkv", [1, 3, 8])
+def test_hash_scores_of_many_requests(ucm, dev, n_req, hkv):
+    """The search for a block's request: trips of 64 requests, requests without blocks, of one, of more than a workgroup's
+    sixteen, and some outside the tables, which count none."""
+    from ucm_amd import ops
+
+    n_layers, rows = 2, 700
+    rng = np.random.default_rng(830 + n_req)
+    lens = rng.choice([0, 1, 2, 3, 5, 17, 40], n_req).astype(np.int32)
+    lens[-1] = 19
+    off = rng.integers(0, rows - 40, n_req).astype(np.int32)
+    if n_req > 2:
+        lens[:2] = 0, -4
+        off[2], lens[2] = rows - 3, 4
+    if n_req > 64:
+        off[63], off[64], lens[63:65] = -1, rows - 40, 40
+    inside = [max(int(n), 0) if o >= 0 and o + max(int(n), 0) <= rows else 0 for o, n in zip(off, lens)]
+    colsum = rng.integers(-128, 129, (n_layers, rows, hkv, 128)).astype(np.int16)
+    q_sum = rng.integers(-32, 33, (n_layers, n_req, 128)).astype(np.int16)
+    codes = torch.zeros((n_layers, rows, hkv, 16), dtype=torch.uint8, device=dev)
+    qbar = torch.zeros((n_layers, n_req, hkv, 16), dtype=torch.uint8, device=dev)
+    # where requests share rows the last writer is not defined: rows of one request only are compared
+    owners = np.zeros(rows, np.int64)
+    want = np.full((n_layers, rows), -1.0, np.float32)
+    for r, n in enumerate(inside):
+        owners[off[r] : off[r] + n] += 1
+        for l in range(n_layers):
+            want[l, off[r] : off[r] + n] = colsum[l, off[r] : off[r] + n].astype(np.int64).sum(1) @ q_sum[l, r].astype(np.int64)
+    scores = torch.full((n_layers, rows), -1.0, device=dev)
+    ops.hash_score_blocks(ops.HASH_SCORE_SUM, torch.from_numpy(q_sum).to(dev), qbar, torch.from_numpy(colsum).to(dev), codes,
+                          i32(off, dev), i32(lens, dev), max(sum(inside), 1), scores)
+    got = scores.cpu().numpy()
+    assert np.array_equal(got[:, owners <= 1], want[:, owners <= 1])
+
+
 def test_hash_queries_scores_and_selection(ucm, dev):
     """Config-5 shape in small: ragged batch, 8 kv heads, 32 query heads, 2 layers."""
     from ucm_amd import ops

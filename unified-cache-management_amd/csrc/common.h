@@ -41,6 +41,17 @@ __device__ __forceinline__ void gstore16_nt(void* p, const u32x4 v)
 {
     __builtin_nontemporal_store(v, (UCM_GLOBAL u32x4*)p);
 }
+// Inclusive sum over the wave's lanes: within rows of sixteen, then from row to row.
+__device__ __forceinline__ int inclusive_scan(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+    return x;
+}
 }  // namespace ucm
 
 #define UCM_REQUIRE(cond, ...)                                   \

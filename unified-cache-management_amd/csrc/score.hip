@@ -191,18 +191,6 @@ __device__ __forceinline__ float quad_dot(const f32x4 (&qr)[kSteps], u32x4 (&kv)
     return (a0 + a2) + (a1 + a3);
 }
 
-// Inclusive sum over the wave's lanes: within rows of sixteen, then from row to row.
-__device__ __forceinline__ int inclusive_scan(int x)
-{
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-    return x;
-}
-
 // Finds the request that owns dense tile index `w` (tiles of all requests laid
 // end to end, request r contributing ceil(seg_len[r] / tile_blocks) of them).
 // Every wave does this on its own: 64 requests per trip, an inclusive wave scan
@@ -228,7 +216,7 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ seg_len, c
         const int qr = live && q_rows ? q_rows[r] : r;
         const int top = live && topk_len ? topk_len[r] : 0;
         const int t = live ? max((len + tile_blocks - 1) / tile_blocks, min_tiles) : 0;
-        const int incl = inclusive_scan(t);
+        const int incl = ucm::inclusive_scan(t);
         const unsigned long long owner = __ballot(w < base + incl);
         if (owner) {
             const int src = __builtin_ctzll(owner);
