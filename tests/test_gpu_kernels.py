@@ -1129,6 +1129,34 @@ def test_delta_plan_slot_counts(ucm, dev, n_slots):
         assert np.array_equal(resident.cpu().numpy(), res_h), step
 
 
+@pytest.mark.parametrize("n_layers,n_req", [(64, 8), (57, 9)])
+@pytest.mark.parametrize("n_slots", [65, 256, 257, 530])
+def test_delta_plan_on_both_sides_of_the_thread_split(ucm, dev, n_layers, n_req, n_slots):
+    """512 rows (four threads per entry) and 513 (one), with slots that hold a block twice or nothing: the last slot of a
+    block wins, and loads, slots, resident sets and counts equal the oracle's."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(n_slots + n_req)
+    sel = np.stack([rng.permutation(2 * n_slots)[: n_slots + 3] for _ in range(n_layers * n_req)]).astype(np.int32)
+    sel = sel.reshape(n_layers, n_req, -1)
+    cnt = rng.integers(0, n_slots + 4, (n_layers, n_req)).astype(np.int32)
+    cnt[0, 0], cnt[-1, -1] = 0, n_slots
+    res_h = rng.integers(-1, 2 * n_slots, (n_layers, n_req, n_slots)).astype(np.int32)
+    resident, phys = i32(res_h, dev), sel + 7
+    load = torch.full((n_layers, n_req, n_slots), -7, dtype=torch.int32, device=dev)
+    slot_of, miss = i32(np.full_like(sel, -7), dev), i32(np.full_like(cnt, -7), dev)
+    ops.delta_plan(i32(sel, dev), i32(phys, dev), i32(cnt, dev), resident, load, slot_of, miss)
+    load_h, slot_h, miss_h = load.cpu().numpy(), slot_of.cpu().numpy(), miss.cpu().numpy()
+    for l in range(n_layers):
+        for r in range(n_req):
+            c = int(cnt[l, r])
+            wl, ws, moved = O.delta_plan(sel[l, r, :c], phys[l, r, :c], res_h[l, r])
+            k = min(c, n_slots)
+            assert np.array_equal(load_h[l, r], wl) and miss_h[l, r] == moved, (l, r)
+            assert np.array_equal(slot_h[l, r, :k], ws[:k]) and np.all(slot_h[l, r, k:] == -7), (l, r)
+    assert np.array_equal(resident.cpu().numpy(), res_h)
+
+
 def test_decode_step_under_graph_capture(ucm, dev):
     """The step's three launches (scores, selection + block table, gather) allocate and synchronise nothing, so a
     caller may capture them in a HIP graph: three replays with fresh queries, eager work and synchronisation in

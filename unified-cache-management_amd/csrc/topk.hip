@@ -206,23 +206,23 @@ __global__ __launch_bounds__(64) void delta_plan_kernel(
     if (lane == 0) { miss_count[lr] = n_move; }
 }
 
-// More than 64 slots: one 256-thread workgroup per (layer, request), entry
-// e*256 + thread in register e.  Both lists sit in LDS and every thread walks
-// the other list four entries per read (all threads read the same address, a
-// broadcast); ranks are ballot prefix counts plus the counts of the (register,
-// wave) groups before the thread's own, so the pairing is the same as above.
+// More than 64 slots: one workgroup per (layer, request), entry e*256 + tid in register e of the kSub threads that share
+// it.  Both lists sit in LDS and a thread walks its share of the other list, every kSub-th run of sixteen entries; ranks are
+// ballot prefix counts plus the counts of the (register, wave) groups before the thread's own, so the pairing is the same
+// as above.  What bounds it is the walk, entries x entries / 256 compares per thread and an LDS latency per run, so few
+// workgroups have four threads per entry: 16 requests of 153, 256, 400 and 1000 slots 7.1, 9.6, 21.3 and 88 us by one thread,
+// 5.0, 5.9, 12.6 and 47 by four; 1 of 65 slots 4.0 and 3.4.
 constexpr int kPlanThreads = 256;
-constexpr int kPlanWaves = kPlanThreads / 64;
 
-template <int E>  // entries per thread: n_slots <= 256 * E
-__global__ __launch_bounds__(kPlanThreads) void delta_plan_wide_kernel(
+template <int E, int kSub>  // entries per thread: n_slots <= 256 * E; threads per entry
+__global__ __launch_bounds__(kPlanThreads * kSub) void delta_plan_wide_kernel(
     const int32_t* __restrict__ sel, const int32_t* __restrict__ sel_phys, const int32_t* __restrict__ count,
     int n_req, int sel_stride, int32_t* __restrict__ resident, int n_slots, int32_t* __restrict__ load_phys,
     int32_t* __restrict__ slot_of_sel, int32_t* __restrict__ miss_count, const int32_t* __restrict__ rows)
 {
-    constexpr int kCap = kPlanThreads * E;
-    const int l = blockIdx.y, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    constexpr int kCap = kPlanThreads * E, kPlanWaves = kPlanThreads * kSub / 64;
+    const int l = blockIdx.y, tid = threadIdx.x / kSub, sub = threadIdx.x % kSub;   // (tid: the thread's entry)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int r = blockIdx.x;
     if (rows) {
         r = rows[r];
@@ -255,9 +255,8 @@ __global__ __launch_bounds__(kPlanThreads) void delta_plan_wide_kernel(
 #pragma unroll
     for (int e = 0; e < E; ++e) { hit_slot[e] = -1; keep[e] = false; }
     // sixteen entries per trip, their reads issued together (past the lists the arrays hold -1): a trip of four is one
-    // LDS latency long, and a budget of 153 slots walks two lists of them
-    // (16 requests: 8.8 us that way, 7.3 this way)
-    for (int i0 = 0; i0 < n_slots; i0 += 16) {
+    // LDS latency long (one thread per entry, 16 requests of 153 slots: 8.8 us that way, 7.1 this way)
+    for (int i0 = sub * 16; i0 < n_slots; i0 += 16 * kSub) {
         int4 v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) { v[u] = *reinterpret_cast<const int4*>(&s_res[i0 + u * 4]); }
@@ -274,7 +273,7 @@ __global__ __launch_bounds__(kPlanThreads) void delta_plan_wide_kernel(
             }
         }
     }
-    for (int i0 = 0; i0 < k; i0 += 16) {
+    for (int i0 = sub * 16; i0 < k; i0 += 16 * kSub) {
         int4 v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) { v[u] = *reinterpret_cast<const int4*>(&s_sel[i0 + u * 4]); }
@@ -287,15 +286,25 @@ __global__ __launch_bounds__(kPlanThreads) void delta_plan_wide_kernel(
         }
     }
 #pragma unroll
-    for (int e = 0; e < E; ++e) { keep[e] = keep[e] && my_res[e] >= 0; }
+    for (int e = 0; e < E; ++e) {
+        if (kSub == 4) {   // the four threads' parts of the lists: the highest slot, and whether any of them holds the block
+            int kept = keep[e];
+            hit_slot[e] = max(hit_slot[e], __builtin_amdgcn_mov_dpp(hit_slot[e], 0xb1, 0xf, 0xf, true));   // quad_perm 1,0,3,2
+            hit_slot[e] = max(hit_slot[e], __builtin_amdgcn_mov_dpp(hit_slot[e], 0x4e, 0xf, 0xf, true));   // quad_perm 2,3,0,1
+            kept |= __builtin_amdgcn_mov_dpp(kept, 0xb1, 0xf, 0xf, true);
+            kept |= __builtin_amdgcn_mov_dpp(kept, 0x4e, 0xf, 0xf, true);
+            keep[e] = kept != 0;
+        }
+        keep[e] = keep[e] && my_res[e] >= 0;
+    }
 
     bool miss[E], freed[E];
     int miss_rank[E], free_rank[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int i = e * kPlanThreads + tid;
-        miss[e] = i < k && hit_slot[e] < 0;
-        freed[e] = i < n_slots && !keep[e];
+        miss[e] = sub == 0 && i < k && hit_slot[e] < 0;
+        freed[e] = sub == 0 && i < n_slots && !keep[e];
         const unsigned long long mm = __ballot(miss[e]), fm = __ballot(freed[e]);
         miss_rank[e] = static_cast<int>(lanes_below(mm));
         free_rank[e] = static_cast<int>(lanes_below(fm));
@@ -326,14 +335,14 @@ __global__ __launch_bounds__(kPlanThreads) void delta_plan_wide_kernel(
         int dst_slot = hit_slot[e], take_sel = -1, take_phys = -1;
         if (freed[e] && free_rank[e] < n_move) { take_sel = s_a[free_rank[e]]; take_phys = s_b[free_rank[e]]; }
         if (miss[e] && miss_rank[e] < n_move) { dst_slot = s_c[miss_rank[e]]; }
-        if (i < n_slots) {
+        if (sub == 0 && i < n_slots) {
             load_phys[lr * n_slots + i] = take_phys;
             if (take_sel >= 0) { res[i] = take_sel; }
             else if (freed[e]) { res[i] = -1; }
         }
-        if (i < k) { slot_of_sel[lr * sel_stride + i] = dst_slot; }
+        if (sub == 0 && i < k) { slot_of_sel[lr * sel_stride + i] = dst_slot; }
     }
-    if (tid == 0) { miss_count[lr] = n_move; }
+    if (threadIdx.x == 0) { miss_count[lr] = n_move; }
 }
 
 }  // namespace
@@ -346,16 +355,24 @@ int delta_plan_launch(const char* name, const int32_t* sel, const int32_t* sel_p
 {
     const dim3 grid(n_launch, n_layers);
     hipStream_t s = ucm::as_stream(stream);
-#define UCM_PLAN_LAUNCH(E)                                                                                    \
-    hipLaunchKernelGGL(delta_plan_wide_kernel<E>, grid, dim3(kPlanThreads), 0, s, sel, sel_phys, count, n_rows, \
+#define UCM_PLAN_LAUNCH(E, SUB)                                                                               \
+    hipLaunchKernelGGL((delta_plan_wide_kernel<E, SUB>), grid, dim3(kPlanThreads * SUB), 0, s, sel, sel_phys, count, n_rows, \
                        sel_stride, resident, n_slots, load_phys, slot_of_sel, miss_count, rows)
+#define UCM_PLAN_WIDE(E)                        \
+    if (split) { UCM_PLAN_LAUNCH(E, 4); }       \
+    else { UCM_PLAN_LAUNCH(E, 1); }
+    // Four threads per entry while all their workgroups of sixteen waves are resident at once, two per compute unit: 512
+    // of 153 / 256 / 400 / 1000 slots 7.7 / 9.4 / 24.4 / 101 us (by one thread 7.9 / 10.6 / 25.2 / 106), but 1024 of 200 slots
+    // 13.6 (11.3).
+    const bool split = static_cast<uint64_t>(n_launch) * n_layers <= 512;
     if (n_slots <= 64) {
         hipLaunchKernelGGL(delta_plan_kernel, grid, dim3(64), 0, s, sel, sel_phys, count, n_rows, sel_stride, resident,
                            n_slots, load_phys, slot_of_sel, miss_count, rows);
     }
-    else if (n_slots <= 256) { UCM_PLAN_LAUNCH(1); }
-    else if (n_slots <= 512) { UCM_PLAN_LAUNCH(2); }
-    else { UCM_PLAN_LAUNCH(4); }
+    else if (n_slots <= 256) { UCM_PLAN_WIDE(1); }
+    else if (n_slots <= 512) { UCM_PLAN_WIDE(2); }
+    else { UCM_PLAN_WIDE(4); }
+#undef UCM_PLAN_WIDE
 #undef UCM_PLAN_LAUNCH
     return ucm::check_hip(hipGetLastError(), name);
 }
