@@ -564,6 +564,35 @@ def test_hash_query_rows_built_to_cancel(ucm, dev, paired, hq, hkv):
     assert np.array_equal(qbar[0].cpu().numpy(), O.hash_encode_f32(qm, w_f32))
 
 
+@pytest.mark.parametrize("exponent", [-62, -61, -60, -59, -58, -57, -56, -55])
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (8, 8)])                                  # (8, 8): a row is its group's mean as well
+def test_hash_query_rows_of_small_norm(ucm, dev, exponent, hq, hkv):
+    """Cancelling rows whose norms all lie in [2^exponent, 2^(exponent+1)), to either side of 2^-60, below which a tile is redone
+    whole: above it the bound that finds the doubtful results must not vanish in fp32."""
+    from ucm_amd import ops
+
+    n_req = 1600 // hq
+    w_bits, w_f32 = make_weights(884)
+    x_bits, _ = cancelling_keys(7700 + hq, w_f32, n_req * hq, np.random.default_rng(7701).permutation(128))
+    x = synth.bf16_widen(x_bits).astype(np.float64)
+    norm = np.sqrt((x * x).sum(1, keepdims=True))
+    q_f32 = (x * 2.0 ** (exponent - np.floor(np.log2(norm)))).astype(np.float32)       # a power of two per row: bf16 values still
+    q_h = synth.bf16_round_bits(q_f32).reshape(1, n_req, hq, 128)
+    assert np.array_equal(synth.bf16_widen(q_h).reshape(-1, 128), q_f32)
+    norm = np.sqrt((q_f32.astype(np.float64) ** 2).sum(1))
+    assert norm.min() >= 2.0 ** exponent and norm.max() < 2.0 ** (exponent + 1)
+    q_codes = torch.zeros((1, n_req, hq, 16), dtype=torch.uint8, device=dev)
+    q_sum = torch.zeros((1, n_req, 128), dtype=torch.int16, device=dev)
+    qbar = torch.zeros((1, n_req, hkv, 16), dtype=torch.uint8, device=dev)
+    ops.hash_encode_queries(bf16_dev(q_h, dev), bf16_dev(w_bits, dev), hkv, q_codes, q_sum, qbar, n_req)
+    want = O.hash_encode(q_h[0], w_f32)
+    assert np.array_equal(q_codes[0].cpu().numpy(), want)
+    pm = np.unpackbits(want, axis=-1, bitorder="little").astype(np.int32) * 2 - 1
+    assert np.array_equal(q_sum[0].cpu().numpy(), pm.sum(1))
+    qm = np.stack([O.q_head_mean(synth.bf16_widen(q_h[0][r]), hkv) for r in range(n_req)])
+    assert np.array_equal(qbar[0].cpu().numpy(), O.hash_encode_f32(qm, w_f32))
+
+
 def test_hash_encode_keys_beyond_the_fp32_range(ucm, dev):
     """Keys whose fp32 sums overflow on the way (components up to 3e38: the exact sum may be finite and of either
     sign where the matrix cores hold an infinity or a NaN), keys with infinite components and keys with NaN: the

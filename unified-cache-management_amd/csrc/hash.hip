@@ -43,8 +43,8 @@ constexpr int kBits = 128;          // code length
 constexpr int kWtStride = kDim + 8; // bf16 elements per transposed weight row (272 B: spreads LDS banks)
 constexpr int kQueueCap = 256;
 constexpr int kMaxHeads = 8;
-constexpr float kTau2 = 0x1p-30f;   // (2^-15)^2: the bound for the queries' group means (three bf16 terms per mean, added afterwards)
-constexpr float kTauBlocks2 = 0x1p-32f;   // (2^-16)^2: the bound for keys and query rows (one chain of 127 additions per result)
+constexpr float kTau = 0x1p-16f;      // the bound for keys and query rows (one chain of 127 additions per result)
+constexpr float kTauMeans = 0x1p-15f; // the bound for the queries' group means (three bf16 terms per mean, added afterwards)
 
 __device__ __forceinline__ unsigned lanes_below(unsigned long long mask)
 {
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(kEncThreads, 2) void hash_encode_blocks_kernel(
 #pragma unroll
         for (int d = 16; d >= 1; d >>= 1) { m = fmaxf(m, __shfl_xor(m, d, 64)); }
         // (the same in all lanes: a scalar register)
-        sw[nb] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sqrtf(kTauBlocks2 * m) * 1.0001f)));
+        sw[nb] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(kTau * sqrtf(m) * 1.0001f)));
     }
 
     // ---- block summaries from the counts in LDS: a wave's own, or those of its team, whose waves take turns at the heads
@@ -692,7 +692,7 @@ __global__ __launch_bounds__(kEncThreads, 2) void hash_encode_blocks_kernel(
 // * (largest ||x|| of the tile) * ||w_col|| - more than the fp32 accumulation can be off by - is redone
 // in fp64 (a product of an fp32 and a bf16 value is exact in fp64): a few of them by the whole wave, many by their lanes,
 // d ascending, every lane working on one of its own results at a time.  A tile whose vectors are all tiny (norm below 2^-60, where
-// bf16 subnormals and the bound itself lose bits) is redone whole.  Query rows are the A operand and weights
+// bf16 subnormals and the squares of the norms lose bits) is redone whole.  Query rows are the A operand and weights
 // the B operand, so a lane holds one weight column and 16 vectors, and a ballot over the lanes is a vector's
 // 32-bit code word.  The weights sit in LDS in their own [d][column] order (a lane reads its column two
 // bytes at a time, neighbours in neighbouring banks); the means are formed once per workgroup, a 16-byte
@@ -965,7 +965,8 @@ __global__ __launch_bounds__(kQueryThreads, 4) void hash_query_kernel(
         nx2 += __shfl_xor(nx2, 32, 64);
         const float max2 = wave_max32(nx2);
         const bool all_exact = (max2 > 0.0f && !(max2 >= 0x1p-120f)) || !(max2 < __builtin_inff());   // tiny norms, or none that is finite
-        const float bound = sqrtf(kTauBlocks2 * max2) * sqrtf(nw2) * 1.01f;
+        // (the factor stays outside the root: squared, it would push a square just above the line of all_exact below fp32's range)
+        const float bound = kTau * sqrtf(max2) * sqrtf(nw2) * 1.01f;
         f32x16 acc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) { acc[i] = 0.0f; }
@@ -1043,7 +1044,7 @@ __global__ __launch_bounds__(kQueryThreads, 4) void hash_query_kernel(
         }
         const float max2 = fmaxf(s.mean_max2[0], s.mean_max2[1]);
         const bool all_exact = (max2 > 0.0f && !(max2 >= 0x1p-120f)) || !(max2 < __builtin_inff());   // tiny norms, or none that is finite
-        const float bound = sqrtf(kTau2 * max2) * sqrtf(nw2) * 1.01f;
+        const float bound = kTauMeans * sqrtf(max2) * sqrtf(nw2) * 1.01f;
         unsigned positive = 0, redo = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
