@@ -835,7 +835,17 @@ def test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_
 @pytest.mark.parametrize("n_layers,rows_n,n_slots,bb", [(32, 32, 2, 8192 + 16), (25, 41, 3, 16384), (40, 41, 2, 8192 + 16),   # a pair a thread, or four
                                                         (3, 5, 40, 3 * 131072 + 16), (2, 7, 6, 8192)])
 def test_counted_loads_of_many_rows_and_long_slices(ucm, dev, n_layers, rows_n, n_slots, bb):
-    """Running totals of 1024 pairs and more, slices of several pieces each, and the short slices that go by slot instead."""
+    """Running totals of 1024 pairs and more, slices of several pieces each, and a short plan of short slices, which goes by slot instead."""
+    test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_slots, bb, True)
+
+
+@pytest.mark.parametrize("n_layers,rows_n,n_slots,bb", [
+    (2, 16, 64, 4096), (2, 16, 65, 4096),                # 4096 slots to copy from, the last plan that goes slot by slot, and more
+    (8, 20, 60, 16), (8, 20, 60, 1024 + 16), (8, 20, 60, 8192 - 16), (8, 20, 60, 8192),      # a wave's part of a slice, one trip of it and all
+    (4, 64, 70, 64),                                     # more slices than there are waves
+    (60, 68, 3, 48)])                                    # four pairs a thread in the running total
+def test_counted_loads_of_short_slices(ucm, dev, n_layers, rows_n, n_slots, bb):
+    """Slices of up to 8 KiB by single waves, on both sides of the rule that takes them."""
     test_planned_loads_of_every_size_of_workgroup(ucm, dev, n_layers, rows_n, n_slots, bb, True)
 
 

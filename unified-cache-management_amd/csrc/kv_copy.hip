@@ -52,11 +52,11 @@ __device__ __forceinline__ void copy_trip(uint8_t* __restrict__ dst, const uint8
 // A workgroup's share of a slice; size is a multiple of 16.  What is left after the 128 KiB trips goes in trips of 64, 32 and 16 KiB (the slices of 64-, 32- and
 // 16-token blocks), each with all its loads in flight at once, and a last partial one.  (kT threads: a trip is kT * 128 bytes.)
 template <int kT = kThreads>
-__device__ __forceinline__ void copy_slice(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t size)
+__device__ __forceinline__ void copy_slice(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, size_t size, unsigned thread = threadIdx.x)
 {
     constexpr size_t kTrip = static_cast<size_t>(kT) * 16 * kUnroll;
     size_t o = 0;
-    const size_t mine = threadIdx.x * 16u;
+    const size_t mine = thread * 16u;
     for (; o + kTrip <= size; o += kTrip) { copy_trip<kUnroll, kT>(dst, src, o + mine); }
     if (o + kTrip / 2 <= size) { copy_trip<kUnroll / 2, kT>(dst, src, o + mine); o += kTrip / 2; }
     if (o + kTrip / 4 <= size) { copy_trip<kUnroll / 4, kT>(dst, src, o + mine); o += kTrip / 4; }
@@ -253,9 +253,17 @@ __global__ __launch_bounds__(kThreads) void kv_load_planned_kernel(
 // of ten barriers, 15.7 so; 116 loads 29.5 and 27.4; 887 loads of 8 layers 170.7 and 169.8.)
 // grid: x = workgroup.
 constexpr unsigned kMaxPlannedPairs = 4096;
+// Slices of up to kShortSlice go through one wave each, in workgroups that are all resident at once: sixteen are found and copied side
+// by side where the whole workgroup took them one after the other.  us, the whole workgroup | a workgroup of 256 threads per slot of
+// the plan (idle ones cost 0.4 ns each) | this, 4 KiB: 8 layers x 64 x 24 slots, all load 141 | 35 | 36, a fifth 34 | 16.7 | 9.9;
+// 8 x 32 x 800, a tenth 221 | 151 | 60 to 64, one in a hundred 27.7 | 123 | 8.2; 32 x 64 x 1000, one in a hundred 251 | 1110 | 61 to 73.
+// 8 KiB: all of 8 x 64 x 24 142 | 64 | 70 to 75, one in a hundred of 32 x 64 x 1000 253 | 1112 | 114 to 118.  Teams of two and four
+// waves 0 to 8 and 10 to 110 % slower at up to 4 KiB, alike at 8; twice the workgroups 2 us slower, half of them waiting for the others.
+constexpr int kTeamThreads = 64;
+constexpr unsigned kTeamGroups = 512;
 
-// kWhole: slices of at most one piece.
-template <bool kWhole>
+// kWhole: slices of at most one piece.  kT threads copy one: the whole workgroup, or a team of it.
+template <bool kWhole, int kT>
 __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
     void* const* __restrict__ layers, size_t kv_stride, size_t block_bytes, unsigned num_blocks,
     const uint8_t* __restrict__ pool, uint64_t pool_blocks, size_t pool_block_bytes, unsigned store_first_layer,
@@ -339,7 +347,15 @@ __global__ __launch_bounds__(kThreads) void kv_load_counted_kernel(
                 kWhole ? block_bytes : min(kLoadPiece, block_bytes - off)};
     };
     unsigned p = blockIdx.x % pieces, w = blockIdx.x / pieces;
-    if constexpr (kWhole) {
+    if constexpr (kT < kThreads) {                       // (the teams meet no barrier)
+        constexpr unsigned kTeams = kThreads / kT;
+        static_assert(kWhole && kT % 64 == 0, "a team is whole waves and copies whole slices");
+        const unsigned team = __builtin_amdgcn_readfirstlane(threadIdx.x / kT);
+        for (w = blockIdx.x + team * gridDim.x; w < slices; w += kTeams * gridDim.x) {
+            const Piece cur = find(w, 0);
+            if (cur.dst) { copy_slice<kT>(cur.dst, cur.src, cur.size, threadIdx.x % kT); }
+        }
+    } else if constexpr (kWhole) {
         for (; w < slices; w += w_step) {                // (uniform in the workgroup)
             const Piece cur = find(w, 0);
             if (!cur.dst) { continue; }
@@ -559,19 +575,23 @@ extern "C" int ucm_kv_load_planned_tp(void* const* layers, int n_layers, size_t 
                 store_first_layer + n_layers - 1, pool_block_bytes);
     UCM_REQUIRE(src_stride >= 1 && dst_stride >= n_slots && dst_layer_stride >= 0,
                 "ucm_kv_load_planned: src_stride=%d dst_stride=%d n_slots=%d", src_stride, dst_stride, n_slots);
-    if (load_count && (block_bytes > kShortSlice || n_slots > 1 << 20) &&
-        static_cast<unsigned>(n_layers) * static_cast<unsigned>(batch) <= kMaxPlannedPairs) {
-        // the rows' counts say exactly what there is to copy: 1024 workgroups share it evenly (short slices are better off with
-        // small workgroups, the idle ones among them: 8 layers x 64 x 24 loads of 4 KiB 144 and 47 us, a tenth of 8 KiB 35.5 and 33)
-        hipLaunchKernelGGL(block_bytes <= kLoadPiece ? kv_load_counted_kernel<true> : kv_load_counted_kernel<false>, dim3(1024),
-                           dim3(kThreads), 0, ucm::as_stream(stream), layers, kv_stride,
+    // A short plan of short slices goes slot by slot: a few idle workgroups cost less than the running total of the counts (1 layer x 8
+    // x 20 of 4 KiB 2.6 and 4.4 us, 2 x 16 x 50, all load, 6.9 and 7.0, 8 x 16 x 50 with two loads a row 5.9 and 4.8).
+    const bool short_slices = block_bytes <= kShortSlice;
+    const bool few_slots = short_slices && static_cast<int64_t>(n_slots) * batch * n_layers * 2 <= 4096;
+    if (load_count && !few_slots && static_cast<unsigned>(n_layers) * static_cast<unsigned>(batch) <= kMaxPlannedPairs) {
+        // the rows' counts say exactly what there is to copy: persistent workgroups share it evenly
+        const auto kernel = short_slices                ? kv_load_counted_kernel<true, kTeamThreads>
+                            : block_bytes <= kLoadPiece ? kv_load_counted_kernel<true, kThreads>
+                                                        : kv_load_counted_kernel<false, kThreads>;
+        hipLaunchKernelGGL(kernel, dim3(short_slices ? kTeamGroups : 1024u), dim3(kThreads), 0, ucm::as_stream(stream), layers, kv_stride,
                            block_bytes, static_cast<unsigned>(num_blocks), static_cast<const uint8_t*>(pool),
                            static_cast<uint64_t>(pool_blocks), pool_block_bytes, static_cast<unsigned>(store_first_layer),
                            load_sel, static_cast<unsigned>(n_slots), src_table, static_cast<unsigned>(src_stride), dst_table,
                            static_cast<unsigned>(dst_stride), dst_layer_stride, load_count, rows,
                            static_cast<unsigned>(table_rows), static_cast<unsigned>(batch), static_cast<unsigned>(n_layers), lay);
     } else {
-        // The entries to load are scattered over a row (or slices are short, or there are too many rows for the counted kernel's table).
+        // The entries to load are scattered over a row (or there are too many rows for the counted kernel's table).
         const int64_t table = static_cast<int64_t>(batch) * n_layers * 2;
         const auto pieces = [&](size_t piece) { return static_cast<int64_t>((block_bytes + piece - 1) / piece); };
         auto follow_slots = [&](auto kernel, int threads) {
