@@ -715,6 +715,38 @@ def test_kv_moves_at_the_sizes_of_pieces(ucm, dev, bb):
     assert np.array_equal(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("bb,n", [(131072, 3), (196608, 64), (196608, 65), (262144 - 16, 300),        # 256 pieces and more: left whole
+                                  (262144, 64), (262144, 65), (262144 + 16, 43), (262144, 256), (262144, 257),   # from 1025 on cut again
+                                  (524288, 32), (524288, 33), (524288, 128), (524288, 129)])
+def test_kv_moves_of_cut_and_whole_slices(ucm, dev, bb, n):
+    """Both sides of the rule that cuts a launch's slices between workgroups: dumps, loads, and gathers whose slots are all in use
+    or nearly all idle (those stay whole), byte for byte."""
+    from ucm_amd import ops
+
+    nb = n + 3
+    rng = np.random.default_rng(bb + n)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(n)
+    cache = torch.randint(0, 256, (2, nb, bb), dtype=torch.uint8, device=dev, generator=gen)
+    lp, ids = ops.LayerPointers([cache]), rng.permutation(nb)[:n].astype(np.int32)
+    ids_d = i32(ids, dev)
+    staging = torch.full((n, 1, 2, bb), 0xAB, dtype=torch.uint8, device=dev)
+    ops.kv_gather_blocks(lp, nb * bb, bb, nb, ids_d, staging)
+    want = cache[:, ids_d.long()].transpose(0, 1)
+    assert torch.equal(staging[:, 0], want)
+    to = rng.permutation(nb)[:n].astype(np.int32)
+    loaded = cache.clone()
+    ops.kv_scatter_blocks(ops.LayerPointers([loaded]), nb * bb, bb, nb, i32(to, dev), staging)
+    after = cache.clone()
+    after[:, i32(to, dev).long()] = want.transpose(0, 1)
+    assert torch.equal(loaded, after)
+    for used in (n, n // 9):                                                                # slots of the launch to blocks of the staging area
+        out = torch.full((2 * used + 1, bb), 0xCD, dtype=torch.uint8, device=dev)
+        ops.kv_gather_selected(lp, nb * bb, bb, nb, ids_d.view(1, 1, n), i32([[used]], dev), torch.zeros(1, dtype=torch.int64, device=dev),
+                               i32([used], dev), n, out, 2 * used)
+        assert torch.equal(out[: 2 * used].view(2, used, bb), cache[:, ids_d[:used].long()]) and (out[2 * used] == 0xCD).all()
+
+
 def test_kv_moves_of_one_tensor_parallel_rank(ucm, dev):
     """Four ranks share the stored block; each moves its own K and V slices to where get_offset (esa.py:124-135) puts
     them, leaves the others' bytes alone, and reads them back - through the block moves and through the planned load."""

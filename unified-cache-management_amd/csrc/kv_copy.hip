@@ -1,8 +1,8 @@
 // Paged-KV block moves: pointer-array batch copy, block-id driven dump/load in
 // the stored-block layout, and the gather of selected blocks from a device
 // block table.  Pure HBM traffic: every byte is read once and written once, so
-// the kernels are 16-byte vector copies with non-temporal hints, one
-// 1024-thread workgroup per 128 KiB of a slice (a 256 KiB K or V block is two),
+// the kernels are 16-byte vector copies with non-temporal hints, a 1024-thread
+// workgroup per slice or per 128 KiB of it (a 256 KiB K or V block is two),
 // launched with far more workgroups than the 256 CUs.  Of the
 // shapes tried on MI355X (8 KiB .. 256 KiB per workgroup, 64 .. 1024 threads,
 // 1 .. 16 loads in flight per thread, persistent grids, with and without the
@@ -18,9 +18,8 @@ constexpr int kThreads = 1024;
 constexpr int kUnroll = 8;
 constexpr size_t kStep = static_cast<size_t>(kThreads) * 16 * kUnroll;  // 128 KiB per trip
 
-// Gathers, dumps and loads by block list: a workgroup moves one trip (128 KiB) of a slice and ends with its stores on their
-// way.  (Both trips of a 256 KiB slice in one workgroup, us: 32 layers x 256 blocks out and back 2845 to 2911 by process, 2769 to 2828
-// this way; 5.1 GB gathered 1751 to 1821, 1707 to 1730; one layer of 20 blocks out and back 23.4, 14.2.)
+// Gathers, dumps and loads by block list: a workgroup moves a whole slice, or one piece of it (a trip, 128 KiB) and ends with its
+// stores on their way: see cut_slices.
 // Slices of up to 8 KiB, the blocks of one or two kv heads, take 256 threads: a compute unit has eight of them under way and only
 // two of 1024 (32 layers x 1024 blocks out and back, 4 KiB 299 -> 175 us = 6.1 TB/s, 8 KiB 435 -> 377; 16 KiB 730 -> 760, so no more).
 constexpr int kShortThreads = 256;
@@ -87,35 +86,36 @@ struct StoredLayout {
     }
 };
 
-// grid: x = index into block_ids * pieces + piece, y = layer, z = K|V
-template <bool kToStaging, int kT>
+// kCut: a workgroup takes one of the slice's `pieces`
+// grid: x = index into block_ids (* pieces + piece), y = layer, z = K|V
+template <bool kToStaging, bool kCut, int kT>
 __global__ __launch_bounds__(kT) void kv_blocks_kernel(void* const* __restrict__ layers,
                                                              size_t kv_stride, size_t block_bytes,
                                                              const int32_t* __restrict__ block_ids,
                                                              unsigned num_blocks,
-                                                             uint8_t* __restrict__ staging, unsigned pieces, size_t piece, StoredLayout lay)
+                                                             uint8_t* __restrict__ staging, unsigned pieces, StoredLayout lay)
 {
-    const unsigned i = pieces == 1 ? blockIdx.x : blockIdx.x / pieces, l = blockIdx.y, kv = blockIdx.z, n_layers = gridDim.y;
-    const size_t off = (blockIdx.x - i * pieces) * piece;
+    const unsigned i = kCut ? blockIdx.x / pieces : blockIdx.x, l = blockIdx.y, kv = blockIdx.z, n_layers = gridDim.y;
+    const size_t off = kCut ? (blockIdx.x - i * pieces) * kStep : 0;
     const unsigned id = static_cast<unsigned>(block_ids[i]);
     if (id >= num_blocks) { return; }  // ids outside the cache are skipped, never dereferenced
     uint8_t* cache = static_cast<uint8_t*>(layers[l]) + kv * kv_stride +
                      static_cast<size_t>(id) * block_bytes + off;
     uint8_t* stage = staging + static_cast<size_t>(i) * n_layers * lay.layer_pitch + lay.slice(l, kv, block_bytes) + off;
-    const size_t size = min(piece, block_bytes - off);
+    const size_t size = kCut ? min(kStep, block_bytes - off) : block_bytes;
     if (kToStaging) { copy_slice<kT>(stage, cache, size); }
     else { copy_slice<kT>(cache, stage, size); }
 }
 
-// grid: x = position in the request's selection * pieces + piece, y = request, z = layer*2 + K|V
-template <int kT>
+// grid: x = position in the request's selection (* pieces + piece), y = request, z = layer*2 + K|V
+template <bool kCut, int kT>
 __global__ __launch_bounds__(kT) void kv_gather_selected_kernel(
     const void* const* __restrict__ layers, size_t kv_stride, size_t block_bytes,
     const int32_t* __restrict__ phys, const int32_t* __restrict__ count, unsigned num_blocks,
     unsigned n_req, unsigned phys_stride, const int64_t* __restrict__ dst_off,
-    const int32_t* __restrict__ region_k, uint8_t* __restrict__ staging, uint64_t staging_blocks, unsigned pieces, size_t piece)
+    const int32_t* __restrict__ region_k, uint8_t* __restrict__ staging, uint64_t staging_blocks, unsigned pieces)
 {
-    const unsigned j = pieces == 1 ? blockIdx.x : blockIdx.x / pieces, r = blockIdx.y, l = blockIdx.z >> 1, kv = blockIdx.z & 1;
+    const unsigned j = kCut ? blockIdx.x / pieces : blockIdx.x, r = blockIdx.y, l = blockIdx.z >> 1, kv = blockIdx.z & 1;
     const size_t lr = static_cast<size_t>(l) * n_req + r;
     if (static_cast<int32_t>(j) >= count[lr]) { return; }
     const unsigned id = static_cast<unsigned>(phys[lr * phys_stride + j]);
@@ -126,8 +126,8 @@ __global__ __launch_bounds__(kT) void kv_gather_selected_kernel(
     if (off < 0 || region < 0) { return; }
     const uint64_t slot = static_cast<uint64_t>(off) + (static_cast<uint64_t>(l) * 2 + kv) * static_cast<uint64_t>(region) + j;
     if (slot >= staging_blocks) { return; }              // never write outside the staging buffer
-    const size_t at = (blockIdx.x - j * pieces) * piece;
-    copy_slice<kT>(staging + slot * block_bytes + at, src + at, min(piece, block_bytes - at));
+    const size_t at = kCut ? (blockIdx.x - j * pieces) * kStep : 0;
+    copy_slice<kT>(staging + slot * block_bytes + at, src + at, kCut ? min(kStep, block_bytes - at) : block_bytes);
 }
 
 // Loads planned on the device: slot j of request row `row` receives logical block load_sel[l][row][j] (or
@@ -413,31 +413,38 @@ int stored_layout(const char* name, size_t block_bytes, int rank, int tp_size, S
     return UCM_OK;
 }
 
-// Pieces of a slice, a trip each; a list so long that its pieces would not fit one launch is moved slice by slice.
-struct Pieces {
-    unsigned count;
-    size_t bytes;
-};
-Pieces pieces_of(size_t block_bytes, int n, int threads)
+// Pieces (a 128 KiB trip each) that `slices` slices are cut into between workgroups, or 1: left whole.  A workgroup with several trips
+// waits before each for the registers of the one before; but a part of a trip at a slice's end takes the place of a whole one, and
+// a launch of a few workgroups more than are resident at once (two per compute unit) ends with the chip half empty.  So slices
+// are cut where every piece has a compute unit of its own, and those of two trips and more where there are several rounds of pieces.
+// us, whole | cut, by process:
+// 256 KiB: one layer of 16 blocks 6.2 | 4.4, 100 blocks 17.4 | 17.5 to 19.1, 200 blocks 35 to 38 | 37 to 40, 400 blocks 75 to 78 | 71 to 73, 32 layers x 256 out and
+// back 2845 to 2937 | 2769 to 2856, 5.1 GB gathered 1724 to 1821 | 1707 to 1757; 512 KiB: 16 blocks 16 | 7.6, 100 blocks 34.5 | 38, 16
+// layers x 64 385 | 360; 160 KiB: 100 blocks 12.2 | 15.0, 16 layers x 64 120 | 129; 192 KiB:
+// 16 blocks 5.1 to 7.0 | 5.2, 100 blocks 13.7 | 15.6, 200 blocks 27.5 | 30.2, 16 layers x 64 145 | 144.
+// (What is never cut has an instance without the division: 16 KiB slices 3.1 us for 200 blocks, 3.4 with it.)
+unsigned cut_slices(size_t block_bytes, uint64_t grid_x, uint64_t slices)
 {
-    const size_t trip = static_cast<size_t>(threads) * 16 * kUnroll, count = (block_bytes + trip - 1) / trip;
-    if (static_cast<uint64_t>(n) * count > 0xffffffffu / static_cast<unsigned>(threads)) { return {1u, block_bytes}; }
-    return {static_cast<unsigned>(count), trip};
+    const uint64_t pieces = (block_bytes + kStep - 1) / kStep, workgroups = slices * pieces;
+    const bool fits = grid_x * pieces <= 0xffffffffu / kThreads;
+    const bool cut = workgroups <= 256 || (block_bytes >= 2 * kStep && workgroups > 1024);
+    return fits && cut ? static_cast<unsigned>(pieces) : 1u;
 }
 
 template <bool kToStaging>
 int move_blocks(const char* name, const void* const* layers, int n_layers, size_t kv_stride, size_t block_bytes, int num_blocks,
                 const int32_t* block_ids, int n, void* staging, const StoredLayout& lay, ucm_stream_t stream)
 {
+    const unsigned pieces = cut_slices(block_bytes, static_cast<uint64_t>(n), static_cast<uint64_t>(n) * n_layers * 2);
     auto launch = [&](auto kernel, int threads) -> int {
-        const Pieces p = pieces_of(block_bytes, n, threads);
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n) * p.count, n_layers, 2), dim3(threads), 0, ucm::as_stream(stream),
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n) * pieces, n_layers, 2), dim3(threads), 0, ucm::as_stream(stream),
                            const_cast<void* const*>(layers), kv_stride, block_bytes, block_ids, static_cast<unsigned>(num_blocks),
-                           static_cast<uint8_t*>(staging), p.count, p.bytes, lay);
+                           static_cast<uint8_t*>(staging), pieces, lay);
         return ucm::check_hip(hipGetLastError(), name);
     };
-    return block_bytes <= kShortSlice ? launch(kv_blocks_kernel<kToStaging, kShortThreads>, kShortThreads)
-                                      : launch(kv_blocks_kernel<kToStaging, kThreads>, kThreads);
+    if (block_bytes <= kShortSlice) { return launch(kv_blocks_kernel<kToStaging, false, kShortThreads>, kShortThreads); }
+    return pieces > 1 ? launch(kv_blocks_kernel<kToStaging, true, kThreads>, kThreads)
+                      : launch(kv_blocks_kernel<kToStaging, false, kThreads>, kThreads);
 }
 
 // dst row dst_idx[i] = src row src_idx[i]: one 256-thread workgroup per pair (a step's query rows are a few KiB each,
@@ -537,16 +544,21 @@ extern "C" int ucm_kv_gather_selected(const void* const* layers, int n_layers, s
     UCM_REQUIRE(block_bytes > 0 && block_bytes % 16 == 0 && kv_stride % 16 == 0 && ucm::aligned16(staging),
                 "ucm_kv_gather_selected: sizes and staging must be multiples of 16");
     if (n_req == 0 || max_count == 0) { return UCM_OK; }
+    // What is selected fits the staging area, so slots far beyond its blocks are known to be idle, and pieces would only double them (8
+    // layers x 16 requests x 1000 slots of 256 KiB, three in use, 227 us whole, 528 cut; 200 slots, five in use, 130 and 161; 100
+    // slots, twenty in use, 462 and 446: level at a tenth).
+    const uint64_t slots = static_cast<uint64_t>(max_count) * n_req * n_layers * 2;
+    const unsigned pieces = slots / 8 > static_cast<uint64_t>(staging_blocks) ? 1u : cut_slices(block_bytes, static_cast<uint64_t>(max_count), slots);
     auto launch = [&](auto kernel, int threads) -> int {
-        const Pieces p = pieces_of(block_bytes, max_count, threads);
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(max_count) * p.count, n_req, n_layers * 2), dim3(threads), 0,
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(max_count) * pieces, n_req, n_layers * 2), dim3(threads), 0,
                            ucm::as_stream(stream), layers, kv_stride, block_bytes, phys, count, static_cast<unsigned>(num_blocks),
                            static_cast<unsigned>(n_req), static_cast<unsigned>(phys_stride), dst_off, region_k,
-                           static_cast<uint8_t*>(staging), static_cast<uint64_t>(staging_blocks), p.count, p.bytes);
+                           static_cast<uint8_t*>(staging), static_cast<uint64_t>(staging_blocks), pieces);
         return ucm::check_hip(hipGetLastError(), "ucm_kv_gather_selected");
     };
-    return block_bytes <= kShortSlice ? launch(kv_gather_selected_kernel<kShortThreads>, kShortThreads)
-                                      : launch(kv_gather_selected_kernel<kThreads>, kThreads);
+    if (block_bytes <= kShortSlice) { return launch(kv_gather_selected_kernel<false, kShortThreads>, kShortThreads); }
+    return pieces > 1 ? launch(kv_gather_selected_kernel<true, kThreads>, kThreads)
+                      : launch(kv_gather_selected_kernel<false, kThreads>, kThreads);
 }
 
 extern "C" int ucm_kv_load_planned_tp(void* const* layers, int n_layers, size_t kv_stride, size_t block_bytes,
