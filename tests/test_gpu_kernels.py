@@ -646,6 +646,43 @@ def test_topk_windows_of_hard_scores(ucm, dev, n, kind):
         assert (idx[l, 0, k:] == -7).all()
 
 
+@pytest.mark.parametrize("L,R,n", [(4, 256, 129), (5, 205, 129), (5, 205, 256), (4, 384, 257), (29, 53, 257), (29, 53, 512), (4, 384, 1000),
+                                   (29, 53, 1000), (3, 513, 1024)])     # 1024 rows and more of up to 256 blocks, 1536 and more of longer ones
+@pytest.mark.parametrize("kind", ["ties", "distinct", "extremes"])
+def test_topk_windows_of_many_rows(ucm, dev, L, R, n, kind):
+    """Both sides of the rule that gives a request one wave or four, every tier it covers, ragged lengths and numbers of picks."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(n + R)
+    if kind == "ties":
+        scores = rng.integers(-6, 7, (L, R, n)).astype(np.float32)
+    elif kind == "distinct":
+        scores = rng.standard_normal((L, R, n)).astype(np.float32)
+    else:
+        scores = rng.choice(np.array([0x7fffffff, 0xffffffff, 0x7f800000, 0xff800000, 0, 0x3f800000], np.uint32), (L, R, n)).view(np.float32)
+    lens = rng.integers(n // 2, n + 1, R).astype(np.int32)
+    lens[0], lens[1] = n, 4
+    ks = np.minimum(rng.integers(3, 40, R), lens - 1).astype(np.int32)
+    table = np.argsort(rng.random((R, n)), axis=1).astype(np.int32)
+    idx = torch.full((L, R, n), -7, dtype=torch.int32, device=dev)
+    phys, cnt = idx.clone(), torch.zeros((L, R), dtype=torch.int32, device=dev)
+    scores_d = torch.from_numpy(scores.view(np.int32)).to(dev).view(torch.float32).view(L, R * n)
+    ops.topk_windows(scores_d, i32(np.arange(R) * n, dev), i32(lens, dev), i32(ks, dev), n, idx, cnt, block_tables=i32(table, dev), phys_out=phys)
+    assert torch.equal(cnt, i32(ks, dev).expand(L, R))
+    # the oracle's order by one sort over all rows: forced blocks first, then the candidates by key, the first index first
+    u = scores.view(np.uint32).astype(np.int64)
+    key = np.where(u >> 31, 0xffffffff - u, u | 0x80000000)
+    i = np.arange(n)
+    key[:, (i < 1) | ((i >= lens[:, None] - 2) & (i < lens[:, None]))] = 1 << 33
+    key[:, i >= lens[:, None]] = -1
+    order = np.argsort(-key, axis=-1, kind="stable")
+    chosen = i < ks[:, None]
+    want = np.sort(np.where(chosen, order, n), axis=-1)
+    got, got_phys = idx.cpu().numpy(), phys.cpu().numpy()
+    assert np.array_equal(np.where(want < n, want, -7), got)
+    assert np.array_equal(np.where(want < n, table[np.arange(R)[None, :, None], np.minimum(want, n - 1)], -7), got_phys)
+
+
 @pytest.mark.parametrize("bb", [262144, 4096, 48, 16 + 32768])
 def test_kv_dump_load_round_trip(ucm, dev, bb):
     """Config-3 shape in small: random block table, scatter staging->cache, gather cache->staging, byte exact."""

@@ -523,6 +523,30 @@ def test_kvstar_topk_heap_ties(ucm, dev, max_len):
         assert np.all(a[np.arange(max_len)[None, :] >= cnt[:, None]] == -1)
 
 
+@pytest.mark.parametrize("n_tasks,max_len", [(1024, 256), (1025, 256), (1536, 512), (1537, 512), (1537, 1024)])
+def test_kvstar_topk_heap_ties_of_many_tasks(ucm, dev, n_tasks, max_len):
+    """The heap's ties on both sides of the rule that gives a task one wave or four."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(n_tasks + max_len)
+    kinds = 40                                                     # tasks repeat: the oracle's heap is run once for each kind
+    lens = rng.integers(max_len // 2, max_len + 1, kinds).astype(np.int32)
+    lens[0] = max_len
+    ks = rng.integers(1, 60, kinds).astype(np.int32)
+    votes = [rng.integers(0, int(rng.integers(2, 40)), n).astype(np.float32) for n in lens]
+    off = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    of = rng.integers(0, kinds, n_tasks)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    idx = torch.full((n_tasks, max_len), -7, dtype=torch.int32, device=dev)
+    cnt = torch.zeros(n_tasks, dtype=torch.int32, device=dev)
+    ops.kvstar_topk(t(np.concatenate(votes)), t(off[of]), t(lens[of]), t(ks[of]), max_len, idx, cnt)
+    got, counts = idx.cpu().numpy(), cnt.cpu().numpy()
+    want = [np.sort(O.kvstar_topk(v, int(k))) for v, k in zip(votes, ks)]
+    for i, kind in enumerate(of):
+        w = want[kind]
+        assert counts[i] == len(w) and np.array_equal(got[i, : len(w)], w) and (got[i, len(w) :] == -7).all(), i
+
+
 def test_kvstar_get_task_result_tie_order(ucm, dev):
     """Through the module surface: blocks 1 and 3 identical, 0 and 2 identical and lower; k = 3.  The reference's heap
     returns [3, 1, 2] (simd_compute_kernel.cpp:955-977)."""

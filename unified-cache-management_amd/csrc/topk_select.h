@@ -191,10 +191,10 @@ __device__ __forceinline__ void select_blocks(const SelectArgs& a, int r, int l,
         if (kOutWaves == 1 || wave == 0) {
             const int m = k - start_w - end_w;           // free picks among the candidates
             bool exact = false;
-            if (m > 0) {
-                unsigned key[kEpl];
+            unsigned key[kEpl];
 #pragma unroll
-                for (int j = 0; j < kEpl; ++j) { key[j] = kWaves == 1 ? own_key[kWaves == 1 ? j : 0] : keys[j * 64 + lane]; }
+            for (int j = 0; j < kEpl; ++j) { key[j] = kWaves == 1 ? own_key[kWaves == 1 ? j : 0] : keys[j * 64 + lane]; }
+            if (m > 0) {
                 T = 0;
 #pragma unroll 1
                 for (int bit = 31; bit >= 0; --bit) {
@@ -205,27 +205,18 @@ __device__ __forceinline__ void select_blocks(const SelectArgs& a, int r, int l,
                     if (cnt == k) { exact = true; T = c - 1u; break; }
                 }
             }
-            if (__builtin_expect(!exact, 0)) {
+            if (!exact) {
                 // T is the k-th largest key and others hold the same (or no candidate is to be taken at all): the ones that are kept
                 // get the largest key there is, the others the smallest
-                auto candidate = [&](int j, unsigned& key_j) {
-                    const int i = j * 64 + lane;
-                    key_j = keys[i];
-                    return i >= start_w && i < hi;
-                };
-                unsigned key_j;
-                int greater = 0;
-#pragma unroll 1
-                for (int j = 0; j < kEpl; ++j) { greater += __popcll(__ballot(candidate(j, key_j) && key_j > T)); }
+                const int greater = T == 0xffffffffu ? 0 : count_at_least<kEpl>(key, T + 1u) - start_w - end_w;
                 int tie_lo = 0, tie_hi = m - greater;    // ranks (among the ties) that are kept
                 if (kHeapTies) {
                     // walk the list in index order up to the m-th block with key >= T
                     int seen = 0, g_p = 0;
-#pragma unroll 1
+#pragma unroll
                     for (int j = 0; j < kEpl; ++j) {
-                        const bool cand = candidate(j, key_j);
-                        const unsigned long long ge_mask = __ballot(cand && key_j >= T && key_j != 0u);
-                        const unsigned long long gt_mask = __ballot(cand && key_j > T);
+                        const unsigned long long ge_mask = __ballot(key[j] >= T && key[j] != 0u);
+                        const unsigned long long gt_mask = __ballot(key[j] > T);
                         const int c = __popcll(ge_mask);
                         if (seen < m) {
                             if (seen + c >= m) {
@@ -245,12 +236,13 @@ __device__ __forceinline__ void select_blocks(const SelectArgs& a, int r, int l,
                     tie_hi = m - g_p;                    // ties inside P
                 }
                 int ties_seen = 0;
-#pragma unroll 1
+#pragma unroll
                 for (int j = 0; j < kEpl; ++j) {
-                    const bool eq = candidate(j, key_j) && key_j == T;
+                    const int i = j * 64 + lane;
+                    const bool eq = key[j] == T && i >= start_w && i < hi;
                     const unsigned long long eq_mask = __ballot(eq);
                     const int rank = ties_seen + static_cast<int>(lanes_below(eq_mask));
-                    if (eq) { keys[j * 64 + lane] = rank >= tie_lo && rank < tie_hi ? 0xffffffffu : 0u; }
+                    if (eq) { keys[i] = rank >= tie_lo && rank < tie_hi ? 0xffffffffu : 0u; }
                     ties_seen += __popcll(eq_mask);
                 }
                 T = min(T, 0xfffffffeu);
