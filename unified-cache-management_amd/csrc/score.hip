@@ -44,6 +44,7 @@ using ucm::u32x4;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
+static_assert(kWaves == ucm::kSelectWaves);
 constexpr int kMaxRow = 16 * 128;  // kv_heads * head_dim: what the staged query row may hold
 constexpr int kStaged = std::max(kMaxRow, ucm::select_scratch(16));   // the staged row's place then serves the selection
 constexpr int kMaxTile = 2048;     // blocks of a workgroup: 128 KiB of the narrowest rows (32 bf16)
@@ -309,17 +310,21 @@ __device__ __forceinline__ float head_sum(float dot, int first, int step, int kv
     return s;
 }
 
-// The request's selection with the smallest tier of key registers that holds it (the host allows at most 1024 blocks here); up to
+// The request's selection with the smallest tier of key registers that holds it (the host allows at most 1024 blocks here): up to
 // kSoloBlocks by the first wave alone, from there on by all four.  scratch: kStaged words of LDS
 constexpr int kSoloBlocks = 128;
 
-__device__ __forceinline__ void select_tier(const ucm::SelectArgs& sel, const TileInfo& t, int l, unsigned* scratch, const float* lds)
+__device__ __forceinline__ void select_solo(const ucm::SelectArgs& sel, const TileInfo& t, int l, const float* lds)
 {
-    if (t.n <= 64) { ucm::select_blocks<1, false, 1, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
-    else if (t.n <= kSoloBlocks) { ucm::select_blocks<2, false, 1, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
-    else if (t.n <= 256) { ucm::select_blocks<4, false, kWaves, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
-    else if (t.n <= 512) { ucm::select_blocks<8, false, kWaves, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
-    else { ucm::select_blocks<16, false, kWaves, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    if (t.n <= 64) { ucm::select_wave<1, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
+    else { ucm::select_wave<2, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
+}
+
+__device__ __forceinline__ void select_shared(const ucm::SelectArgs& sel, const TileInfo& t, int l, unsigned* scratch, const float* lds)
+{
+    if (t.n <= 256) { ucm::select_blocks<4, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    else if (t.n <= 512) { ucm::select_blocks<8, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    else { ucm::select_blocks<16, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
 }
 
 // A tile's scores on their way out: collected in LDS and written as whole lines when the tile is done.  (One store per
@@ -341,35 +346,47 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
         for (int i = threadIdx.x; i < n_tile; i += kThreads) { sout[i] = tile_scores[i]; }
         return;
     }
+    if (t.n <= kSoloBlocks && threadIdx.x >= 64) { return; }     // the other waves are done: their registers are free again
+    asm volatile("" ::: "memory");
     const int tiles = max((t.n + a.tile_blocks - 1) / a.tile_blocks, 1);
     const bool alone = tiles == 1 && t.ok;                       // all of the request's scores are here: nobody to wait for
-    const bool solo = t.n <= kSoloBlocks;
-    if (threadIdx.x >= 64 && solo) { return; }
+    auto store = [&]() {
+        for (int i = threadIdx.x; i < n_tile; i += 64) { sout[i] = tile_scores[i]; }
+    };
+    auto draws_last_ticket = [&]() -> bool {
+        const int lane = threadIdx.x;
+        for (int i = lane; i < n_tile; i += 64) {
+            __hip_atomic_store(sout + i, tile_scores[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // (the stores are complete when the wave's memory counter is zero)
+        __builtin_amdgcn_s_waitcnt(0);
+        int32_t* ticket = a.tickets + static_cast<int64_t>(l) * sel.cnt_layer_stride + t.r;
+        int drawn = 0;
+        if (lane == 0) { drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+        if (__builtin_amdgcn_readfirstlane(drawn) != tiles - 1) { return false; }
+        if (lane == 0) { __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+        return true;
+    };
+    if (t.n <= kSoloBlocks) {
+        if (alone) {
+            store();
+            select_solo(sel, t, l, tile_scores);
+            return;
+        }
+        if (draws_last_ticket()) { select_solo(sel, t, l, nullptr); }
+        return;
+    }
     bool last = true;
     if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        if (alone) {
-            for (int i = lane; i < n_tile; i += 64) { sout[i] = tile_scores[i]; }
-        } else {
-            for (int i = lane; i < n_tile; i += 64) {
-                __hip_atomic_store(sout + i, tile_scores[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // (the stores are complete when the wave's memory counter is zero)
-            __builtin_amdgcn_s_waitcnt(0);
-            int32_t* ticket = a.tickets + static_cast<int64_t>(l) * sel.cnt_layer_stride + t.r;
-            int drawn = 0;
-            if (lane == 0) { drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-            last = __builtin_amdgcn_readfirstlane(drawn) == tiles - 1;
-            if (last && lane == 0) { __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-        }
+        if (alone) { store(); } else { last = draws_last_ticket(); }
     }
-    if (!solo && !alone) {
+    if (!alone) {
         __shared__ int draws_last;
         if (threadIdx.x == 0) { draws_last = last ? 1 : 0; }
         __syncthreads();
         last = __builtin_amdgcn_readfirstlane(draws_last) != 0;
     }
-    if (last) { select_tier(sel, t, l, reinterpret_cast<unsigned*>(qbar), alone ? tile_scores : nullptr); }
+    if (last) { select_shared(sel, t, l, reinterpret_cast<unsigned*>(qbar), alone ? tile_scores : nullptr); }
 }
 
 // grid: x = layer, y = dense tile index over all requests (workgroups past the

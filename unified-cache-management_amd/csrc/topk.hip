@@ -1,5 +1,5 @@
-// Per-request block selection with forced windows: one workgroup per
-// (layer, request); the selection itself is ucm::select_blocks (topk_select.h).
+// Per-request block selection with forced windows: one workgroup of one or four waves per
+// (layer, request); the selection itself is ucm::select_wave or select_blocks (topk_select.h).
 //
 // A few KB in, a few hundred bytes out per workgroup: this kernel is latency-bound,
 // not bandwidth-bound; it only has to stay small next to scoring and gather.
@@ -12,31 +12,41 @@ using ucm::lanes_below;
 using ucm::ordered_key;
 
 // grid: x = request, y = layer
-template <int kEpl, bool kHeapTies>
-__global__ __launch_bounds__(kEpl > 2 ? 256 : 64) void topk_windows_kernel(const ucm::SelectArgs a)
+template <int kEpl, bool kHeapTies, int kWaves>
+__global__ __launch_bounds__(kWaves * 64) void topk_windows_kernel(const ucm::SelectArgs a)
 {
-    __shared__ unsigned scratch[ucm::select_scratch(kEpl)];
     const int r = blockIdx.x;
     const int n = a.seg_len[r], off = a.seg_off[r], k = a.topk_len[r];
     asm volatile("" ::"s"(n), "s"(off), "s"(k));         // all three on their way at once, not each where it is first looked at
-    ucm::select_blocks<kEpl, kHeapTies, (kEpl > 2 ? 4 : 1)>(a, r, blockIdx.y, n, off, k, scratch);
+    if constexpr (kWaves == 1) {
+        ucm::select_wave<kEpl, kHeapTies>(a, r, blockIdx.y, threadIdx.x, n, off, k);
+    } else {
+        __shared__ unsigned scratch[ucm::select_scratch(kEpl)];
+        ucm::select_blocks<kEpl, kHeapTies>(a, r, blockIdx.y, n, off, k, scratch);
+    }
 }
 
 template <bool kHeapTies>
 void launch_select(const ucm::SelectArgs& a, int max_seg_len, int n_layers, hipStream_t s)
 {
-    const dim3 grid(a.n_req, n_layers);
-#define UCM_TOPK_LAUNCH(EPL) hipLaunchKernelGGL((topk_windows_kernel<EPL, kHeapTies>), grid, dim3(EPL > 2 ? 256 : 64), 0, s, a)
+    auto launch = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, dim3(a.n_req, n_layers), dim3(waves * 64), 0, s, a); };
+    // Four waves make a request's selection shorter while the chip has room for them; in launches of many requests the three that
+    // wait for the first one's threshold only take places.  us by one wave | four, of integers that tie and of distinct scores: 256 blocks,
+    // 256 requests 5.1 | 4.8 and 4.4 | 3.5, 1024 5.4 | 5.4 and 4.5 | 4.2, 1536 6.0 | 6.8 and 4.8 | 5.0, 5120 9.2 | 15.5 and 6.9 | 10.7;
+    // 512 blocks, 1536 8.9 | 8.9 and 7.5 | 6.1, 2048 9.0 | 10.0 and 7.5 | 6.9, 5120 13.7 | 21.8 and 10.5 | 13.5; 1024 blocks, 1536 14.8 |
+    // 12.5 and 12.2 | 8.4, 2048 15.0 | 18.0 and 12.6 | 10.8, 5120 24.0 | 35.4 and 18.2 | 21.4.  Beyond that by four: 2000 blocks,
+    // 1024 requests 24.8 | 16.4 and 21.8 | 10.9, 4096 43 | 50 and 35 | 29, 5120 63 | 59 and 51 | 35.
+    const int64_t rows = static_cast<int64_t>(a.n_req) * n_layers;
+    const bool four = rows <= (max_seg_len <= 256 ? 1024 : 1536);
     // registers per lane for the keys: the smallest tier that holds the longest request (the radix steps cost
     // one ballot per register and bit)
-    if (max_seg_len <= 64) { UCM_TOPK_LAUNCH(1); }
-    else if (max_seg_len <= 128) { UCM_TOPK_LAUNCH(2); }
-    else if (max_seg_len <= 256) { UCM_TOPK_LAUNCH(4); }
-    else if (max_seg_len <= 512) { UCM_TOPK_LAUNCH(8); }
-    else if (max_seg_len <= 1024) { UCM_TOPK_LAUNCH(16); }
-    else if (max_seg_len <= 2048) { UCM_TOPK_LAUNCH(32); }
-    else { UCM_TOPK_LAUNCH(64); }
-#undef UCM_TOPK_LAUNCH
+    if (max_seg_len <= 64) { launch(topk_windows_kernel<1, kHeapTies, 1>, 1); }
+    else if (max_seg_len <= 128) { launch(topk_windows_kernel<2, kHeapTies, 1>, 1); }
+    else if (max_seg_len <= 256) { four ? launch(topk_windows_kernel<4, kHeapTies, 4>, 4) : launch(topk_windows_kernel<4, kHeapTies, 1>, 1); }
+    else if (max_seg_len <= 512) { four ? launch(topk_windows_kernel<8, kHeapTies, 4>, 4) : launch(topk_windows_kernel<8, kHeapTies, 1>, 1); }
+    else if (max_seg_len <= 1024) { four ? launch(topk_windows_kernel<16, kHeapTies, 4>, 4) : launch(topk_windows_kernel<16, kHeapTies, 1>, 1); }
+    else if (max_seg_len <= 2048) { launch(topk_windows_kernel<32, kHeapTies, 4>, 4); }
+    else { launch(topk_windows_kernel<64, kHeapTies, 4>, 4); }
 }
 
 }  // namespace
