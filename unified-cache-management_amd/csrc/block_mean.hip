@@ -22,7 +22,8 @@ constexpr int kUnroll = 16;   // token rows in flight
 constexpr unsigned kStreamThreads = 256;                  // of block_mean_stream_kernel,
 constexpr unsigned kStreamGroups = 256;                   // one workgroup on each compute unit
 constexpr unsigned kFewGroups = 256;                      // see block_mean_kernel
-constexpr uint64_t kStreamBytes = uint64_t{256} << 20;    // see block_mean_stream_kernel
+constexpr unsigned kStreamLeast = 192;                    // groups: see block_mean_stream_kernel
+constexpr uint64_t kStreamBytes = uint64_t{320} << 20;    // see block_mean_stream_kernel
 constexpr unsigned kKeepBytes = 158 * 1024;               // of the 160 KiB of LDS: means on their way out
 
 __device__ __forceinline__ float bf16_lo(unsigned w) { return __uint_as_float(w << 16); }
@@ -144,8 +145,9 @@ __device__ __forceinline__ void store_means(const u32x4 (&o)[2], float* __restri
 }
 
 // kFew: no more workgroups than compute units, each of which is then alone with its chain of trips to memory: the next
-// 16 tokens are in flight while the current ones are added (128 blocks of 128 tokens 12.1 -> 8.6 us, 256 blocks 14.2 -> 11.9 us; with
-// more workgroups others fill the gaps, and the registers of a second set cost more: 400 blocks 18.5 -> 19.3 us).
+// 16 tokens are in flight while the current ones are added (128 blocks of 128 tokens 12.1 -> 8.6 us, 256 blocks 14.2 -> 11.9 us, of 32
+// tokens 3.9 -> 3.7, of 16 tokens, whose next ones are the same again, 3.2 or, in some processes, 4.2 -> 3.4; with more workgroups
+// others fill the gaps, and the registers of a second set cost more: 400 blocks 18.5 -> 19.3 us).
 //
 // grid: x = block index in the list * col_groups + column group of 1024, y = layer; rows narrower than 1024
 // columns whose thread count divides the workgroup (a tensor-parallel rank's 4, 2 or 1 kv heads of 128) share a
@@ -209,8 +211,12 @@ __global__ __launch_bounds__(kThreads) void block_mean_kernel(
 // the means are 1/128 of the bytes.  So the workgroups are persistent, one per compute unit: each steps over (layer, list
 // entries) groups, with the loads of the next unit - of the same block or the next one - in flight while the current one is
 // added, and keeps the means in LDS until that is full or its work is done: 632 us (6.8 TB/s), 655 when they leave eight
-// groups at a time, 725 -> 672 us into an fp32 table, 166 -> 156 us for 4 layers x 1000 blocks.  Four workgroups of 128
-// threads per compute unit: 667 us.  From 256 MiB of keys on: 1100 blocks 47.1 -> 46.0 us, 600 blocks 27.0 -> 27.6 us.
+// groups at a time, 725 -> 672 us into an fp32 table.  Four workgroups of 128 threads per compute unit: 667 us.  How much that brings depends on
+// the memory a process gets: 691 -> 633, 710 -> 662, and on one machine 645 either way.
+// From 320 MiB of keys and a group for three in four of the compute units on.  us, block_mean_kernel | this, 4 layers x 8 heads: 256 MiB in
+// blocks of 16, 64, 128, 256 tokens 47.5 | 46.4, 43.7 | 43.3, 42.2 | 43.2, 41.9 | 43.4; 325 MiB of 128 tokens 57.7 | 54.5; 384 MiB 72 | 69,
+// 64.3 | 63.0, 61.8 | 61.6, 60.3 | 60.1; 2 GiB 396 | 382, 369 | 342, 355 | 337, 340 | 334.  256 groups of 512 tokens 163 | 165, 192 of 512
+// and of 1024 tokens 61.7 | 59.1 and 125 | 121; 128 of 512 tokens 44 | 51, 96 of 1024 tokens 73 | 85, 64 of 2048 tokens 142 | 166.
 //
 // The block is whole 16-token units.  kT threads take `share` = kT / per_item list entries side by side (per_item = row / 8
 // threads), or, of a row too wide for that, one of col_groups column groups.  kWaveEntry: a wave's threads belong to one entry,
@@ -334,23 +340,34 @@ struct MeanArgs {
     bool of_abs, keys_f16;
 };
 
-int launch_stream(const MeanArgs& a, hipStream_t s)
+// How a launch's work falls into groups: `share` list entries side by side, or one of an entry's column groups.
+struct StreamGroups {
+    unsigned share, col_groups, groups, total;           // groups: of a layer
+};
+StreamGroups stream_groups(const MeanArgs& a)
 {
     constexpr unsigned kT = kStreamThreads;
     const unsigned per_item = a.row / kCols, share = per_item < kT && kT % per_item == 0 ? kT / per_item : 1u;
     const unsigned col_groups = share > 1 ? 1u : (per_item + kT - 1) / kT;
-    const unsigned groups = share > 1 ? (a.n_items + share - 1) / share : a.n_items * col_groups, total = groups * a.n_layers;
+    const unsigned groups = share > 1 ? (a.n_items + share - 1) / share : a.n_items * col_groups;
+    return {share, col_groups, groups, groups * a.n_layers};
+}
+
+int launch_stream(const MeanArgs& a, const StreamGroups& g, hipStream_t s)
+{
+    constexpr unsigned kT = kStreamThreads;
+    const unsigned share = g.share, total = g.total;
     const unsigned each = (total + kStreamGroups - 1) / kStreamGroups, wgs = (total + each - 1) / each;
     const unsigned group_bytes = (a.mode == UCM_MEAN_BF16_STORE ? 16u : 32u) * kT + std::max(share, kT / 64) * 4;
     const unsigned keep = std::min(each, kKeepBytes / group_bytes);
     const unsigned lds = std::max(keep * group_bytes, 82u * 1024u);      // more than half of a compute unit's: never two workgroups on one
-    const bool wave_entry = share == 1 || per_item % 64 == 0;
+    const bool wave_entry = share == 1 || a.row / kCols % 64 == 0;
     auto launch = [&](auto kernel) -> int {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                  static_cast<int>(lds));
         if (e != hipSuccess) { return ucm::check_hip(e, "ucm_block_mean (LDS size)"); }
         hipLaunchKernelGGL(kernel, dim3(wgs), dim3(kT), lds, s, a.k_layers, a.block_ids, a.slots, a.num_blocks, a.repre_rows, a.block_size,
-                           a.row, a.repre, a.repre_layer_stride, a.mode, col_groups, share, a.n_items, groups, total, keep);
+                           a.row, a.repre, a.repre_layer_stride, a.mode, g.col_groups, share, a.n_items, g.groups, total, keep);
         return ucm::check_hip(hipGetLastError(), "ucm_block_mean");
     };
     if (wave_entry) {
@@ -398,7 +415,8 @@ extern "C" int ucm_block_mean(const void* const* k_layers, int n_layers, int num
                             static_cast<unsigned>(block_size), row, static_cast<unsigned>(n), static_cast<unsigned>(n_layers),
                             static_cast<float*>(repre), repre_layer_stride, mode, of_abs, keys_f16};
         const uint64_t bytes = static_cast<uint64_t>(n) * n_layers * block_size * row * 2;
-        if (bytes >= kStreamBytes) { return launch_stream(a, ucm::as_stream(stream)); }
+        const StreamGroups g = stream_groups(a);
+        if (bytes >= kStreamBytes && g.total >= kStreamLeast) { return launch_stream(a, g, ucm::as_stream(stream)); }
     }
 #define UCM_BLOCK_MEAN_ARGS dim3(groups, n_layers), dim3(kThreads), 0, ucm::as_stream(stream), k_layers, block_ids, slots, \
         static_cast<unsigned>(num_blocks), static_cast<unsigned>(repre_rows), static_cast<unsigned>(block_size), row,       \
