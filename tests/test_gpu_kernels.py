@@ -2,6 +2,8 @@
 Bar: bit-exact for indices, bytes and fp32 scores/means (the kernels reproduce
 the reference's summation order, so scores are compared bit for bit as well;
 the looser rel 1e-3 bound of the north star is implied)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -617,6 +619,39 @@ def make_caches(dev, n_layers, nb, bb, seed):
     hs = [np.frombuffer(synth.u64(seed + l, 2 * nb * bb // 8).tobytes(), np.uint8).copy() for l in range(n_layers)]
     ds = [torch.from_numpy(h).to(dev) for h in hs]
     return hs, ds
+
+
+def test_block_mean_of_large_launches_from_two_threads(ucm, dev):
+    """Launches of one kernel that ask for LDS of different sizes, from two threads with streams of their own."""
+    from ucm_amd import ops
+
+    nb, bs, hkv, d = 16, 128, 8, 128
+    cache = torch.empty((nb, bs, hkv, d), dtype=torch.bfloat16, device=dev).normal_()
+    lp = ops.LayerPointers([cache])
+    want = torch.zeros((1, nb, hkv * d), device=dev)
+    ops.block_mean(lp, i32(np.arange(nb), dev), i32(np.arange(nb), dev), want, bs, hkv, d, nb)      # (another kernel: a small launch)
+    torch.cuda.synchronize()
+    faults = []
+
+    def calls(n):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                ids = np.arange(n) % nb
+                ids_d, slots = i32(ids, dev), i32(np.arange(n), dev)
+                for _ in range(20):
+                    out = torch.zeros((1, n, hkv * d), device=dev)
+                    ops.block_mean(lp, ids_d, slots, out, bs, hkv, d, nb)
+                    if not torch.equal(out[0], want[0, ids_d.long()]):
+                        faults.append(n)
+        except Exception as e:  # noqa: BLE001
+            faults.append(repr(e))
+
+    threads = [threading.Thread(target=calls, args=(n,)) for n in (1300, 12000)]                  # 3 and 24 groups a workgroup: 82 and 152 KiB
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not faults
 
 
 @pytest.mark.parametrize("n", [5, 64, 128, 129, 256, 300, 512, 1000, 1024, 2048, 4096])

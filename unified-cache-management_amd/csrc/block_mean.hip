@@ -363,9 +363,7 @@ int launch_stream(const MeanArgs& a, const StreamGroups& g, hipStream_t s)
     const unsigned lds = std::max(keep * group_bytes, 82u * 1024u);      // more than half of a compute unit's: never two workgroups on one
     const bool wave_entry = share == 1 || a.row / kCols % 64 == 0;
     auto launch = [&](auto kernel) -> int {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 static_cast<int>(lds));
-        if (e != hipSuccess) { return ucm::check_hip(e, "ucm_block_mean (LDS size)"); }
+        if (int rc = ucm::allow_lds(kernel, kKeepBytes, "ucm_block_mean")) { return rc; }
         hipLaunchKernelGGL(kernel, dim3(wgs), dim3(kT), lds, s, a.k_layers, a.block_ids, a.slots, a.num_blocks, a.repre_rows, a.block_size,
                            a.row, a.repre, a.repre_layer_stride, a.mode, g.col_groups, share, a.n_items, g.groups, total, keep);
         return ucm::check_hip(hipGetLastError(), "ucm_block_mean");

@@ -17,6 +17,15 @@ char* error_buffer();
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 int check_hip(hipError_t e, const char* what);
 
+// Allows a kernel dynamic LDS beyond 64 KiB.  The runtime keeps one number per kernel, so `most` is the largest any call of it asks
+// for and the same in every call: another thread's call may come between this one and the launch.
+template <typename Kernel>
+int allow_lds(Kernel kernel, size_t most, const char* what)
+{
+    return check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         static_cast<int>(most)), what);
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline hipStream_t as_stream(ucm_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 

@@ -1272,9 +1272,7 @@ extern "C" int ucm_kvstar_block_repre_keys(const void* const* k_layers, int key_
         const unsigned total = static_cast<unsigned>(n) * static_cast<unsigned>(n_layers);
         const unsigned each = (total + kWideGroups - 1) / kWideGroups, wgs = (total + each - 1) / each;
         auto launch = [&](auto kernel) -> int {
-            const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                      static_cast<int>(lds_bytes));
-            if (ea != hipSuccess) { return ucm::check_hip(ea, "ucm_kvstar_block_repre (LDS size)"); }
+            if (int rc = ucm::allow_lds(kernel, kWideLds, "ucm_kvstar_block_repre")) { return rc; }
             hipLaunchKernelGGL(kernel, dim3(wgs), dim3(kWideThreads), lds_bytes, hs, k_layers, block_ids, slots,
                                static_cast<unsigned>(num_blocks), static_cast<unsigned>(n), static_cast<unsigned>(repre_rows),
                                static_cast<unsigned>(block_size), static_cast<unsigned>(kv_heads), static_cast<unsigned>(head_dim),
