@@ -1254,7 +1254,7 @@ def test_delta_plan_slot_counts(ucm, dev, n_slots):
 @pytest.mark.parametrize("n_layers,n_req", [(64, 8), (57, 9)])
 @pytest.mark.parametrize("n_slots", [65, 256, 257, 530])
 def test_delta_plan_on_both_sides_of_the_thread_split(ucm, dev, n_layers, n_req, n_slots):
-    """512 rows (four threads per entry) and 513 (one), with slots that hold a block twice or nothing: the last slot of a
+    """512 rows (four threads per entry of 256 slots, one otherwise) and 513 (one), with slots that hold a block twice or nothing: the last slot of a
     block wins, and loads, slots, resident sets and counts equal the oracle's."""
     from ucm_amd import ops
 
@@ -1277,6 +1277,13 @@ def test_delta_plan_on_both_sides_of_the_thread_split(ucm, dev, n_layers, n_req,
             assert np.array_equal(load_h[l, r], wl) and miss_h[l, r] == moved, (l, r)
             assert np.array_equal(slot_h[l, r, :k], ws[:k]) and np.all(slot_h[l, r, k:] == -7), (l, r)
     assert np.array_equal(resident.cpu().numpy(), res_h)
+
+
+@pytest.mark.parametrize("n_layers,n_req,n_slots", [(32, 8, 65), (1, 257, 99), (1, 257, 100), (57, 9, 100), (32, 8, 257), (1, 257, 299), (64, 8, 300),
+                                                    (32, 8, 513), (1, 257, 831), (64, 8, 832), (57, 9, 832)])
+def test_delta_plan_of_longer_walks_on_both_sides_of_the_thread_split(ucm, dev, n_layers, n_req, n_slots):
+    """256 rows always have four threads per entry, up to 512 only with enough slots."""
+    test_delta_plan_on_both_sides_of_the_thread_split(ucm, dev, n_layers, n_req, n_slots)
 
 
 def test_decode_step_under_graph_capture(ucm, dev):

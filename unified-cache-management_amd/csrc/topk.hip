@@ -371,10 +371,14 @@ int delta_plan_launch(const char* name, const int32_t* sel, const int32_t* sel_p
 #define UCM_PLAN_WIDE(E)                        \
     if (split) { UCM_PLAN_LAUNCH(E, 4); }       \
     else { UCM_PLAN_LAUNCH(E, 1); }
-    // Four threads per entry while all their workgroups of sixteen waves are resident at once, two per compute unit: 512
-    // of 153 / 256 / 400 / 1000 slots 7.7 / 9.4 / 24.4 / 101 us (by one thread 7.9 / 10.6 / 25.2 / 106), but 1024 of 200 slots
-    // 13.6 (11.3).
-    const bool split = static_cast<uint64_t>(n_launch) * n_layers <= 512;
+    // Four threads per entry while every row has a compute unit of its own, and up to two rows per unit where the walk is long: the pair
+    // shares the unit (up to 256 slots) or, for want of registers, takes it in turns, and what a row costs beside the walk, by the 256
+    // slots, counts twice.  us by one thread | four, 256 rows and 384: 65 slots 4.8 | 4.4 and 5.1 | 5.9, 100 5.7 | 4.4 and 6.0 | 6.0,
+    // 200 8.6 | 6.2 and 9.1 | 8.7, 256 9.8 | 6.1 and 10.2 | 8.9; 257 15.6 | 10.2 and 17.6 | 18.9, 300 17.3 | 10.4 and 19.5 | 19.1, 512 27.0 |
+    // 15.1 and 31.3 | 28.3; 513 44 | 33 and 53 | 63, 768 63 | 42 and 77 | 80, 850 80 | 48 and 96 | 93, 1024 95 | 56 and 113 | 109 (there it
+    // spills 34 registers).  1024 rows of 200 slots 11.3 | 13.6.
+    const uint64_t planned = static_cast<uint64_t>(n_launch) * n_layers;
+    const bool split = planned <= 256 || (planned <= 512 && n_slots >= (n_slots <= 256 ? 100 : n_slots <= 512 ? 300 : 832));
     if (n_slots <= 64) {
         hipLaunchKernelGGL(delta_plan_kernel, grid, dim3(64), 0, s, sel, sel_phys, count, n_rows, sel_stride, resident,
                            n_slots, load_phys, slot_of_sel, miss_count, rows);
