@@ -795,9 +795,9 @@ def test_kv_moves_at_the_sizes_of_pieces(ucm, dev, bb):
     assert np.array_equal(out.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("bb,n", [(131072, 3), (196608, 64), (196608, 65), (262144 - 16, 300),        # 256 pieces and more: left whole
-                                  (262144, 64), (262144, 65), (262144 + 16, 43), (262144, 256), (262144, 257),   # from 1025 on cut again
-                                  (524288, 32), (524288, 33), (524288, 128), (524288, 129)])
+@pytest.mark.parametrize("bb,n", [(131072, 3), (163840, 400), (196608, 64), (196608, 65),             # cut: 196608 x 64 only
+                                  (262144, 64), (262144, 65), (262144, 128), (262144, 129), (262144, 384), (262144, 385),   # cut: 64, 129 and 385
+                                  (262144 - 16, 385), (262144 + 16, 43), (262144 + 16, 100), (524288, 32), (524288, 100)])   # cut: all but the 100s
 def test_kv_moves_of_cut_and_whole_slices(ucm, dev, bb, n):
     """Both sides of the rule that cuts a launch's slices between workgroups: dumps, loads, and gathers whose slots are all in use
     or nearly all idle (those stay whole), byte for byte."""

@@ -413,22 +413,23 @@ int stored_layout(const char* name, size_t block_bytes, int rank, int tp_size, S
     return UCM_OK;
 }
 
-// Pieces (a 128 KiB trip each) that `slices` slices are cut into between workgroups, or 1: left whole.  A workgroup with several trips
-// waits before each for the registers of the one before; but a part of a trip at a slice's end takes the place of a whole one, and
-// a launch of a few workgroups more than are resident at once (two per compute unit) ends with the chip half empty.  So slices
-// are cut where every piece has a compute unit of its own, and those of two trips and more where there are several rounds of pieces.
-// us, whole | cut, by process:
-// 256 KiB: one layer of 16 blocks 6.2 | 4.4, 100 blocks 17.4 | 17.5 to 19.1, 200 blocks 35 to 38 | 37 to 40, 400 blocks 75 to 78 | 71 to 73, 32 layers x 256 out and
-// back 2845 to 2937 | 2769 to 2856, 5.1 GB gathered 1724 to 1821 | 1707 to 1757; 512 KiB: 16 blocks 16 | 7.6, 100 blocks 34.5 | 38, 16
-// layers x 64 385 | 360; 160 KiB: 100 blocks 12.2 | 15.0, 16 layers x 64 120 | 129; 192 KiB:
-// 16 blocks 5.1 to 7.0 | 5.2, 100 blocks 13.7 | 15.6, 200 blocks 27.5 | 30.2, 16 layers x 64 145 | 144.
+// Pieces (a 128 KiB trip each) that `slices` slices are cut into between workgroups, or 1: left whole.  A launch takes as long as the
+// compute unit with the most to move: of 288 slices of 256 KiB some have two, of their 576 pieces none has more than three.  Where
+// that is no less for pieces, whole slices are better balanced still; in launches of more than three slices per unit a workgroup that ends
+// with its stores on their way is worth more than that, if no part-trips take places of whole ones.  us, whole | cut: 256 KiB, 128 slices
+// 14.9 | 10.0, 192 16.6 | 19.8, 256 21.5 | 21.7 to 24, 288 31 to 33 | 26.8, 352 33 to 37 | 31 to 33, 448 40.2 | 41.8 to 46, 512 45 to 47 | 44 to
+// 56, 1000 92 to 108 | 91 to 98, 1296 120 to 130 | 114 to 121, 32 layers x 256 blocks out and back 2845 to 2937 | 2769 to 2856, 5.1 GB
+// gathered 1724 to 1821 | 1707 to 1757; 384 KiB, 128 21 | 17, 200 27.0 | 27.5, 288 49 | 39; 512 KiB, 96 25.5 | 17.1, 200 34.2 | 37.8, 352 67.5 |
+// 63, 512 88 | 90 to 100, 1296 245 | 230; 160 KiB, 200 12.2 | 15.0, 2048 120 | 129; 192 KiB, 400 27.5 | 30.2.
 // (What is never cut has an instance without the division: 16 KiB slices 3.1 us for 200 blocks, 3.4 with it.)
+constexpr uint64_t kUnits = 256;         // compute units
+
 unsigned cut_slices(size_t block_bytes, uint64_t grid_x, uint64_t slices)
 {
-    const uint64_t pieces = (block_bytes + kStep - 1) / kStep, workgroups = slices * pieces;
-    const bool fits = grid_x * pieces <= 0xffffffffu / kThreads;
-    const bool cut = workgroups <= 256 || (block_bytes >= 2 * kStep && workgroups > 1024);
-    return fits && cut ? static_cast<unsigned>(pieces) : 1u;
+    const uint64_t pieces = (block_bytes + kStep - 1) / kStep;
+    const uint64_t most_whole = (slices + kUnits - 1) / kUnits * block_bytes, most_cut = (slices * pieces + kUnits - 1) / kUnits * kStep;
+    const bool cut = most_cut < most_whole || (slices > 3 * kUnits && block_bytes >= 2 * kStep);
+    return cut && grid_x * pieces <= 0xffffffffu / kThreads ? static_cast<unsigned>(pieces) : 1u;
 }
 
 template <bool kToStaging>
