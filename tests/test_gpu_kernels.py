@@ -112,7 +112,7 @@ def test_block_mean_of_fp16_caches(ucm, dev, hkv, d, bs):
     (8, 128, 1024, "bfloat16", "bfloat16", "few"),    # 192 groups are the least for persistent ones
 ])
 def test_block_mean_of_large_launches(ucm, dev, hkv, d, bs, keys, table, groups):
-    """320 MiB of keys and more (by repeated blocks) take persistent workgroups, which write their means out when they are done or,
+    """More than 256 MiB of keys (by repeated blocks) take persistent workgroups, which write their means out when they are done or,
     of more groups than LDS holds, on the way: every entry like the oracle's mean of its block, bad ids and slots skipped."""
     from ucm_amd import ops
 
