@@ -422,12 +422,14 @@ __global__ __launch_bounds__(kWideThreads) void kvstar_repre_wide_kernel(
         }
         return n;
     };
-    auto load_unit = [&](u32x4 (&v)[kWideUnroll], const Unit& u) {
+    // (a unit that does not exist reads one piece of another, not all of it: the loads are unconditional)
+    auto load_unit = [&](u32x4 (&v)[kWideUnroll], const Unit& u, bool exists) {
         const unsigned short* src = u.blk + static_cast<size_t>(u.m0) * kMerge * row;
+        const unsigned all = exists ? ~0u : 0u;
 #pragma unroll
         for (unsigned j = 0; j < kItems; ++j) {
 #pragma unroll
-            for (unsigned t = 0; t < kMerge; ++t) { v[j * kMerge + t] = ucm::gload16_nt(src + (j * item_subs * kMerge + t) * row + mine); }
+            for (unsigned t = 0; t < kMerge; ++t) { v[j * kMerge + t] = ucm::gload16_nt(src + ((j * item_subs * kMerge + t) * row & all) + (mine & all)); }
         }
         // keeps the compiler from sinking the loads to their use, and from forming the other unit's means before they are issued
         asm volatile("" ::: "memory");
@@ -435,7 +437,7 @@ __global__ __launch_bounds__(kWideThreads) void kvstar_repre_wide_kernel(
     };
     PieceMap pm = {};
     unsigned cur_layer = kNoRow, cur_list = 0;
-    auto finish_unit = [&](const u32x4 (&v)[kWideUnroll], const Unit& u, bool exists) {
+    auto finish_unit = [&](const u32x4 (&v)[kWideUnroll], const Unit& u) {
         const unsigned chunk0 = u.m0 / m_chunk * m_chunk;
 #pragma unroll
         for (unsigned j = 0; j < kItems; ++j) {
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(kWideThreads) void kvstar_repre_wide_kernel(
         const unsigned end = u.m0 + unit_subs;
         if (end != M && end != chunk0 + m_chunk) { return; }
         // the chunk is staged: write its pieces (all conditions here are the same for all threads)
-        const bool live = exists && u.slot != kNoRow;
+        const bool live = u.slot != kNoRow;
         if (live && pruned && (u.layer != cur_layer || u.list != cur_list)) {
             cur_layer = u.layer;
             cur_list = u.list;
@@ -475,16 +477,16 @@ __global__ __launch_bounds__(kWideThreads) void kvstar_repre_wide_kernel(
     Unit a;
     open(a, blockIdx.x);
     u32x4 va[kWideUnroll], vb[kWideUnroll];
-    load_unit(va, a);
+    load_unit(va, a, true);
     for (;;) {                                           // one way out, at the end: see kvstar_repre_kernel
         bool has_b = true, has_c = true;
         const Unit b = next_of(a, has_b);
-        load_unit(vb, has_b ? b : a);
-        finish_unit(va, a, true);
+        load_unit(vb, has_b ? b : a, has_b);
+        finish_unit(va, a);
         const Unit c = has_b ? next_of(b, has_c) : b;
         has_c = has_c && has_b;
-        load_unit(va, has_c ? c : a);
-        finish_unit(vb, has_b ? b : a, has_b);
+        load_unit(va, has_c ? c : a, has_c);
+        if (has_b) { finish_unit(vb, b); }
         if (!has_c) { break; }
         a = c;
     }
