@@ -109,12 +109,12 @@ def test_kvstar_block_repre_of_fp16_keys(ucm, dev, merge, hkv, d, bs):
     (8, 16, 128, 64, 64, "float16"),
     (2, 1, 64, 1024, 16, "bfloat16"),
 ])
-def test_kvstar_block_repre_of_blocks_in_whole_units(ucm, dev, merge, hkv, d, bs, kept, keys):
+def test_kvstar_block_repre_of_blocks_in_whole_units(ucm, dev, merge, hkv, d, bs, kept, keys, n=203):
     """Blocks of 128 KiB and multiples go through the workgroups of sixteen waves, several entries to each, with channel
     lists named per entry (and layer): like the oracle's, bad blocks, rows and lists skipped."""
     from ucm_amd import ops
 
-    L, nb, n, M, n_lists = 3, 5, 203, bs // merge, 2
+    L, nb, M, n_lists = 3, 5, bs // merge, 2
     rows, d_pad, f16 = n + 4, (kept + 15) // 16 * 16, keys == "float16"
     caches = [torch.from_numpy(synth.normal_f32(1700 + l, (nb, bs, hkv, d))).to(torch.float16 if f16 else torch.bfloat16) for l in range(L)]
     caches_h = [c.view(torch.int16).numpy().view(np.uint16) for c in caches]
@@ -145,6 +145,14 @@ def test_kvstar_block_repre_of_blocks_in_whole_units(ucm, dev, merge, hkv, d, bs
             mine = good & ((sel == s) if pruned is not None else True)
             want[slots[mine]] = of_block[ids[mine]]
         assert np.array_equal(got[l], want), l
+
+
+@pytest.mark.parametrize("n", [6, 85, 86, 170, 171])                   # of three layers: up to 256 blocks, one, two and three a workgroup
+@pytest.mark.parametrize("merge,hkv,bs,kept,keys", [(1, 8, 64, 32, "bfloat16"), (4, 8, 64, 32, "float16"), (4, 8, 64, 128, "bfloat16"),
+                                                    (8, 4, 128, 48, "bfloat16"), (8, 8, 128, 32, "bfloat16")])
+def test_kvstar_block_repre_of_few_blocks_in_whole_units(ucm, dev, merge, hkv, bs, kept, keys, n):
+    """Workgroups with one, two and three units of loads, and the launches of single units that smaller workgroups take."""
+    test_kvstar_block_repre_of_blocks_in_whole_units(ucm, dev, merge, hkv, 128, bs, kept, keys, n)
 
 
 @pytest.mark.parametrize("merge", [2, 16, 3])      # the persistent kernel, and the one for other sub-block sizes (16 and 3)

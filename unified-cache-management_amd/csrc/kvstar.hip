@@ -1263,7 +1263,12 @@ extern "C" int ucm_kvstar_block_repre_keys(const void* const* k_layers, int key_
     if (wide) {
         const unsigned unit_subs = kWideThreads / ncg * (kWideUnroll / merge);
         const unsigned fit = kWideLds > list_bytes ? (kWideLds - list_bytes) / ((row + 8) * 2) / unit_subs * unit_subs : 0u;
-        wide = M % unit_subs == 0 && fit > 0;
+        // (one block of one unit per compute unit, lists to fetch first and few means to write: the smaller workgroups are done sooner.  256
+        // blocks of 64 tokens x 8 heads, a quarter of the channels kept, merge 8 7.2 us and 8.0, merge 4 8.0 and 8.1, of float16 keys 7.4
+        // and 8.1; 64 blocks, merge 8, 6.2 and 6.8)
+        const bool brief = static_cast<unsigned>(M) == unit_subs && pruned && merge >= 4 &&
+                           static_cast<uint64_t>(n) * n_layers <= kWideGroups;
+        wide = M % unit_subs == 0 && fit > 0 && !brief;
         if (wide) { m_chunk = std::min<unsigned>(static_cast<unsigned>(M), fit); }
     }
     const size_t lds_bytes = static_cast<size_t>(m_chunk) * (row + 8) * 2 + list_bytes;
