@@ -726,6 +726,37 @@ def test_topk_windows_of_many_rows(ucm, dev, L, R, n, kind):
     assert np.array_equal(np.where(want < n, table[np.arange(R)[None, :, None], np.minimum(want, n - 1)], -7), got_phys)
 
 
+@pytest.mark.parametrize("L,R,longest", [(24, 32, 300), (25, 31, 300), (24, 64, 600), (29, 53, 600), (29, 53, 200)])   # 768, 775, 1536 and 1537 requests
+@pytest.mark.parametrize("tile", [0, 2048])                              # tiles the library picks, and one for each request
+def test_score_select_of_many_requests(ucm, dev, L, R, longest, tile):
+    """Both sides of the rule that gives a request's selection one wave or four in the fused launch: what is selected is what the
+    launch's own scores say, the first index of equal scores first."""
+    from ucm_amd import ops
+
+    rng = np.random.default_rng(R + longest)
+    lens = rng.integers(4, longest + 1, R).astype(np.int32)
+    lens[:6] = longest, 128, 129, min(longest, 256), min(longest, 257), 3
+    off = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    rows, ks = int(lens.sum()), np.minimum(rng.integers(4, 40, R), lens).astype(np.int32)
+    q = torch.empty((L, R, 2, 64), dtype=torch.bfloat16, device=dev).normal_()
+    repre = torch.empty((L, rows, 64), dtype=torch.bfloat16, device=dev).normal_()
+    scores = torch.zeros((L, rows), device=dev)
+    idx = torch.full((L, R, longest), -7, dtype=torch.int32, device=dev)
+    cnt, tickets = torch.zeros((L, R), dtype=torch.int32, device=dev), torch.zeros((L, R), dtype=torch.int32, device=dev)
+    for _ in range(2):                                                   # (the tickets are left as they were found)
+        ops.score_select(q, repre, i32(off, dev), i32(lens, dev), i32(ks, dev), longest, 1, scores, idx, cnt, tickets, total_blocks=rows,
+                         tile_blocks=tile)
+    assert not tickets.any() and torch.equal(cnt, i32(ks, dev).expand(L, R))
+    i = np.arange(longest)
+    at = np.minimum(off[:, None] + i, rows - 1)
+    s = scores.cpu().numpy()[:, at]
+    s[:, (i < 1) | ((i >= lens[:, None] - 2) & (i < lens[:, None]))] = np.inf
+    s[:, i >= lens[:, None]] = -np.inf
+    order = np.argsort(-s, axis=-1, kind="stable")
+    want = np.sort(np.where(i < ks[:, None], order, longest), axis=-1)
+    assert np.array_equal(np.where(want < longest, want, -7), idx.cpu().numpy())
+
+
 @pytest.mark.parametrize("bb", [262144, 4096, 48, 16 + 32768])
 def test_kv_dump_load_round_trip(ucm, dev, bb):
     """Config-3 shape in small: random block table, scatter staging->cache, gather cache->staging, byte exact."""

@@ -311,13 +311,21 @@ __device__ __forceinline__ float head_sum(float dot, int first, int step, int kv
 }
 
 // The request's selection with the smallest tier of key registers that holds it (the host allows at most 1024 blocks here): up to
-// kSoloBlocks by the first wave alone, from there on by all four.  scratch: kStaged words of LDS
+// kSoloBlocks by the first wave alone, from there on by all four - or alone for longer, where a launch has so many requests that the
+// three waves that wait would keep others from running.  us by four | by one: 5120 requests of 130 to 140 blocks 32.7 | 28.5, 1178 of
+// 106 to 212 39.7 | 38.3, 1024 of 129 to 256 x 8 heads 72.6 | 71.2, 512 of 129 to 256 7.0 | 7.3; 2048 of 300 to 500 25.4 | 24.4, 1550 32.8 |
+// 31.5, 5120 of 300 to 500 (fp32) 91.5 | 93.0, 512 of 300 9.5 | 11.1; 5120 of 600 to 1000 102.8 | 103.5.
+// scratch: kStaged words of LDS
 constexpr int kSoloBlocks = 128;
+
+__device__ __forceinline__ int solo_blocks(int requests) { return requests <= 768 ? kSoloBlocks : requests <= 1536 ? 256 : 512; }
 
 __device__ __forceinline__ void select_solo(const ucm::SelectArgs& sel, const TileInfo& t, int l, const float* lds)
 {
     if (t.n <= 64) { ucm::select_wave<1, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
-    else { ucm::select_wave<2, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
+    else if (t.n <= 128) { ucm::select_wave<2, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
+    else if (t.n <= 256) { ucm::select_wave<4, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
+    else { ucm::select_wave<8, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
 }
 
 __device__ __forceinline__ void select_shared(const ucm::SelectArgs& sel, const TileInfo& t, int l, unsigned* scratch, const float* lds)
@@ -346,7 +354,8 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
         for (int i = threadIdx.x; i < n_tile; i += kThreads) { sout[i] = tile_scores[i]; }
         return;
     }
-    if (t.n <= kSoloBlocks && threadIdx.x >= 64) { return; }     // the other waves are done: their registers are free again
+    const bool solo = t.n <= solo_blocks(sel.n_req * static_cast<int>(gridDim.x));
+    if (solo && threadIdx.x >= 64) { return; }                   // the other waves are done: their registers are free again
     asm volatile("" ::: "memory");
     const int tiles = max((t.n + a.tile_blocks - 1) / a.tile_blocks, 1);
     const bool alone = tiles == 1 && t.ok;                       // all of the request's scores are here: nobody to wait for
@@ -367,7 +376,7 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
         if (lane == 0) { __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
         return true;
     };
-    if (t.n <= kSoloBlocks) {
+    if (solo) {
         if (alone) {
             store();
             select_solo(sel, t, l, tile_scores);
