@@ -100,29 +100,32 @@ def test_block_mean_of_fp16_caches(ucm, dev, hkv, d, bs):
                        bs, hkv, d, nb)
 
 
-@pytest.mark.parametrize("hkv,d,bs,keys,table,groups", [    # groups: what a persistent workgroup goes through, fits its LDS or more
-    (8, 128, 16, "bfloat16", "bfloat16", "fits"),     # two list entries side by side
-    (8, 128, 16, "float16", "float32", "more"),
-    (8, 128, 128, "float16", "float32", "fits"),
-    (1, 8, 16, "bfloat16", "float32", "more"),        # 256 entries side by side, several to a wave
-    (1, 64, 16, "bfloat16", "float32", "more"),
-    (1, 64, 32, "bfloat16", "bfloat16", "fits"),
-    (3, 96, 48, "bfloat16", "float32", "more"),       # a row that does not divide the workgroup
-    (16, 256, 16, "bfloat16", "bfloat16", "fits"),    # two column groups
-    (8, 128, 1024, "bfloat16", "bfloat16", "few"),    # 192 groups are the least for persistent ones
+@pytest.mark.parametrize("hkv,d,bs,keys,table,mb,groups", [    # groups: what a persistent workgroup goes through, fits its LDS or more
+    (8, 128, 16, "bfloat16", "bfloat16", 384, "fits"),     # two list entries side by side
+    (8, 128, 32, "float16", "float32", 768, "more"),
+    (8, 128, 16, "float16", "float32", 384, "short"),      # blocks of 16 tokens into an fp32 table: not persistent
+    (8, 128, 128, "float16", "float32", 384, "fits"),
+    (1, 8, 32, "bfloat16", "float32", 768, "more"),        # 256 entries side by side, several to a wave
+    (1, 64, 32, "bfloat16", "float32", 768, "more"),
+    (1, 64, 16, "bfloat16", "bfloat16", 384, "fits"),
+    (1, 64, 32, "bfloat16", "bfloat16", 384, "fits"),
+    (3, 96, 48, "bfloat16", "float32", 384, "more"),       # a row that does not divide the workgroup
+    (16, 256, 16, "bfloat16", "bfloat16", 384, "fits"),    # two column groups
+    (8, 128, 1024, "bfloat16", "bfloat16", 384, "few"),    # 192 groups are the least for persistent ones
 ])
-def test_block_mean_of_large_launches(ucm, dev, hkv, d, bs, keys, table, groups):
+def test_block_mean_of_large_launches(ucm, dev, hkv, d, bs, keys, table, mb, groups):
     """More than 256 MiB of keys (by repeated blocks) take persistent workgroups, which write their means out when they are done or,
     of more groups than LDS holds, on the way: every entry like the oracle's mean of its block, bad ids and slots skipped."""
     from ucm_amd import ops
 
     nb, L, row = 37 if bs < 1024 else 9, 3, hkv * d
-    n = (384 << 20) // (L * bs * row * 2) + (333 if bs < 1024 else 33)
+    n = (mb << 20) // (L * bs * row * 2) + (333 if bs < 1024 else 33)
     threads = row // 8                                             # the launch as the host lays it out
     share = 256 // threads if threads < 256 and 256 % threads == 0 else 1
     total = L * (-(-n // share) if share > 1 else n * -(-threads // 256))
     kept = 158 * 1024 // ((32 if table == "float32" else 16) * 256 + 4 * max(share, 4))
-    assert groups == ("few" if total < 192 else "fits" if -(-total // 256) <= kept else "more")
+    short = bs == 16 and table == "float32"
+    assert groups == ("few" if total < 192 else "short" if short else "fits" if -(-total // 256) <= kept else "more")
     rows = n + 5
     f16 = keys == "float16"
     host = np.stack([synth.normal_f32(140 + l, (nb, bs, hkv, d)) for l in range(L)])

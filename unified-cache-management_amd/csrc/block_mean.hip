@@ -213,8 +213,8 @@ __global__ __launch_bounds__(kThreads) void block_mean_kernel(
 // added, and keeps the means in LDS until that is full or its work is done: 632 us (6.8 TB/s), 655 when they leave eight
 // groups at a time, 725 -> 672 us into an fp32 table.  Four workgroups of 128 threads per compute unit: 667 us.  How much that brings depends on
 // the memory a process gets: 691 -> 633, 710 -> 662, and on one machine 645 either way.
-// For more than 256 MiB of keys, what the memory-side cache holds, and a group for three in four of the compute units.  us,
-// block_mean_kernel | this, 8 heads: 256 MiB in blocks of 16, 64, 128, 256 tokens 47.5 | 46.4, 43.7 | 43.3, 42.2 | 43.2, 41.9 | 43.4; 271
+// For more than 256 MiB of keys, what the memory-side cache holds, a group for three in four of the compute units, and not for blocks of
+// 16 tokens into an fp32 table, whose means fill LDS too often (1000 MiB 200 | 224, into a bf16 one 186 | 183).  us, block_mean_kernel | this, 8 heads: 256 MiB in blocks of 16, 64, 128, 256 tokens 47.5 | 46.4, 43.7 | 43.3, 42.2 | 43.2, 41.9 | 43.4; 271
 // and 289 MiB 46.7 | 43.7 and 51.2 | 49.1; 384 MiB 72 | 69, 64.3 | 63.0, 61.8 | 61.6, 60.3 | 60.1; 2 GiB 396 | 382, 369 | 342, 355 | 337,
 // 340 | 334.  256 groups of 512 tokens 163 | 165, 192 of 512 and of 1024 tokens 61.7 | 59.1 and 125 | 121; 128 of 512 tokens 44 | 51,
 // 96 of 1024 tokens 73 | 85, 64 of 2048 tokens 142 | 166.
@@ -415,7 +415,8 @@ extern "C" int ucm_block_mean(const void* const* k_layers, int n_layers, int num
                             static_cast<float*>(repre), repre_layer_stride, mode, of_abs, keys_f16};
         const uint64_t bytes = static_cast<uint64_t>(n) * n_layers * block_size * row * 2;
         const StreamGroups g = stream_groups(a);
-        if (bytes > kStreamBytes && g.total >= kStreamLeast) { return launch_stream(a, g, ucm::as_stream(stream)); }
+        const bool few_means = mode == UCM_MEAN_BF16_STORE || block_size >= 2 * kUnroll;      // at most a sixteenth of the keys' bytes
+        if (bytes > kStreamBytes && g.total >= kStreamLeast && few_means) { return launch_stream(a, g, ucm::as_stream(stream)); }
     }
 #define UCM_BLOCK_MEAN_ARGS dim3(groups, n_layers), dim3(kThreads), 0, ucm::as_stream(stream), k_layers, block_ids, slots, \
         static_cast<unsigned>(num_blocks), static_cast<unsigned>(repre_rows), static_cast<unsigned>(block_size), row,       \
