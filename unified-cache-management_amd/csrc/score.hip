@@ -314,23 +314,32 @@ __device__ __forceinline__ float head_sum(float dot, int first, int step, int kv
 // kSoloBlocks by the first wave alone, from there on by all four - or alone for longer, where a launch has so many requests that the
 // three waves that wait would keep others from running.  us by four | by one: 5120 requests of 130 to 140 blocks 32.7 | 28.5, 1178 of
 // 106 to 212 39.7 | 38.3, 1024 of 129 to 256 x 8 heads 72.6 | 71.2, 512 of 129 to 256 7.0 | 7.3; 2048 of 300 to 500 25.4 | 24.4, 1550 32.8 |
-// 31.5, 5120 of 300 to 500 (fp32) 91.5 | 93.0, 512 of 300 9.5 | 11.1; 5120 of 600 to 1000 102.8 | 103.5.
+// 31.5, 5120 of 300 to 500 (fp32) 91.5 | 93.0, 512 of 300 9.5 | 11.1; 5120 of 600 to 1000 102.8 | 103.5.  Such launches have instances of
+// their own (kMany): the longer selections' code costs a launch of 16 requests 0.1 us.
 // scratch: kStaged words of LDS
 constexpr int kSoloBlocks = 128;
+constexpr int kManyRequests = 768;
 
-__device__ __forceinline__ int solo_blocks(int requests) { return requests <= 768 ? kSoloBlocks : requests <= 1536 ? 256 : 512; }
+template <bool kMany>
+__device__ __forceinline__ int solo_blocks(const ucm::SelectArgs& sel)
+{
+    if (!kMany) { return kSoloBlocks; }
+    return sel.n_req * static_cast<int>(gridDim.x) <= 2 * kManyRequests ? 256 : 512;
+}
 
+template <bool kMany>
 __device__ __forceinline__ void select_solo(const ucm::SelectArgs& sel, const TileInfo& t, int l, const float* lds)
 {
     if (t.n <= 64) { ucm::select_wave<1, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
-    else if (t.n <= 128) { ucm::select_wave<2, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
+    else if (!kMany || t.n <= 128) { ucm::select_wave<2, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
     else if (t.n <= 256) { ucm::select_wave<4, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
     else { ucm::select_wave<8, false, true>(sel, t.r, l, threadIdx.x, t.n, t.seg0, t.topk, lds); }
 }
 
+template <bool kMany>
 __device__ __forceinline__ void select_shared(const ucm::SelectArgs& sel, const TileInfo& t, int l, unsigned* scratch, const float* lds)
 {
-    if (t.n <= 256) { ucm::select_blocks<4, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
+    if (!kMany && t.n <= 256) { ucm::select_blocks<4, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
     else if (t.n <= 512) { ucm::select_blocks<8, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
     else { ucm::select_blocks<16, false, true>(sel, t.r, l, t.n, t.seg0, t.topk, scratch, lds); }
 }
@@ -345,6 +354,7 @@ __device__ __forceinline__ void select_shared(const ucm::SelectArgs& sel, const 
 // runs the request's selection (TopkBlockSelector::TopKImpl, select_topk_block.cpp:20-51) on the scores all of
 // them wrote, which it reads with device-scope loads after it has seen every other ticket.  (A device-scope
 // release/acquire pair would also do, but it writes the whole L2 back per wave: 7x the kernel's time.)
+template <bool kMany>
 __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::SelectArgs& sel, const TileInfo& t, int l, int tile0,
                                             int n_tile, const float* tile_scores, float* qbar)
 {
@@ -354,7 +364,7 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
         for (int i = threadIdx.x; i < n_tile; i += kThreads) { sout[i] = tile_scores[i]; }
         return;
     }
-    const bool solo = t.n <= solo_blocks(sel.n_req * static_cast<int>(gridDim.x));
+    const bool solo = t.n <= solo_blocks<kMany>(sel);
     if (solo && threadIdx.x >= 64) { return; }                   // the other waves are done: their registers are free again
     asm volatile("" ::: "memory");
     const int tiles = max((t.n + a.tile_blocks - 1) / a.tile_blocks, 1);
@@ -379,10 +389,10 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
     if (solo) {
         if (alone) {
             store();
-            select_solo(sel, t, l, tile_scores);
+            select_solo<kMany>(sel, t, l, tile_scores);
             return;
         }
-        if (draws_last_ticket()) { select_solo(sel, t, l, nullptr); }
+        if (draws_last_ticket()) { select_solo<kMany>(sel, t, l, nullptr); }
         return;
     }
     bool last = true;
@@ -395,7 +405,7 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
         __syncthreads();
         last = __builtin_amdgcn_readfirstlane(draws_last) != 0;
     }
-    if (last) { select_shared(sel, t, l, reinterpret_cast<unsigned*>(qbar), alone ? tile_scores : nullptr); }
+    if (last) { select_shared<kMany>(sel, t, l, reinterpret_cast<unsigned*>(qbar), alone ? tile_scores : nullptr); }
 }
 
 // grid: x = layer, y = dense tile index over all requests (workgroups past the
@@ -406,7 +416,7 @@ __device__ __forceinline__ void finish_tile(const ScoreArgs& a, const ucm::Selec
 // the grid from its own bounds on the segment lengths - are dispatched last: in
 // between the others each of them held a workgroup's registers and LDS for the
 // time it takes to find that out (12 us for 1600 of them among 2500).
-template <int kD, typename QT>
+template <int kD, typename QT, bool kMany>
 __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, const ucm::SelectArgs sel)
 {
     constexpr int kSteps = kD / 16;
@@ -470,7 +480,7 @@ __global__ __launch_bounds__(kThreads) void score_kernel(const ScoreArgs a, cons
             b0 = b2;
         }
     }
-    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores, qbar);
+    finish_tile<kMany>(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores, qbar);
 }
 
 // ---- bf16 representative table ------------------------------------------------
@@ -518,7 +528,7 @@ __device__ __forceinline__ float pair_dot(const f32x4 (&qlo)[kKept], const float
     return (b0 + b2) + (b1 + b3);
 }
 
-template <int kD, typename QT>
+template <int kD, typename QT, bool kMany>
 __global__ __launch_bounds__(kThreads, kD <= 128 ? 4 : 2) void score_kernel_bf16(const ScoreArgs a, const ucm::SelectArgs sel)
 {
     constexpr int kSteps = kD / 16;
@@ -585,14 +595,16 @@ __global__ __launch_bounds__(kThreads, kD <= 128 ? 4 : 2) void score_kernel_bf16
             b0 = b2;
         }
     }
-    finish_tile(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores, qbar);
+    finish_tile<kMany>(a, sel, t, l, tile0, t.ok ? max(tile_end - tile0, 0) : 0, tile_scores, qbar);
 }
 
 template <int kD, typename QT>
 void launch_dim(const ScoreArgs& a, const ucm::SelectArgs& sel, bool bf16_table, dim3 grid, hipStream_t s)
 {
-    if (bf16_table) { hipLaunchKernelGGL((score_kernel_bf16<kD, QT>), grid, dim3(kThreads), 0, s, a, sel); }
-    else { hipLaunchKernelGGL((score_kernel<kD, QT>), grid, dim3(kThreads), 0, s, a, sel); }
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, a, sel); };
+    const bool many = a.tickets && static_cast<int64_t>(a.n_req) * grid.x > kManyRequests;       // (grid.x: layers)
+    if (bf16_table) { many ? launch(score_kernel_bf16<kD, QT, true>) : launch(score_kernel_bf16<kD, QT, false>); }
+    else { many ? launch(score_kernel<kD, QT, true>) : launch(score_kernel<kD, QT, false>); }
 }
 
 template <int kD>
