@@ -379,7 +379,9 @@ __global__ __launch_bounds__(kThreads) void kvstar_repre_kernel(
 // group never changes and its items lie at the same places of every unit, so a load is a scalar base and an offset kept in
 // a register.  32 layers x 1024 blocks of 128 tokens x 8 heads, a quarter of the channels kept, against kvstar_repre_kernel:
 // merge 2 1892 -> 1702 us, 4 1727 -> 1639; half the blocks: merge 8 817 -> 748, merge 2 with all channels 1280 -> 1171; 64-token
-// blocks 950 -> 849, 4 heads 944 -> 853; one layer, 600 blocks 43.4 -> 35.4, 64 blocks 13.6 -> 11.7, 16 blocks 12.0 -> 11.8.
+// blocks 950 -> 849, 4 heads 944 -> 853.  One layer, 512 blocks 30.5 -> 25.2, 64 blocks 12.8 -> 8.2, 16 blocks 12.6 -> 8.1 (with a
+// last unit that does not exist read in full 28.7, 8.2 and 8.1; blocks of 64 tokens, which are one unit each, 256 of them 10.6 that
+// way and 8.4 now, 768 of them 26.9 and 20.8, and 9.3 and 25.3 in kvstar_repre_kernel).
 template <int kMerge, bool kF16>
 __global__ __launch_bounds__(kWideThreads) void kvstar_repre_wide_kernel(
     const void* const* __restrict__ k_layers, const int32_t* __restrict__ block_ids,
